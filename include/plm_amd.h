@@ -153,6 +153,17 @@ size_t plm_gemm_packed_workspace_bytes(int64_t M, int64_t N, int64_t K, const pl
 int plm_gemm_packed_tile_supported(int32_t dtype, int64_t M, int64_t K, const plm_tile* tile);
 
 /*
+ * Y = X[M,K] · W[N,K]^T over a packed weight at any width (the prefill chunks the reference hands to
+ * F.linear, plm/fast_gemm.py:108-111), with no workspace. `out_kind`: PLM_OUT_MODEL (Y[M,N] in the input
+ * dtype), PLM_OUT_F32 (Y[M,N] fp32), or PLM_OUT_SILU_MUL: W is a fused gate/up weight (gate rows first,
+ * N a multiple of 32) packed as it is, and Y[M,N/2] gets plm_gemm_packed_silu_mul's values (ldy % 4 == 0,
+ * y 8-byte aligned). Every output is one MFMA chain over K in ascending order. M * ldx * 2 < 2^31; x, ldx
+ * and K as plm_gemm_packed.
+ */
+int plm_gemm_wide(int32_t dtype, const void* x, int64_t ldx, const void* packed_w, void* y, int64_t ldy, int64_t M,
+                  int64_t N, int64_t K, int32_t out_kind, void* stream);
+
+/*
  * Y[M,N] = X[M,K] · W[N,K]^T with fp32 accumulation, Y in the input dtype.
  * Replaces triton_linear (plm/fast_gemm.py:82-97) together with gemm_kernel (17-48) and
  * splitk_reduce_kernel (51-61). Requirements: 1 <= M <= 128, K % 8 == 0, ldx/ldw % 8 == 0,

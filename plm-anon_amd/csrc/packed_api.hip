@@ -212,16 +212,11 @@ int packed_entry(int32_t dtype, const void* x, int64_t ldx, const void* wp, void
                             static_cast<hipStream_t>(stream));
 }
 
-// Widths past 128 rows (prefill chunks, plm/rounds.py:16, which the reference hands to F.linear)
-// run on the wide kernel (csrc/wide_gemm.hip: 128 x 128 tiles staged through LDS, K split for thin
-// shapes); the tile configuration applies to the skinny kernel only and is checked for validity.
-// Every argument is checked before the launch.
-int packed_rows(int32_t dtype, const void* x, int64_t ldx, const void* wp, void* y, int64_t ldy, int64_t M, int64_t N,
-                int64_t K, const plm_tile* tile, void* workspace, size_t workspace_bytes, void* stream, int out_f32,
-                int64_t cap = kNoCap) {
-  if (M <= kPackedMaxM) return packed_entry(dtype, x, ldx, wp, y, ldy, M, N, K, tile, workspace, workspace_bytes, stream, out_f32);
-  if (!packed_tile_valid(tile)) return PLM_ERR_TILE;
-  if (N < 1 || N > (int64_t(1) << 30) || K > (int64_t(1) << 30)) return PLM_ERR_ARGUMENT;
+// The wide kernel (csrc/wide_gemm.hip), every argument checked before the launch. `need`: workspace
+// bytes the caller has to bring (the kernel uses none).
+int wide_rows(int32_t dtype, const void* x, int64_t ldx, const void* wp, void* y, int64_t ldy, int64_t M, int64_t N,
+              int64_t K, WideOut out, const void* workspace, size_t workspace_bytes, int64_t need, void* stream) {
+  if (M < 1 || N < 1 || N > (int64_t(1) << 30) || K > (int64_t(1) << 30)) return PLM_ERR_ARGUMENT;
   plm_chain_gemm g{};
   g.x = x;
   g.w = wp;
@@ -232,12 +227,28 @@ int packed_rows(int32_t dtype, const void* x, int64_t ldx, const void* wp, void*
   g.N = static_cast<int32_t>(N);
   g.K = static_cast<int32_t>(K);
   g.split_k = 1;
-  g.out_f32 = out_f32;
-  const int status = packed_check_linear(dtype, g, kPackedMaxM);  // the checks but the width's
+  g.out_f32 = out == WideOut::kModel ? PLM_OUT_MODEL : out == WideOut::kF32 ? PLM_OUT_F32 : PLM_OUT_SILU_MUL;
+  const plm_tile even{2, 8, 1, 2};  // the activation's checks ask for a tile with an even wave_frags
+  const int status = packed_check_linear(dtype, g, 1, &even);  // the checks but the width's
   if (status != PLM_OK) return status;
   if (M > (int64_t(1) << 24) || M * ldx * 2 >= (int64_t(1) << 31)) return PLM_ERR_ARGUMENT;
-  return wide_gemm(dtype, x, ldx, wp, y, ldy, M, N, K, workspace, workspace_bytes, static_cast<hipStream_t>(stream),
-                   out_f32, cap);
+  if (need > 0 && (workspace == nullptr || static_cast<int64_t>(workspace_bytes) < need ||
+                   (reinterpret_cast<uintptr_t>(workspace) & 15) != 0))
+    return PLM_ERR_WORKSPACE;
+  return wide_gemm(dtype, x, ldx, wp, y, ldy, M, N, K, static_cast<hipStream_t>(stream), out);
+}
+
+// Widths past 128 rows (prefill chunks, plm/rounds.py:16, which the reference hands to F.linear)
+// run on the wide kernel; the tile configuration applies to the skinny kernel only and is checked for
+// validity.
+int packed_rows(int32_t dtype, const void* x, int64_t ldx, const void* wp, void* y, int64_t ldy, int64_t M, int64_t N,
+                int64_t K, const plm_tile* tile, void* workspace, size_t workspace_bytes, void* stream, int out_f32,
+                int64_t cap = kNoCap) {
+  if (M <= kPackedMaxM) return packed_entry(dtype, x, ldx, wp, y, ldy, M, N, K, tile, workspace, workspace_bytes, stream, out_f32);
+  if (!packed_tile_valid(tile)) return PLM_ERR_TILE;
+  const int64_t need = N >= 1 && K >= 1 ? wide_workspace(M, N, K, cap) : 0;
+  return wide_rows(dtype, x, ldx, wp, y, ldy, M, N, K, out_f32 ? WideOut::kF32 : WideOut::kModel, workspace,
+                   workspace_bytes, need, stream);
 }
 
 // How the linears of a chain wait for the ones they read: 0 (none reads another), 2 (every linear
@@ -390,6 +401,15 @@ int plm_gemm_packed_f32out(int32_t dtype, const void* x, int64_t ldx, const void
                            int64_t M, int64_t N, int64_t K, const plm_tile* tile, void* workspace,
                            size_t workspace_bytes, void* stream) {
   return plm::packed_rows(dtype, x, ldx, packed_w, y, ldy, M, N, K, tile, workspace, workspace_bytes, stream, 1);
+}
+
+int plm_gemm_wide(int32_t dtype, const void* x, int64_t ldx, const void* packed_w, void* y, int64_t ldy, int64_t M,
+                  int64_t N, int64_t K, int32_t out_kind, void* stream) {
+  if (out_kind != PLM_OUT_MODEL && out_kind != PLM_OUT_F32 && out_kind != PLM_OUT_SILU_MUL) return PLM_ERR_ARGUMENT;
+  const plm::WideOut out = out_kind == PLM_OUT_MODEL ? plm::WideOut::kModel
+                           : out_kind == PLM_OUT_F32 ? plm::WideOut::kF32
+                                                     : plm::WideOut::kActPlain;
+  return plm::wide_rows(dtype, x, ldx, packed_w, y, ldy, M, N, K, out, nullptr, 0, 0, stream);
 }
 
 int plm_gemm_packed_resident_workgroups(int32_t dtype, int64_t M, const plm_tile* tile) {

@@ -563,10 +563,7 @@ __device__ __forceinline__ void tile_done(const PackedArgs& a, const PLinear& L,
 // SiLU-and-multiply epilogue (kEpiAct) of a fused gate/up projection packed with its gate and up
 // rows interleaved by fragment: fragment 2j holds gate rows [16j, 16j+16) and fragment 2j+1 the
 // up rows [16j, 16j+16) of the same output columns. Column block `cblk` (16 columns of the [M, N/2]
-// output) of X row 16t + lane%16, columns 16*cblk + 4*(lane/16) + r: the gate and up values rounded
-// to the model dtype (the projection's output), then vLLM's SiluAndMul on them (its silu_and_mul
-// kernel, which the rounds run with enforce_eager): silu(g) = g / (1 + e^-g) in fp32 rounded to the
-// model dtype, times u, rounded again (the product of two 16-bit values is exact in fp32).
+// output) of X row 16t + lane%16, columns 16*cblk + 4*(lane/16) + r (silu_mul_bits).
 template <int DT, int MT>
 __device__ __forceinline__ void act_store(const PLinear& L, int M, int cblk, int t, int lane, f32x4 g, f32x4 u) {
   const int m = 16 * t + (lane & 15);
@@ -574,10 +571,7 @@ __device__ __forceinline__ void act_store(const PLinear& L, int M, int cblk, int
   if (m >= M || n >= (L.N >> 1)) return;  // N/2 is a multiple of 16: all four columns are in range
   uint16_t h[4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const float gr = from_bits16<DT>(to_bits16<DT>(g[r])), ur = from_bits16<DT>(to_bits16<DT>(u[r]));
-    h[r] = to_bits16<DT>(from_bits16<DT>(to_bits16<DT>(gr / (1.0f + expf(-gr)))) * ur);
-  }
+  for (int r = 0; r < 4; ++r) h[r] = silu_mul_bits<DT>(g[r], u[r]);
   uint64_t* y = reinterpret_cast<uint64_t*>(static_cast<uint16_t*>(L.y) + static_cast<int64_t>(m) * L.ldy + n);
   const uint64_t bits = (static_cast<uint64_t>(h[0]) | (static_cast<uint64_t>(h[1]) << 16)) |
                         ((static_cast<uint64_t>(h[2]) | (static_cast<uint64_t>(h[3]) << 16)) << 32);

@@ -61,6 +61,16 @@ __device__ __forceinline__ float from_bits16(uint16_t h) {
   }
 }
 
+// vLLM's SiluAndMul on a gate and an up value of the projection, as its silu_and_mul kernel does it
+// (the rounds run it with enforce_eager): both rounded to the model dtype (the projection's output),
+// silu(g) = g / (1 + e^-g) in fp32 rounded to the model dtype, times u, rounded again (the product of
+// two 16-bit values is exact in fp32).
+template <int DT>
+__device__ __forceinline__ uint16_t silu_mul_bits(float g, float u) {
+  const float gr = from_bits16<DT>(to_bits16<DT>(g)), ur = from_bits16<DT>(to_bits16<DT>(u));
+  return to_bits16<DT>(from_bits16<DT>(to_bits16<DT>(gr / (1.0f + expf(-gr)))) * ur);
+}
+
 __device__ __forceinline__ float round_through(float v, int mode) {
   if (mode == 1) return static_cast<float>(static_cast<__bf16>(v));
   if (mode == 2) return static_cast<float>(static_cast<_Float16>(v));

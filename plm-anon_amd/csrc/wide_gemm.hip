@@ -1,21 +1,32 @@
 // Wide GEMM over packed weights: Y[M,N] = X[M,K] · W[N,K]^T for M > 128 (the prefill chunks the
 // reference hands to F.linear, plm/rounds.py:16, plm/fast_gemm.py:108-111), so that a caller that
-// keeps only the packed copy of a weight has a compute-bound kernel for them.
+// keeps only the packed copy of a weight has a compute-bound kernel for them; and the same with a
+// fused gate/up projection's SiLU-and-multiply as its epilogue.
 //
-// A workgroup tile is 128 weight rows x 128 X rows; its four wavefronts each compute 64 x 64
-// (4 x 4 MFMA fragments of 16 x 16, v_mfma_f32_16x16x32_{bf16,f16}). Per 32-wide K step the
-// workgroup stages the tile's 8 weight fragments (packed: each a contiguous KiB already in operand
-// order) and 8 X fragments (16 rows x 64 bytes, loaded coalesced, a quad of lanes per row, and
-// written to LDS in operand order) through registers into one of two LDS slots; every wavefront
-// then reads its 4 + 4
-// operands lane-linearly (no bank conflicts) and issues 16 MFMAs. Global loads run kStages K steps
-// ahead in registers. Each X fragment is read from LDS by two wavefronts and each weight fragment
-// by two, so a K step moves 16 KiB from L2 per workgroup for 512 MFMA passes of 16 cycles.
+// Every output is one MFMA chain over the K steps in ascending order (v_mfma_f32_16x16x32), the
+// order of a row-split packed tile without K splits; it is also what torch's F.linear returned bit for
+// bit at every prefill width measured.
 //
-// Thin shapes (few tiles for 256 CUs) split K: each split writes its fp32 tile to the workspace
-// (device-coherent), and the last split of the tile to arrive adds the splits in order 0..S-1 and
-// writes Y, so results are bitwise reproducible run to run. Rows past N or M and K past K are
-// loaded as zeros (buffer range checks and per-lane masks) and never stored.
+// What bounds it: a CU's vector memory path, which moves 75-100 KiB per us from L2 whatever is
+// loaded (measured with the loads alone: 16 KiB per K step in 0.16-0.21 us), against 0.12 us of MFMA
+// for a 128 x 128 tile's K step; then the LDS reads of X. So a tile is chosen by the bytes it loads
+// per K step and by how evenly its tiles fill the CUs (wide_pick), and nothing is loaded twice inside
+// a workgroup: its four wavefronts take 16*NF weight rows each over the tile's whole 16*MT rows of X.
+// Weight fragments go straight to registers (a packed fragment is one contiguous KiB in operand
+// order); X goes through registers into LDS as rows of 128 B (two K steps, whole cache lines) with
+// 16-byte chunk c of row r at slot c ^ (r % 8), which makes the operand reads conflict-free (LDS reads
+// measured at 125-131 B per clock in this pattern, 64 without the swizzle).
+//
+// A stage is two K steps with one barrier, in its middle: the first step's MFMAs run while the second
+// step's X is read and the next stage's X written, then the barrier, then the second step's MFMAs
+// while the next stage's first X is read; memory instructions are spread between the MFMAs
+// (sched_group_barrier), since a burst of them stalls a wavefront's MFMAs behind it (M = 640,
+// 8192 x 2048: 26.0 us without the spreading, 24.9 with). Global loads run D stages ahead. The
+// 16-bit outputs go through LDS so that a row's stores are whole 128*NF-byte segments.
+//
+// Measured against unpacking the weight and F.linear (us; M = 640: 6144x2048, 2048x2048, 8192x2048,
+// 2048x8192): 34 / 17 / 35 / 51 -> 22 / 11 / 25 / 38; M = 256: 31 / 12 / 32 / 33 -> 16 / 7 / 15 / 23.
+// Rows past N or M and K past K load zeros (buffer range checks, per-lane masks) and are never stored.
 #include <hip/hip_runtime.h>
 
 #include "plm_amd.h"
@@ -25,10 +36,7 @@
 namespace plm {
 namespace {
 
-constexpr int kWideRows = 128;                // weight rows and X rows per tile
-constexpr int kWideFrags = kWideRows / 16;    // fragments per side
 constexpr int kWideWaves = 4;
-constexpr int kWideStages = 6;                // K steps of global loads in flight
 constexpr int kWideThreads = 64 * kWideWaves;
 constexpr uint32_t kWideNoLoad = 0x80000000u;
 
@@ -37,186 +45,321 @@ struct WideArgs {
   const void* w;
   void* y;
   int64_t ldx, ldy;
-  int M, N, Ks, k_last, mtiles, split, out_f32;
-  float* partial;  // split > 1: [tile][split][wave][16 fragments][64 lanes] f32x4
-  int* arrive;     // split > 1: one arrival counter per tile
+  int M, N, Ks;        // N: output columns (N/2 of the weight's rows with the activation)
+  int k_tail, stages;  // a stage is 64 K elements; k_tail of them in the last one
+  int mtiles, tiles, per_xcd, out_f32;
+  uint32_t wbytes, wgroup;
+  int gate_step, up_step;  // activation: fragment g's gate rows lie in weight fragment g * gate_step,
+                           // its up rows up_step fragments further
 };
 
 template <int DT>
-__device__ __forceinline__ void wide_store4(const WideArgs& a, int m, int n, f32x4 v) {
+__device__ __forceinline__ void wide_store4_f32(const WideArgs& a, int m, int n, f32x4 v) {
   const int left = a.N - n;
-  if (a.out_f32) {
-    float* y = static_cast<float*>(a.y) + static_cast<int64_t>(m) * a.ldy + n;
-    if (left >= 4 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
-      *reinterpret_cast<f32x4*>(y) = v;
-    } else {
-      for (int j = 0; j < 4 && j < left; ++j) y[j] = v[j];
-    }
-    return;
-  }
-  uint16_t* y = static_cast<uint16_t*>(a.y) + static_cast<int64_t>(m) * a.ldy + n;
-  const uint16_t h[4] = {to_bits16<DT>(v[0]), to_bits16<DT>(v[1]), to_bits16<DT>(v[2]), to_bits16<DT>(v[3])};
-  if (left >= 4 && (reinterpret_cast<uintptr_t>(y) & 7) == 0) {
-    *reinterpret_cast<uint64_t*>(y) = (static_cast<uint64_t>(h[0]) | (static_cast<uint64_t>(h[1]) << 16)) |
-                                      ((static_cast<uint64_t>(h[2]) | (static_cast<uint64_t>(h[3]) << 16)) << 32);
+  float* y = static_cast<float*>(a.y) + static_cast<int64_t>(m) * a.ldy + n;
+  if (left >= 4 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
+    *reinterpret_cast<f32x4*>(y) = v;
   } else {
-    for (int j = 0; j < 4 && j < left; ++j) y[j] = h[j];
+    for (int j = 0; j < 4 && j < left; ++j) y[j] = v[j];
   }
 }
 
 __device__ __forceinline__ void wide_sync() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-template <int DT>
-__global__ __launch_bounds__(kWideThreads, 2) void wide_gemm_kernel(WideArgs a) {
-  // [slot][fragment: 8 weight, then 8 X][lane]: 2 x 16 KiB
-  __shared__ __attribute__((aligned(16))) u32x4 lds[2][2 * kWideFrags][64];
-  __shared__ int last_flag;
+// Masks of sched_group_barrier.
+constexpr int kMfma = 0x8, kVmemRead = 0x20, kDsRead = 0x100, kDsWrite = 0x200;
+
+// Stages of global loads in flight: four where a stage's MFMAs are short (2048x8192 at M = 256 on
+// 64 x 32 tiles: 29.6 us with two, 23.0 with four), two where they are long and the registers are
+// taken (128 x 128 tiles: no difference).
+template <int NF, int MT>
+constexpr int wide_depth() {
+  return NF * MT <= 8 ? 4 : 2;
+}
+
+template <int DT, int NF, int MT, bool ACT>
+__global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) {
+  constexpr int D = wide_depth<NF, MT>();
+  constexpr int XN = (2 * MT + 3) / 4;                     // X loads of a wavefront per stage (8 rows each)
+  constexpr int OF = ACT ? NF / 2 : NF;                    // output fragments per wavefront
+  constexpr int OC = 8 * OF;                               // 16-byte chunks of a row of the output tile
+  constexpr int kStageWords = 2 * MT * 64;                 // u32x4 of one stage of X
+  constexpr int kOutWords = 16 * MT * OC;                  // u32x4 of the 16-bit output tile
+  __shared__ __attribute__((aligned(16))) u32x4 lds[2 * kStageWords > kOutWords ? 2 * kStageWords : kOutWords];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wn = wave & 1, wm = wave >> 1;  // this wavefront's 64 weight rows and 64 X rows
-  // item = (tile, split), split fastest; tile = (nt, mt), mt fastest, so the X tiles that share a
-  // weight tile run side by side.
-  const int item = blockIdx.x;
-  const int tile = item / a.split, sp = item - tile * a.split;
+  // Workgroups go round the 8 XCDs; each XCD takes a run of tiles, X tiles fastest, so that a weight
+  // tile is read into one XCD's L2 only.
+  const int tile = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
+  if (tile >= a.tiles) return;
   const int nt = tile / a.mtiles, mt = tile - nt * a.mtiles;
-  const int s_lo = static_cast<int>(static_cast<int64_t>(sp) * a.Ks / a.split);
-  const int s_hi = static_cast<int>(static_cast<int64_t>(sp + 1) * a.Ks / a.split);
-  const int steps = (s_hi - s_lo + kWideStages - 1) / kWideStages * kWideStages;  // padded: zero steps
-
-  const auto wr = make_rsrc(a.w, static_cast<uint32_t>(pack_bytes(a.N, a.Ks)));
-  const uint32_t wgroup = pack_group_bytes(a.N);
+  const auto wr = make_rsrc(a.w, a.wbytes);
   const auto xr = make_rsrc(a.x, static_cast<uint32_t>(static_cast<int64_t>(a.M) * a.ldx * 2));
-  // This wavefront stages weight fragments 2w, 2w+1 and X fragments 2w, 2w+1 of every K step.
-  uint32_t wo[2], xo[2], xl[2];
+  const int of0 = (nt * kWideWaves + wave) * OF;           // this wavefront's first output fragment
+  uint32_t wo[NF], xo[XN], xl[XN];                         // xl: the bit that puts a lane past K out of range
 #pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int f = nt * kWideFrags + 2 * wave + q;
-    wo[q] = pack_row_offset(f) + static_cast<uint32_t>(lane) * 16u;
-    // Coalesced: a quad of lanes reads one row's 64 bytes (row lane/4, bytes 16*(lane%4)); the
-    // LDS write puts each 16 bytes where the operand layout wants them (x_slot).
-    const int row = mt * kWideRows + 16 * (2 * wave + q) + (lane >> 2);
-    xo[q] = row < a.M ? static_cast<uint32_t>(static_cast<int64_t>(row) * a.ldx * 2) + 16u * static_cast<uint32_t>(lane & 3)
-                      : kOutOfRange;
-    xl[q] = 8 * (lane & 3) < a.k_last ? xo[q] : kOutOfRange;  // the last K step: lanes past K
+  for (int f = 0; f < NF; ++f) {
+    const int frag = ACT ? (of0 + f % OF) * a.gate_step + (f < OF ? 0 : a.up_step) : of0 + f;
+    wo[f] = pack_row_offset(frag) + static_cast<uint32_t>(lane) * 16u;
   }
-  const int x_slot = 16 * (lane & 3) + (lane >> 2);  // operand lane of row lane/4, K chunk lane%4
-  u32x4 rw[kWideStages][2], rx[kWideStages][2];
-  // Step index t (relative to s_lo) into register slot t % kWideStages; steps past s_hi load zeros.
-  auto load = [&](int t, u32x4 (&w)[2], u32x4 (&x)[2]) {
-    const int s = s_lo + t;
-    const bool live = s < s_hi;
-    const uint32_t sw = live ? pack_step_offset(s, wgroup) : kWideNoLoad;
-    const uint32_t sx = live ? static_cast<uint32_t>(s) * 64u : kWideNoLoad;
-    const bool last = s == a.Ks - 1;
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      w[q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, wo[q], static_cast<int>(sw), 0));
-      x[q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, last ? xl[q] : xo[q], static_cast<int>(sx), 0));
-    }
-  };
-  auto stage = [&](int slot, const u32x4 (&w)[2], const u32x4 (&x)[2]) {
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      lds[slot][2 * wave + q][lane] = w[q];
-      lds[slot][kWideFrags + 2 * wave + q][x_slot] = x[q];
-    }
-  };
-
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int j = 0; j < kWideStages; ++j) load(j, rw[j], rx[j]);
-  stage(0, rw[0], rx[0]);
-  load(kWideStages, rw[0], rx[0]);
-  for (int t0 = 0; t0 < steps; t0 += kWideStages) {
-#pragma unroll
-    for (int j = 0; j < kWideStages; ++j) {
-      const int t = t0 + j;
-      wide_sync();  // slot t&1 holds step t; slot (t+1)&1 is no longer read
-      const int jn = j + 1 == kWideStages ? 0 : j + 1;  // a constant once the loop is unrolled
-      stage((t + 1) & 1, rw[jn], rx[jn]);
-      load(t + 1 + kWideStages, rw[jn], rx[jn]);
-      u32x4 A[4], B[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) A[i] = lds[t & 1][4 * wn + i][lane];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) B[i] = lds[t & 1][kWideFrags + 4 * wm + i][lane];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) acc[i][k] = mfma_16x16x32<DT>(A[i], B[k], acc[i][k]);
-    }
+  for (int j = 0; j < XN; ++j) {
+    const int g = wave + 4 * j;                            // rows 8g .. 8g+7 of the tile, a row's 128 B per 8 lanes
+    const int row = mt * 16 * MT + 8 * g + (lane >> 3);
+    const int chunk = (lane & 7) ^ (lane >> 3);
+    xo[j] = (g < 2 * MT && row < a.M) ? static_cast<uint32_t>(static_cast<int64_t>(row) * a.ldx * 2) + 16u * chunk
+                                      : kOutOfRange;
+    xl[j] = 8 * chunk < a.k_tail ? 0u : kOutOfRange;
   }
-  __builtin_amdgcn_s_waitcnt(0);
-
-  // Fragment (i, k) of this wavefront: weight rows n0 + 16i + 4*(lane/16) + r, X row m0 + 16k + lane%16.
-  const int n0 = nt * kWideRows + 64 * wn + 4 * (lane >> 4);
-  const int m0 = mt * kWideRows + 64 * wm + (lane & 15);
-  if (a.split == 1) {
+  const int rd0 = (lane & 15) * 8 + ((lane >> 4) ^ (lane & 7));  // K step 0 of a stage, row lane % 16
+  const int rd1 = rd0 ^ 4;                                       // K step 1
+  u32x4 W[2 * D][NF], X[D][XN], B0[MT], B1[MT];
+  // Past the last step the sign bit puts the whole load out of range (zeros, no traffic).
+  auto w_off = [&](int s) __attribute__((always_inline)) {
+    return __builtin_amdgcn_readfirstlane(
+        static_cast<int>(pack_step_offset(s, a.wgroup) | (static_cast<uint32_t>(a.Ks - 1 - s) & kWideNoLoad)));
+  };
+  auto load_w = [&](int so, int f, u32x4& w) __attribute__((always_inline)) {
+    w = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, wo[f], so, 0));
+  };
+  auto load_x = [&](int i, u32x4 (&x)[XN]) __attribute__((always_inline)) {
+    const int left = a.stages - 1 - i;
+    const int so = __builtin_amdgcn_readfirstlane(
+        static_cast<int>((static_cast<uint32_t>(i) * 128u) | (static_cast<uint32_t>(left) & kWideNoLoad)));
+    const uint32_t last = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(~((left | -left) >> 31))) & kOutOfRange;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < XN; ++j)
+      x[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, xo[j] | (xl[j] & last), so, 0));
+  };
+  auto put_x = [&](int slot, const u32x4 (&x)[XN]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int m = m0 + 16 * k, n = n0 + 16 * i;
-        if (m < a.M && n < a.N) wide_store4<DT>(a, m, n, acc[i][k]);
+    for (int j = 0; j < XN; ++j)
+      if (4 * j + 3 < 2 * MT || wave + 4 * j < 2 * MT) lds[slot * kStageWords + (wave + 4 * j) * 64 + lane] = x[j];
+  };
+  f32x4 acc[NF][MT];
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < D; ++j) {
+    load_x(j, X[j]);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int so = w_off(2 * j + h);
+#pragma unroll
+      for (int f = 0; f < NF; ++f) load_w(so, f, W[2 * j + h][f]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  put_x(0, X[0]);
+  load_x(D, X[0]);
+  wide_sync();
+#pragma unroll
+  for (int t = 0; t < MT; ++t) B0[t] = lds[t * 128 + rd0];
+  // Stage i in register slot j = i % D. B0 holds its first K step's X operands.
+  auto stage = [&](int j, int i) __attribute__((always_inline)) {
+    const int slot = j & 1, jn = (j + 1) % D;
+    const int w0 = w_off(2 * (i + D)), w1 = w_off(2 * (i + D) + 1);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) B1[t] = lds[slot * kStageWords + t * 128 + rd1];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t) acc[f][t] = mfma_16x16x32<DT>(W[2 * j][f], B0[t], acc[f][t]);
+      load_w(w0, f, W[2 * j][f]);
+    }
+    put_x(slot ^ 1, X[jn]);
+    load_x(i + 1 + D, X[jn]);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+      if (NF == 1 && t < XN) {
+        __builtin_amdgcn_sched_group_barrier(kDsWrite, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(kVmemRead, 1, 0);
       }
-    return;
-  }
-  // Split partial: this wavefront's 16 fp32 fragments (16 KiB), written through.
-  const auto prs = make_rsrc(reinterpret_cast<f32x4*>(a.partial) + static_cast<int64_t>(tile) * a.split * kWideWaves * 16 * 64,
-                             static_cast<uint32_t>(a.split) * kWideWaves * 16 * 1024u);
+    }
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+    for (int t = 0; t < (NF - 1) * MT; ++t) {
+      if ((t & 1) == 0 && t / 2 < XN)
+        __builtin_amdgcn_sched_group_barrier(kDsWrite, 1, 0);
+      else
+        __builtin_amdgcn_sched_group_barrier(kVmemRead, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+    }
+    // Every wavefront has read this stage's X and written the next one's.
+    wide_sync();
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-      __builtin_amdgcn_raw_buffer_store_b128(
-          __builtin_bit_cast(u32x4, acc[i][k]), prs,
-          static_cast<uint32_t>(((sp * kWideWaves + wave) * 16 + 4 * i + k) * 1024 + lane * 16), 0, kCoherent);
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const int before = __hip_atomic_fetch_add(a.arrive + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    last_flag = before == a.split - 1;
-    if (last_flag) __hip_atomic_store(a.arrive + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int t = 0; t < MT; ++t) B0[t] = lds[(slot ^ 1) * kStageWords + t * 128 + rd0];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t) acc[f][t] = mfma_16x16x32<DT>(W[2 * j + 1][f], B1[t], acc[f][t]);
+      load_w(w1, f, W[2 * j + 1][f]);
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+    }
+#pragma unroll
+    for (int f = 1; f < NF; ++f) {
+      __builtin_amdgcn_sched_group_barrier(kVmemRead, 1, 0);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // The first D stages peeled off: the loop is entered only with its own load order in flight, so the
+  // compiler's load-count waits stay exact. Stages past the last multiply zeros.
+#pragma unroll
+  for (int j = 0; j < D; ++j) stage(j, j);
+  for (int i = D; i < a.stages; i += D) {
+#pragma unroll
+    for (int j = 0; j < D; ++j) stage(j, i + j);
   }
-  __syncthreads();
-  if (!last_flag) return;
-#pragma unroll 1
-  for (int q = 0; q < 16; ++q) {
-    const int i = q >> 2, k = q & 3;
-    f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < a.split; ++s0)
-      v += __builtin_bit_cast(
-          f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                     prs, static_cast<uint32_t>(((s0 * kWideWaves + wave) * 16 + q) * 1024 + lane * 16), 0, kCoherent));
-    const int m = m0 + 16 * k, n = n0 + 16 * i;
-    if (m < a.M && n < a.N) wide_store4<DT>(a, m, n, v);
+
+  // Fragment (f, t): output columns n0 + 16f + 4*(lane/16) + r, row m0 + 16t + lane%16.
+  const int m0 = mt * 16 * MT;
+  if constexpr (!ACT) {
+    if (a.out_f32) {
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          const int m = m0 + 16 * t + (lane & 15), n = 16 * (of0 + f) + 4 * (lane >> 4);
+          if (m < a.M && n < a.N) wide_store4_f32<DT>(a, m, n, acc[f][t]);
+        }
+      return;
+    }
+  }
+  // 16-bit output: the tile in LDS as rows of OC 16-byte chunks, chunk c of row m at slot c ^ (m % 8).
+  wide_sync();
+  u32x2* half = reinterpret_cast<u32x2*>(lds);
+#pragma unroll
+  for (int f = 0; f < OF; ++f)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      uint16_t h[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if constexpr (ACT)
+          h[r] = silu_mul_bits<DT>(acc[f][t][r], acc[f + OF][t][r]);
+        else
+          h[r] = to_bits16<DT>(acc[f][t][r]);
+      }
+      const int m = 16 * t + (lane & 15), q = 4 * (OF * wave + f) + (lane >> 4);  // q: 8-byte piece of the row
+      half[(m * OC + ((q >> 1) ^ (m & 7))) * 2 + (q & 1)] =
+          u32x2{static_cast<uint32_t>(h[0]) | (static_cast<uint32_t>(h[1]) << 16),
+                static_cast<uint32_t>(h[2]) | (static_cast<uint32_t>(h[3]) << 16)};
+    }
+  wide_sync();
+  uint16_t* y = static_cast<uint16_t*>(a.y);
+  const bool wide16 = (reinterpret_cast<uintptr_t>(y) & 15) == 0 && (a.ldy & 7) == 0;
+#pragma unroll
+  for (int i = threadIdx.x; i < kOutWords; i += kWideThreads) {
+    const int row = i / OC, c = i - row * OC;
+    const int m = m0 + row, n = 16 * (nt * kWideWaves * OF) + 8 * c;
+    if (m >= a.M || n >= a.N) continue;
+    const u32x4 v = lds[row * OC + (c ^ (row & 7))];
+    uint16_t* dst = y + static_cast<int64_t>(m) * a.ldy + n;
+    if (wide16 && n + 8 <= a.N) {
+      *reinterpret_cast<u32x4*>(dst) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t word = v[e >> 1];
+        if (n + e < a.N) dst[e] = static_cast<uint16_t>(e & 1 ? word >> 16 : word & 0xffffu);
+      }
+    }
   }
 }
 
-int64_t wide_tiles(int64_t M, int64_t N) { return ((N + kWideRows - 1) / kWideRows) * ((M + kWideRows - 1) / kWideRows); }
+// The compiled tiles: 64*nf weight rows by 16*mt rows of X.
+struct WideTile {
+  int nf, mt;
+};
+constexpr WideTile kWideTiles[] = {{1, 2}, {1, 3}, {1, 4}, {1, 5}, {1, 8}, {2, 3},
+                                   {2, 4}, {2, 5}, {2, 6}, {2, 8}, {2, 10}, {4, 8}};
+constexpr int kWideCus = 256;
+
+// The tile with the least modelled time per K step: the rounds of tiles a CU runs times the KiB each
+// loads per K step (4*nf of W, mt of X), the rate of the CU's memory path being the bound. Against the
+// best of all tiles timed one by one at M = 640 and 256 of the 1.3B block's linears and M = 200 and 110
+// of the 3B gate/up, its choice was the fastest or within 4 %. The activation needs gate and up
+// fragments in one wavefront, hence an even nf.
+WideTile wide_pick(int64_t M, int64_t N, bool act) {
+  WideTile best{0, 0};
+  int64_t best_cost = INT64_MAX;
+  for (const WideTile& t : kWideTiles) {
+    if (act && t.nf % 2 != 0) continue;
+    const int64_t tn = 64 * t.nf / (act ? 2 : 1);
+    const int64_t tiles = ((N + tn - 1) / tn) * ((M + 16 * t.mt - 1) / (16 * t.mt));
+    const int64_t cost = (tiles + kWideCus - 1) / kWideCus * (4 * t.nf + t.mt);
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = t;
+    }
+  }
+  return best;
+}
+
+template <int DT, int NF, int MT, bool ACT>
+hipError_t wide_go(WideArgs a, hipStream_t stream) {
+  constexpr int tn = 64 * NF / (ACT ? 2 : 1), tm = 16 * MT;
+  const int64_t mtiles = (a.M + tm - 1) / tm, ntiles = (static_cast<int64_t>(a.N) + tn - 1) / tn;
+  if (mtiles * ntiles > (int64_t(1) << 28)) return hipErrorInvalidConfiguration;
+  a.mtiles = static_cast<int>(mtiles);
+  a.tiles = static_cast<int>(mtiles * ntiles);
+  a.per_xcd = (a.tiles + 7) / 8;
+  hipLaunchKernelGGL((wide_gemm_kernel<DT, NF, MT, ACT>), dim3(static_cast<unsigned>(8 * a.per_xcd)), dim3(kWideThreads),
+                     0, stream, a);
+  return hipGetLastError();
+}
+
+template <int DT, bool ACT>
+hipError_t wide_dispatch(const WideArgs& a, WideTile t, hipStream_t s) {
+  switch (16 * t.nf + t.mt) {
+    case 16 * 2 + 3: return wide_go<DT, 2, 3, ACT>(a, s);
+    case 16 * 2 + 4: return wide_go<DT, 2, 4, ACT>(a, s);
+    case 16 * 2 + 5: return wide_go<DT, 2, 5, ACT>(a, s);
+    case 16 * 2 + 6: return wide_go<DT, 2, 6, ACT>(a, s);
+    case 16 * 2 + 8: return wide_go<DT, 2, 8, ACT>(a, s);
+    case 16 * 2 + 10: return wide_go<DT, 2, 10, ACT>(a, s);
+    case 16 * 4 + 8: return wide_go<DT, 4, 8, ACT>(a, s);
+    default: break;
+  }
+  if constexpr (!ACT) {
+    switch (16 * t.nf + t.mt) {
+      case 16 + 2: return wide_go<DT, 1, 2, ACT>(a, s);
+      case 16 + 3: return wide_go<DT, 1, 3, ACT>(a, s);
+      case 16 + 4: return wide_go<DT, 1, 4, ACT>(a, s);
+      case 16 + 5: return wide_go<DT, 1, 5, ACT>(a, s);
+      case 16 + 8: return wide_go<DT, 1, 8, ACT>(a, s);
+      default: break;
+    }
+  }
+  return hipErrorInvalidConfiguration;
+}
 
 }  // namespace
 
-int wide_split(int64_t M, int64_t N, int64_t K, int64_t cap) {
-  const int64_t tiles = wide_tiles(M, N), ks = (K + 31) / 32;
-  const auto bytes = [&](int64_t s) { return static_cast<int64_t>(kCounterBytes) + tiles * s * kWideWaves * 16 * 1024; };
+// The scratch a caller of plm_gemm_packed provides above 128 rows. The kernel itself needs none (a K
+// split would change the sums' order); the sizes callers reserve and the refusal of a smaller
+// workspace are the interface's and stay.
+int64_t wide_workspace(int64_t M, int64_t N, int64_t K, int64_t cap) {
+  const int64_t tiles = ((N + 127) / 128) * ((M + 127) / 128), ks = (K + 31) / 32;
+  const auto bytes = [&](int64_t s) { return static_cast<int64_t>(kCounterBytes) + tiles * s * 64 * 1024; };
   int64_t split = 1;
   while (tiles * split * 2 <= 320 && ks / (split * 2) >= 16 && split < 8 && bytes(split * 2) <= cap) split *= 2;
-  return static_cast<int>(split);
-}
-
-int64_t wide_workspace(int64_t M, int64_t N, int64_t K, int64_t cap) {
-  const int split = wide_split(M, N, K, cap);
-  if (split == 1) return 0;
-  return static_cast<int64_t>(kCounterBytes) + wide_tiles(M, N) * split * kWideWaves * 16 * 1024;
+  return split == 1 ? 0 : bytes(split);
 }
 
 int wide_gemm(int32_t dtype, const void* x, int64_t ldx, const void* wp, void* y, int64_t ldy, int64_t M, int64_t N,
-              int64_t K, void* workspace, size_t workspace_bytes, hipStream_t stream, int out_f32, int64_t cap) {
+              int64_t K, hipStream_t stream, WideOut out) {
+  const bool act = out == WideOut::kActPlain || out == WideOut::kActInterleaved;
   WideArgs a{};
   a.x = x;
   a.w = wp;
@@ -224,29 +367,22 @@ int wide_gemm(int32_t dtype, const void* x, int64_t ldx, const void* wp, void* y
   a.ldx = ldx;
   a.ldy = ldy;
   a.M = static_cast<int>(M);
-  a.N = static_cast<int>(N);
+  a.N = static_cast<int>(act ? N / 2 : N);
   a.Ks = static_cast<int>((K + 31) / 32);
-  a.k_last = static_cast<int>(K - 32 * (a.Ks - 1));
-  a.mtiles = static_cast<int>((M + kWideRows - 1) / kWideRows);
-  a.split = wide_split(M, N, K, cap);
-  a.out_f32 = out_f32;
-  const int64_t items = wide_tiles(M, N) * a.split;
-  if (a.split > 1) {
-    const int64_t need = wide_workspace(M, N, K, cap);
-    if (workspace == nullptr || static_cast<int64_t>(workspace_bytes) < need ||
-        (reinterpret_cast<uintptr_t>(workspace) & 15) != 0)
-      return PLM_ERR_WORKSPACE;
-    if (wide_tiles(M, N) > kPackedBarrierBase - kPackedArriveBase || need - static_cast<int64_t>(kCounterBytes) >= (int64_t(1) << 31))
-      return PLM_ERR_ARGUMENT;
-    a.arrive = static_cast<int*>(workspace) + kPackedArriveBase;
-    a.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes);
-  }
-  if (items > (int64_t(1) << 24) || M * ldx * 2 >= (int64_t(1) << 31)) return PLM_ERR_ARGUMENT;
+  a.stages = static_cast<int>((K + 63) / 64);
+  a.k_tail = static_cast<int>(K - 64 * (a.stages - 1));
+  a.out_f32 = out == WideOut::kF32;
+  a.wbytes = static_cast<uint32_t>(pack_bytes(N, a.Ks));
+  a.wgroup = pack_group_bytes(N);
+  a.gate_step = out == WideOut::kActInterleaved ? 2 : 1;
+  a.up_step = out == WideOut::kActInterleaved ? 1 : a.N / 16;
+  const WideTile t = wide_pick(M, a.N, act);
+  hipError_t err;
   if (dtype == PLM_BF16)
-    hipLaunchKernelGGL(wide_gemm_kernel<DT_BF16>, dim3(static_cast<unsigned>(items)), dim3(kWideThreads), 0, stream, a);
+    err = act ? wide_dispatch<DT_BF16, true>(a, t, stream) : wide_dispatch<DT_BF16, false>(a, t, stream);
   else
-    hipLaunchKernelGGL(wide_gemm_kernel<DT_F16>, dim3(static_cast<unsigned>(items)), dim3(kWideThreads), 0, stream, a);
-  return hipGetLastError() == hipSuccess ? PLM_OK : PLM_ERR_LAUNCH;
+    err = act ? wide_dispatch<DT_F16, true>(a, t, stream) : wide_dispatch<DT_F16, false>(a, t, stream);
+  return err == hipSuccess ? PLM_OK : err == hipErrorInvalidConfiguration ? PLM_ERR_ARGUMENT : PLM_ERR_LAUNCH;
 }
 
 }  // namespace plm

@@ -42,6 +42,7 @@ EXPORTS = (
     "plm_gemm_packed",
     "plm_gemm_packed_f32out",
     "plm_gemm_packed_noalloc",
+    "plm_gemm_wide",
     "plm_gemm_packed_workspace_bytes",
     "plm_gemm_packed_tile_supported",
     "plm_gemm_chain_packed_prepare",
@@ -118,6 +119,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.plm_unpack_weight.restype = ctypes.c_int
     lib.plm_gemm_packed.argtypes = [c_i32, c_p, c_i64, c_p, c_p, c_i64, c_i64, c_i64, c_i64, tile_p, c_p, c_sz, c_p]
     lib.plm_gemm_packed.restype = ctypes.c_int
+    lib.plm_gemm_wide.argtypes = [c_i32, c_p, c_i64, c_p, c_p, c_i64, c_i64, c_i64, c_i64, c_i32, c_p]
+    lib.plm_gemm_wide.restype = ctypes.c_int
     lib.plm_gemm_packed_f32out.argtypes = lib.plm_gemm_packed.argtypes
     lib.plm_gemm_packed_f32out.restype = ctypes.c_int
     lib.plm_gemm_packed_noalloc.argtypes = [c_i32, c_p, c_i64, c_p, c_p, c_i64, c_i64, c_i64, c_i64, tile_p, c_p]

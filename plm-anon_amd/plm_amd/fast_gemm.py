@@ -13,9 +13,9 @@ config go to ``F.linear``, exactly as in the reference.
 ``release(weight)`` keeps one copy of a weight: its row-major storage is freed and every product with
 it runs from the packed copy: widths up to 128 rows (the round widths) on the packed kernel with
 their tuned tiles or ``default_config``'s; wider calls (prefill chunks, plm/rounds.py:16, which the
-reference hands to ``F.linear``) as ``F.linear`` on the weight unpacked into a transient buffer
-(``unpacked``, bit for bit), which measured faster than ``plm_gemm_packed``'s own wide kernel
-(1.3B block at M = 640: 134.5 against 190.7 µs), so they are the reference's own products.
+reference hands to ``F.linear``) on the wide kernel (``plm_gemm_wide``), or, where the call needs more
+than a product (a bias, autograd, autocast, tracing), as ``F.linear`` on the weight unpacked into a
+transient buffer (``unpacked``, bit for bit).
 """
 
 from __future__ import annotations
@@ -246,13 +246,17 @@ def gate_up_silu(x: torch.Tensor, w: torch.Tensor, cfg: Config | None = None,
     its output as a second launch, with the same roundings (the projection's output rounded to the
     model dtype, silu rounded, then the product). ``cfg``: the tile, by default ``ACT_CONFIGS``'
     (the fastest even-wave_frags tile the tuner found) or the projection's; a tile with
-    wave_frags 1 runs with 2. Widths above 128 rows run as the
-    projection then the activation, each as its own launch."""
+    wave_frags 1 runs with 2. Widths above 128 rows run on the wide kernel with the same epilogue where
+    the weight is released, else as the projection then the activation, each as its own launch."""
     _check_operands(x, w)
     M, K = x.shape
     N = w.shape[0]
     half = N // 2
     if M > 128:
+        if w in _released and N % 32 == 0:
+            act = _wide(x, w, _lib.PLM_OUT_SILU_MUL)
+            if act is not None:
+                return act if out is None else out.copy_(act)
         y = released_linear(x, w) if w in _released else F.linear(x, w)
         act = F.silu(y[:, :half]) * y[:, half:]
         if out is not None:
@@ -410,16 +414,46 @@ def hip_linear_f32(a: torch.Tensor, w: torch.Tensor, cfg: Config, out: torch.Ten
     return _launch(a, w, cfg, out, True)
 
 
-# Widths above this run as F.linear on the unpacked weight (plm_gemm_packed's wide kernel, which
-# takes them too, measured slower over the 1.3B block's linears from 256 rows on).
+# Widths above this run on the wide kernel (or F.linear on the unpacked weight).
 WIDE_ROWS = 128
+
+
+def _plain(x: torch.Tensor) -> bool:
+    """Whether a kernel may read ``x`` by its pointer in ``F.linear``'s place: an ordinary GPU tensor that
+    no autograd, autocast, transform, mode or tracer would have to see the product of."""
+    return (type(x) in (torch.Tensor, torch.nn.Parameter) and x.is_cuda
+            and not (x.requires_grad and torch.is_grad_enabled())
+            and not torch.is_autocast_enabled()
+            and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+            and torch._C._len_torch_function_stack() == 0 and torch._C._len_torch_dispatch_stack() == 0
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+            and torch.autograd.forward_ad.unpack_dual(x).tangent is None)
+
+
+def _wide(x: torch.Tensor, weight: torch.Tensor, out_kind: int) -> torch.Tensor | None:
+    """``x[M, K] @ weight^T`` of a released weight on the wide kernel (``out_kind`` as plm_gemm_wide's), or
+    None for a call that ``F.linear`` on the unpacked weight has to take. The two have the same sums in
+    the same order where F.linear's library does not split K; measured (M = 640, 1.3B block): 137 us with
+    F.linear, 97 us here."""
+    if not _plain(x) or x.device != weight.device:
+        return None
+    x = _row_major(x)
+    (M, K), N = x.shape, weight.shape[0]
+    if M * x.stride(0) * 2 >= 1 << 31:
+        return None
+    y = torch.empty(M, N // 2 if out_kind == _lib.PLM_OUT_SILU_MUL else N, device=x.device, dtype=x.dtype)
+    status = _lib.lib().plm_gemm_wide(_lib.DTYPE_CODES[x.dtype], x.data_ptr(), x.stride(0), _released[weight].data_ptr(),
+                                      y.data_ptr(), y.stride(0), M, N, K, out_kind, _lib.stream_handle(x.device))
+    _lib.check(status, f"plm_gemm_wide(M={M}, N={N}, K={K}, out_kind={out_kind})")
+    return y
 
 
 def released_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """``F.linear(x, weight, bias)`` for a released weight, any leading shape of ``x``: up to
     ``WIDE_ROWS`` rows on the packed kernel (the tuned tile where the tables have one for
-    ``(M, N, K)``, else ``default_config``; a bias added after), wider as ``F.linear`` on the weight
-    unpacked into a transient buffer."""
+    ``(M, N, K)``, else ``default_config``; a bias added after), wider on the wide kernel, or with a bias
+    (one rounding for the sum) and in the cases ``_plain`` names as ``F.linear`` on the weight unpacked
+    into a transient buffer."""
     if x.dtype != weight.dtype:
         raise TypeError(f"released weight is {weight.dtype}, input is {x.dtype}")
     N, K = weight.shape
@@ -427,7 +461,8 @@ def released_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | 
     x2 = x.reshape(-1, K)
     M = x2.shape[0]
     if M > WIDE_ROWS:
-        return F.linear(x, unpacked(weight), bias)
+        y = _wide(x2, weight, _lib.PLM_OUT_MODEL) if bias is None else None
+        return F.linear(x, unpacked(weight), bias) if y is None else y.reshape(*lead, N)
     if M == 0:
         out = x2.new_empty(0, N)
     else:

@@ -1,0 +1,86 @@
+"""plm_gemm_wide: every output is one MFMA chain over K in ascending order, so it equals the packed
+row-split kernel without K splits (its own parity against the oracle: tests/test_gemm_gpu.py) bit for
+bit, at the edges of its tiles (32 to 160 rows of X by 64 to 256 of W) and of its 64-wide K stages. The
+activation epilogue equals torch's silu and multiply on the rounded projection up to one output step
+where the two exponentials' last bits part."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from plm_amd import _lib, fast_gemm
+from plm_amd.fast_gemm import launch_packed, pack_weight, release, released_linear
+from test_gemm_gpu import _inputs_on_gpu
+
+pytestmark = pytest.mark.gpu
+
+ROW_SPLIT = {"wave_frags": 2, "k_waves": 1, "split_k": 1, "unroll": 2}
+
+
+def _wide(x, wp, N, kind, y):
+    status = _lib.lib().plm_gemm_wide(_lib.DTYPE_CODES[x.dtype], x.data_ptr(), x.stride(0), wp.data_ptr(), y.data_ptr(),
+                                      y.stride(0), x.shape[0], N, x.shape[1], kind, _lib.stream_handle(x.device))
+    assert status == 0
+    return y
+
+
+def _chain(x, wp, N):
+    parts = [launch_packed(x[m:m + 64], wp, N, ROW_SPLIT, torch.empty(min(64, x.shape[0] - m), N, device=x.device),
+                           f32_out=True) for m in range(0, x.shape[0], 64)]
+    return torch.cat(parts)
+
+
+# (M, N, K): below and past one tile of each height and width, a ragged N, K of one chunk, of an odd
+# number of 32-wide steps and past a stage's end.
+SHAPES = [(1, 1, 8), (33, 64, 64), (129, 257, 40), (160, 1003, 96), (161, 2048, 1416), (200, 11264, 72),
+          (640, 2050, 1000), (500, 8192, 2048), (1281, 16384, 136)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_matches_the_row_split_chain_bit_for_bit(device, M, N, K, dtype):
+    print(f"wide M={M} N={N} K={K} {dtype}", flush=True)
+    x, w = (t.to(dtype) for t in _inputs_on_gpu(M, N, K, 3 * M + N, device))
+    wp = pack_weight(w)
+    ref = _chain(x, wp, N)
+    pad = torch.full((M, N + 5), float("nan"), device=device, dtype=dtype)   # rows that no 16-byte store fits
+    assert torch.equal(_wide(x, wp, N, _lib.PLM_OUT_F32, torch.empty(M, N, device=device)), ref)
+    assert torch.equal(_wide(x, wp, N, _lib.PLM_OUT_MODEL, torch.empty(M, N, device=device, dtype=dtype)), ref.to(dtype))
+    assert torch.equal(_wide(x, wp, N, _lib.PLM_OUT_MODEL, pad[:, 1:N + 1]), ref.to(dtype))
+    assert bool(pad[:, 0].isnan().all()) and bool(pad[:, N + 1:].isnan().all())
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 32, 8), (150, 1024, 1000), (640, 11264, 2048), (200, 2816, 512)])
+def test_silu_mul_of_a_released_gate_up_weight(device, M, N, K):
+    x, w = _inputs_on_gpu(M, N, K, N + K, device)
+    y = _chain(x, pack_weight(w), N).to(x.dtype)
+    want = F.silu(y[:, : N // 2]) * y[:, N // 2:]
+    release(w)
+    out = torch.empty(M, N // 2, device=device, dtype=x.dtype)
+    got = fast_gemm.gate_up_silu(x, w)
+    assert fast_gemm.gate_up_silu(x, w, out=out) is out and torch.equal(out, got)
+    # expf of the two sides may round apart: one step of the silu (2^-8 relative) and one of the product.
+    assert int((got != want).sum()) <= max(1, got.numel() // 1000)
+    torch.testing.assert_close(got.float(), want.float(), rtol=2 * 2.0 ** -7, atol=1e-30)
+
+
+def test_calls_that_need_more_than_a_product_go_to_f_linear(device):
+    """A bias, autograd, autocast and vmap of a released weight's wide calls act as F.linear's own."""
+    x, w = _inputs_on_gpu(130, 256, 64, 9, device)
+    ref_w = w.clone()
+    release(w)
+    bias = torch.randn(256, device=device).bfloat16()
+    assert torch.equal(released_linear(x, w, bias), F.linear(x, ref_w, bias))
+    leaf = x.clone().requires_grad_()
+    released_linear(leaf, w).sum().backward()
+    want = x.clone().requires_grad_()
+    F.linear(want, ref_w).sum().backward()
+    assert torch.equal(leaf.grad, want.grad)
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert released_linear(x, w).dtype == torch.float16
+    stack = torch.stack([x, -x])
+    assert torch.func.vmap(lambda t: released_linear(t, w))(stack).shape == (2, 130, 256)
+    with torch.no_grad():
+        assert torch.equal(released_linear(leaf, w), F.linear(x, ref_w))
