@@ -181,6 +181,36 @@ int packed_launch_args(int32_t dtype, PackedArgs& a, const plm_tile& t, void* wo
   return packed_dispatch_dt(dtype, a, t, cus, s, false, epi) == hipSuccess ? PLM_OK : PLM_ERR_LAUNCH;
 }
 
+// Whether a single linear on a row-split tile (k_waves = 1) runs on the wide kernel, whose sums are the
+// row-split kernel's bit for bit: weights below 128 MiB, or widths above 64 rows. There the wide
+// kernel's X, read once per workgroup into LDS, and its smaller tiles win (us, best tile of the packed
+// kernel against it: M = 56, 6144x2048 11.9 / 8.8, 16384x3072 24.1 / 20.8; M = 110, 3072x3072 17.4 /
+// 11.0, 50257x2048 62.0 / 48.2); a longer stream at few rows is bound by HBM either way and the
+// row-split kernel's deeper pipeline is level or ahead (50257x2048: M = 7 40.2 / 41.4, M = 56 46.6 / 46.7).
+bool wide_preferred(int64_t M, int64_t N, int64_t K, const plm_tile& t) {
+  if (t.k_waves != 1 || (M <= 64 && packed_bytes(N, K) >= (int64_t(128) << 20))) return false;
+  // Split partials lie behind one 32-bit buffer range.
+  return t.split_k == 1 || t.split_k * ((N + 15) / 16) * ((M + 15) / 16) * kFragBytes < (int64_t(1) << 31);
+}
+
+// The wide kernel in a row-split tile's place, with that tile's refusals; kNotRun if the shape has more
+// tiles than the kernel takes.
+constexpr int kNotRun = 1;
+int wide_in_place(int32_t dtype, const plm_chain_gemm& g, int64_t M, const plm_tile& t, WideOut out, void* workspace,
+                  size_t workspace_bytes, void* stream) {
+  const int64_t need = packed_workspace(M, g.N, t);
+  if (need > 0 && (workspace == nullptr || static_cast<int64_t>(workspace_bytes) < need ||
+                   (reinterpret_cast<uintptr_t>(workspace) & 15) != 0))
+    return PLM_ERR_WORKSPACE;
+  PackedArgs a{};
+  a.M = static_cast<int>(M);
+  const int epi = out == WideOut::kActInterleaved ? kEpiAct : kEpiPlain;
+  if (packed_dispatch_dt(dtype, a, t, 1, nullptr, true, epi) != hipSuccess) return PLM_ERR_TILE;
+  const int status = wide_gemm(dtype, g.x, g.ldx, g.w, g.y, g.ldy, M, g.N, g.K, static_cast<hipStream_t>(stream), out,
+                               t.split_k, workspace);
+  return status == PLM_ERR_ARGUMENT ? kNotRun : status;
+}
+
 int packed_entry(int32_t dtype, const void* x, int64_t ldx, const void* wp, void* y, int64_t ldy, int64_t M, int64_t N,
                  int64_t K, const plm_tile* tile, void* workspace, size_t workspace_bytes, void* stream, int out_f32) {
   if (!packed_tile_valid(tile)) return PLM_ERR_TILE;
@@ -202,6 +232,11 @@ int packed_entry(int32_t dtype, const void* x, int64_t ldx, const void* wp, void
   if (status != PLM_OK) return status;
   const int64_t tiles = packed_tiles(N, t);
   if (t.split_k > 1 && tiles > kPackedBarrierBase - kPackedArriveBase) return PLM_ERR_ARGUMENT;
+  if (wide_preferred(M, N, K, t)) {
+    const int ran = wide_in_place(dtype, g, M, t, out_f32 ? WideOut::kF32 : WideOut::kModel, workspace, workspace_bytes,
+                                  stream);
+    if (ran != kNotRun) return ran;
+  }
   g.arrive_base = kPackedArriveBase;
   PackedArgs a{};
   a.single = g;
@@ -594,6 +629,10 @@ int plm_gemm_packed_silu_mul(int32_t dtype, const void* x, int64_t ldx, const vo
   if (status != PLM_OK) return status;
   const int64_t tiles = plm::packed_tiles(N, t);
   if (t.split_k > 1 && tiles > plm::kPackedBarrierBase - plm::kPackedArriveBase) return PLM_ERR_ARGUMENT;
+  if (plm::wide_preferred(M, N, K, t)) {
+    const int ran = plm::wide_in_place(dtype, g, M, t, plm::WideOut::kActInterleaved, workspace, workspace_bytes, stream);
+    if (ran != plm::kNotRun) return ran;
+  }
   g.arrive_base = plm::kPackedArriveBase;
   plm::PackedArgs a{};
   a.single = g;

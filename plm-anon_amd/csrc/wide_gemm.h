@@ -18,8 +18,10 @@ int64_t wide_workspace(int64_t M, int64_t N, int64_t K, int64_t cap = kNoCap);
 // fused gate/up weight packed as it is (gate rows first) or with its halves interleaved by fragment.
 enum class WideOut { kModel, kF32, kActPlain, kActInterleaved };
 
-// Y = X W^T; returns a PLM_* status.
+// Y = X W^T; returns a PLM_* status. With split > 1 each of `split` ranges of K steps is one chain and
+// the ranges' sums are added in order (the sums of a row-split packed tile with that split_k, bit for
+// bit); `workspace` then holds the counter area and split * ceil(N/16) * ceil(M/16) fp32 fragments.
 int wide_gemm(int32_t dtype, const void* x, int64_t ldx, const void* wp, void* y, int64_t ldy, int64_t M, int64_t N,
-              int64_t K, hipStream_t stream, WideOut out);
+              int64_t K, hipStream_t stream, WideOut out, int split = 1, void* workspace = nullptr);
 
 }  // namespace plm

@@ -1,11 +1,13 @@
 // Wide GEMM over packed weights: Y[M,N] = X[M,K] · W[N,K]^T for M > 128 (the prefill chunks the
 // reference hands to F.linear, plm/rounds.py:16, plm/fast_gemm.py:108-111), so that a caller that
-// keeps only the packed copy of a weight has a compute-bound kernel for them; and the same with a
-// fused gate/up projection's SiLU-and-multiply as its epilogue.
+// keeps only the packed copy of a weight has a compute-bound kernel for them; for single linears of a
+// round on row-split tiles (packed_api.hip, wide_preferred), where its X, read once per workgroup, beats
+// the packed kernel's; and both with a fused gate/up projection's SiLU-and-multiply as the epilogue.
 //
 // Every output is one MFMA chain over the K steps in ascending order (v_mfma_f32_16x16x32), the
 // order of a row-split packed tile without K splits; it is also what torch's F.linear returned bit for
-// bit at every prefill width measured.
+// bit at every prefill width measured. With K splits each range is such a chain and the ranges' sums
+// are added in order, as the packed kernel does.
 //
 // What bounds it: a CU's vector memory path, which moves 75-100 KiB per us from L2 whatever is
 // loaded (measured with the loads alone: 16 KiB per K step in 0.16-0.21 us), against 0.12 us of MFMA
@@ -26,7 +28,9 @@
 //
 // Measured against unpacking the weight and F.linear (us; M = 640: 6144x2048, 2048x2048, 8192x2048,
 // 2048x8192): 34 / 17 / 35 / 51 -> 22 / 11 / 25 / 38; M = 256: 31 / 12 / 32 / 33 -> 16 / 7 / 15 / 23.
-// Rows past N or M and K past K load zeros (buffer range checks, per-lane masks) and are never stored.
+// Rounds, against the packed kernel's best tile (us; 6144x2048, 2048x2048, 8192x2048, 2048x8192 split 4):
+// M = 56 12.8 / 9.5 / 13.6 / 15.8 -> 9.6 / 7.5 / 10.2 / 14.1, M = 110 18.4 / 12.1 / 19.2 / 21.8 -> 11.5 /
+// 7.9 / 12.0 / 16.6. Rows past N or M and K past K load zeros (buffer range checks, per-lane masks) and are never stored.
 #include <hip/hip_runtime.h>
 
 #include "plm_amd.h"
@@ -46,9 +50,11 @@ struct WideArgs {
   void* y;
   int64_t ldx, ldy;
   int M, N, Ks;        // N: output columns (N/2 of the weight's rows with the activation)
-  int k_tail, stages;  // a stage is 64 K elements; k_tail of them in the last one
   int mtiles, tiles, per_xcd, out_f32;
   uint32_t wbytes, wgroup;
+  int K, split;            // split > 1: an item is a tile and one of `split` ranges of K steps
+  float* partial;          // split > 1: fp32 fragments [split][weight fragments][X fragments][64 lanes]
+  int* arrive;             // split > 1: one arrival counter per tile
   int gate_step, up_step;  // activation: fragment g's gate rows lie in weight fragment g * gate_step,
                            // its up rows up_step fragments further
 };
@@ -88,11 +94,18 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
   __shared__ __attribute__((aligned(16))) u32x4 lds[2 * kStageWords > kOutWords ? 2 * kStageWords : kOutWords];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // Workgroups go round the 8 XCDs; each XCD takes a run of tiles, X tiles fastest, so that a weight
-  // tile is read into one XCD's L2 only.
-  const int tile = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
-  if (tile >= a.tiles) return;
-  const int nt = tile / a.mtiles, mt = tile - nt * a.mtiles;
+  // Workgroups go round the 8 XCDs; each XCD takes a run of items, X tiles fastest, then splits, so
+  // that a weight tile is read into one XCD's L2 only.
+  const int item = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
+  if (item >= a.tiles * a.split) return;
+  const int ns = item / a.mtiles, mt = item - ns * a.mtiles;
+  const int nt = a.split == 1 ? ns : ns / a.split, sp = ns - nt * a.split;
+  // K steps [lo, hi), stages of two from lo; k_tail of the last stage's 64 K elements are real.
+  const int lo = a.split == 1 ? 0 : static_cast<int>(static_cast<uint32_t>(sp * a.Ks) / static_cast<uint32_t>(a.split));
+  const int hi = a.split == 1 ? a.Ks
+                              : static_cast<int>(static_cast<uint32_t>((sp + 1) * a.Ks) / static_cast<uint32_t>(a.split));
+  const int stages = (hi - lo + 1) >> 1;
+  const int k_tail = min(a.K, 32 * hi) - 32 * lo - 64 * (stages - 1);
   const auto wr = make_rsrc(a.w, a.wbytes);
   const auto xr = make_rsrc(a.x, static_cast<uint32_t>(static_cast<int64_t>(a.M) * a.ldx * 2));
   const int of0 = (nt * kWideWaves + wave) * OF;           // this wavefront's first output fragment
@@ -109,23 +122,23 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
     const int chunk = (lane & 7) ^ (lane >> 3);
     xo[j] = (g < 2 * MT && row < a.M) ? static_cast<uint32_t>(static_cast<int64_t>(row) * a.ldx * 2) + 16u * chunk
                                       : kOutOfRange;
-    xl[j] = 8 * chunk < a.k_tail ? 0u : kOutOfRange;
+    xl[j] = 8 * chunk < k_tail ? 0u : kOutOfRange;
   }
   const int rd0 = (lane & 15) * 8 + ((lane >> 4) ^ (lane & 7));  // K step 0 of a stage, row lane % 16
   const int rd1 = rd0 ^ 4;                                       // K step 1
   u32x4 W[2 * D][NF], X[D][XN], B0[MT], B1[MT];
   // Past the last step the sign bit puts the whole load out of range (zeros, no traffic).
   auto w_off = [&](int s) __attribute__((always_inline)) {
-    return __builtin_amdgcn_readfirstlane(
-        static_cast<int>(pack_step_offset(s, a.wgroup) | (static_cast<uint32_t>(a.Ks - 1 - s) & kWideNoLoad)));
+    return __builtin_amdgcn_readfirstlane(static_cast<int>(
+        pack_step_offset(lo + s, a.wgroup) | (static_cast<uint32_t>(hi - lo - 1 - s) & kWideNoLoad)));
   };
   auto load_w = [&](int so, int f, u32x4& w) __attribute__((always_inline)) {
     w = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, wo[f], so, 0));
   };
   auto load_x = [&](int i, u32x4 (&x)[XN]) __attribute__((always_inline)) {
-    const int left = a.stages - 1 - i;
+    const int left = stages - 1 - i;
     const int so = __builtin_amdgcn_readfirstlane(
-        static_cast<int>((static_cast<uint32_t>(i) * 128u) | (static_cast<uint32_t>(left) & kWideNoLoad)));
+        static_cast<int>((static_cast<uint32_t>(i) * 128u + static_cast<uint32_t>(lo) * 64u) | (static_cast<uint32_t>(left) & kWideNoLoad)));
     const uint32_t last = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(~((left | -left) >> 31))) & kOutOfRange;
 #pragma unroll
     for (int j = 0; j < XN; ++j)
@@ -216,9 +229,71 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
   // compiler's load-count waits stay exact. Stages past the last multiply zeros.
 #pragma unroll
   for (int j = 0; j < D; ++j) stage(j, j);
-  for (int i = D; i < a.stages; i += D) {
+  for (int i = D; i < stages; i += D) {
 #pragma unroll
     for (int j = 0; j < D; ++j) stage(j, i + j);
+  }
+
+  if (a.split > 1) {
+    // This split's sums, written through; the last of the tile's splits to arrive adds all of them in
+    // split order. Weight fragment wf of the packed order, X fragment xf; fragments past N or M are
+    // neither stored nor loaded (out of range).
+    const int wfrags = ((ACT ? 2 * a.N : a.N) + 15) >> 4, xfrags = (a.M + 15) >> 4;
+    const auto pr = make_rsrc(a.partial, static_cast<uint32_t>(a.split * wfrags * xfrags) * 1024u);
+    uint32_t po[NF];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const int wf = ACT ? 2 * (of0 + f % OF) + f / OF : of0 + f;
+      po[f] = wf < wfrags ? static_cast<uint32_t>(wf * xfrags + mt * MT) * 1024u + static_cast<uint32_t>(lane) * 16u
+                          : kOutOfRange;
+    }
+    const uint32_t plane = static_cast<uint32_t>(wfrags * xfrags) * 1024u;
+    const int mts = min(MT, xfrags - mt * MT);
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        if (t < mts)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[f][t]), pr, po[f] + t * 1024u,
+                                                 static_cast<int>(static_cast<uint32_t>(sp) * plane), kCoherent);
+    __builtin_amdgcn_s_waitcnt(0);
+    wide_sync();  // every wavefront's partials are written, and no one reads X in LDS any more
+    if (threadIdx.x == 0) {
+      int* counter = a.arrive + nt * a.mtiles + mt;
+      const int before = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const bool last = before == a.split - 1;
+      if (last) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      lds[0][0] = last;
+    }
+    wide_sync();
+    if (lds[0][0] == 0) return;
+    // Four splits' loads in flight at a time (two where a wavefront holds many fragments).
+    constexpr int kBatch = NF * MT <= 8 ? 4 : 2;
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < a.split; s0 += kBatch) {
+      u32x4 v[kBatch][NF][MT];
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b) {
+        const int so = static_cast<int>(s0 + b < a.split ? static_cast<uint32_t>(s0 + b) * plane : kWideNoLoad);
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+          for (int t = 0; t < MT; ++t)
+            v[b][f][t] = __builtin_bit_cast(
+                u32x4, __builtin_amdgcn_raw_buffer_load_b128(pr, t < mts ? po[f] + t * 1024u : kOutOfRange, so, kCoherent));
+      }
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b) {
+        if (s0 + b >= a.split) break;
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+          for (int t = 0; t < MT; ++t) acc[f][t] += __builtin_bit_cast(f32x4, v[b][f][t]);
+      }
+    }
   }
 
   // Fragment (f, t): output columns n0 + 16f + 4*(lane/16) + r, row m0 + 16t + lane%16.
@@ -281,22 +356,23 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
 struct WideTile {
   int nf, mt;
 };
-constexpr WideTile kWideTiles[] = {{1, 2}, {1, 3}, {1, 4}, {1, 5}, {1, 8}, {2, 3},
-                                   {2, 4}, {2, 5}, {2, 6}, {2, 8}, {2, 10}, {4, 8}};
+constexpr WideTile kWideTiles[] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {1, 5}, {1, 8}, {2, 1}, {2, 2},
+                                   {2, 3}, {2, 4}, {2, 5}, {2, 6}, {2, 8}, {2, 10}, {4, 8}};
 constexpr int kWideCus = 256;
 
 // The tile with the least modelled time per K step: the rounds of tiles a CU runs times the KiB each
 // loads per K step (4*nf of W, mt of X), the rate of the CU's memory path being the bound. Against the
 // best of all tiles timed one by one at M = 640 and 256 of the 1.3B block's linears and M = 200 and 110
-// of the 3B gate/up, its choice was the fastest or within 4 %. The activation needs gate and up
+// of the 3B gate/up, its choice was the fastest or within 4 %; M = 7 to 110 of the round linears within
+// 10 % (a few of the shortest, by 0.1-0.3 us). The activation needs gate and up
 // fragments in one wavefront, hence an even nf.
-WideTile wide_pick(int64_t M, int64_t N, bool act) {
+WideTile wide_pick(int64_t M, int64_t N, int64_t split, bool act) {
   WideTile best{0, 0};
   int64_t best_cost = INT64_MAX;
   for (const WideTile& t : kWideTiles) {
     if (act && t.nf % 2 != 0) continue;
     const int64_t tn = 64 * t.nf / (act ? 2 : 1);
-    const int64_t tiles = ((N + tn - 1) / tn) * ((M + 16 * t.mt - 1) / (16 * t.mt));
+    const int64_t tiles = ((N + tn - 1) / tn) * ((M + 16 * t.mt - 1) / (16 * t.mt)) * split;
     const int64_t cost = (tiles + kWideCus - 1) / kWideCus * (4 * t.nf + t.mt);
     if (cost < best_cost) {
       best_cost = cost;
@@ -310,10 +386,11 @@ template <int DT, int NF, int MT, bool ACT>
 hipError_t wide_go(WideArgs a, hipStream_t stream) {
   constexpr int tn = 64 * NF / (ACT ? 2 : 1), tm = 16 * MT;
   const int64_t mtiles = (a.M + tm - 1) / tm, ntiles = (static_cast<int64_t>(a.N) + tn - 1) / tn;
-  if (mtiles * ntiles > (int64_t(1) << 28)) return hipErrorInvalidConfiguration;
+  if (mtiles * ntiles * a.split > (int64_t(1) << 28)) return hipErrorInvalidConfiguration;
+  if (a.split > 1 && mtiles * ntiles > kPackedBarrierBase - kPackedArriveBase) return hipErrorInvalidConfiguration;
   a.mtiles = static_cast<int>(mtiles);
   a.tiles = static_cast<int>(mtiles * ntiles);
-  a.per_xcd = (a.tiles + 7) / 8;
+  a.per_xcd = (a.tiles * a.split + 7) / 8;
   hipLaunchKernelGGL((wide_gemm_kernel<DT, NF, MT, ACT>), dim3(static_cast<unsigned>(8 * a.per_xcd)), dim3(kWideThreads),
                      0, stream, a);
   return hipGetLastError();
@@ -322,6 +399,8 @@ hipError_t wide_go(WideArgs a, hipStream_t stream) {
 template <int DT, bool ACT>
 hipError_t wide_dispatch(const WideArgs& a, WideTile t, hipStream_t s) {
   switch (16 * t.nf + t.mt) {
+    case 16 * 2 + 1: return wide_go<DT, 2, 1, ACT>(a, s);
+    case 16 * 2 + 2: return wide_go<DT, 2, 2, ACT>(a, s);
     case 16 * 2 + 3: return wide_go<DT, 2, 3, ACT>(a, s);
     case 16 * 2 + 4: return wide_go<DT, 2, 4, ACT>(a, s);
     case 16 * 2 + 5: return wide_go<DT, 2, 5, ACT>(a, s);
@@ -333,6 +412,7 @@ hipError_t wide_dispatch(const WideArgs& a, WideTile t, hipStream_t s) {
   }
   if constexpr (!ACT) {
     switch (16 * t.nf + t.mt) {
+      case 16 + 1: return wide_go<DT, 1, 1, ACT>(a, s);
       case 16 + 2: return wide_go<DT, 1, 2, ACT>(a, s);
       case 16 + 3: return wide_go<DT, 1, 3, ACT>(a, s);
       case 16 + 4: return wide_go<DT, 1, 4, ACT>(a, s);
@@ -358,7 +438,7 @@ int64_t wide_workspace(int64_t M, int64_t N, int64_t K, int64_t cap) {
 }
 
 int wide_gemm(int32_t dtype, const void* x, int64_t ldx, const void* wp, void* y, int64_t ldy, int64_t M, int64_t N,
-              int64_t K, hipStream_t stream, WideOut out) {
+              int64_t K, hipStream_t stream, WideOut out, int split, void* workspace) {
   const bool act = out == WideOut::kActPlain || out == WideOut::kActInterleaved;
   WideArgs a{};
   a.x = x;
@@ -368,15 +448,19 @@ int wide_gemm(int32_t dtype, const void* x, int64_t ldx, const void* wp, void* y
   a.ldy = ldy;
   a.M = static_cast<int>(M);
   a.N = static_cast<int>(act ? N / 2 : N);
+  a.K = static_cast<int>(K);
   a.Ks = static_cast<int>((K + 31) / 32);
-  a.stages = static_cast<int>((K + 63) / 64);
-  a.k_tail = static_cast<int>(K - 64 * (a.stages - 1));
   a.out_f32 = out == WideOut::kF32;
   a.wbytes = static_cast<uint32_t>(pack_bytes(N, a.Ks));
   a.wgroup = pack_group_bytes(N);
   a.gate_step = out == WideOut::kActInterleaved ? 2 : 1;
   a.up_step = out == WideOut::kActInterleaved ? 1 : a.N / 16;
-  const WideTile t = wide_pick(M, a.N, act);
+  a.split = split;
+  if (split > 1) {
+    a.arrive = static_cast<int*>(workspace) + kPackedArriveBase;
+    a.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes);
+  }
+  const WideTile t = wide_pick(M, a.N, split, act);
   hipError_t err;
   if (dtype == PLM_BF16)
     err = act ? wide_dispatch<DT_BF16, true>(a, t, stream) : wide_dispatch<DT_BF16, false>(a, t, stream);

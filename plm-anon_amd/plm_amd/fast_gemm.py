@@ -20,6 +20,7 @@ transient buffer (``unpacked``, bit for bit).
 
 from __future__ import annotations
 
+import functools
 import threading
 
 import torch
@@ -205,11 +206,16 @@ def default_config(M: int, N: int, K: int) -> Config:
     """The tile for a width the tables do not tune: round widths (M <= 128) take
     ``tiles.heuristic_tile``; wider calls run on the wide kernel, which has its own fixed tiling
     (any valid tile is accepted and not used)."""
+    if M <= 128:
+        return dict(_default_tile(M, N, K))
+    return {"wave_frags": 2, "k_waves": 8, "split_k": 1, "unroll": 2}  # unused: the wide kernel runs
+
+
+@functools.lru_cache(maxsize=4096)
+def _default_tile(M: int, N: int, K: int) -> Config:
     from .tiles import heuristic_tile
 
-    if M <= 128:
-        return heuristic_tile(M, N, K, supported=lambda cfg: tile_supported(M, K, cfg))
-    return {"wave_frags": 2, "k_waves": 8, "split_k": 1, "unroll": 2}  # unused: the wide kernel runs
+    return heuristic_tile(M, N, K, supported=lambda cfg: tile_supported(M, K, cfg))
 
 
 def gate_up_order(w: torch.Tensor) -> torch.Tensor:

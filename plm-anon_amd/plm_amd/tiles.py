@@ -111,16 +111,57 @@ def _first_compiled(M: int, nf: int, layouts, supported) -> dict | None:
     return None
 
 
+# The wide kernel (csrc/wide_gemm.hip), which runs single linears on row-split tiles: its tiles as
+# (64-row weight blocks, 16-row X fragments), and above this packed size at up to 64 rows the row-split
+# kernel proper (``wide_preferred`` in csrc/packed_api.hip).
+WIDE_TILES = ((1, 1), (1, 2), (1, 3), (1, 4), (1, 5), (1, 8), (2, 1), (2, 2), (2, 3), (2, 4), (2, 5), (2, 6), (2, 8),
+              (2, 10), (4, 8))
+WIDE_WEIGHT_BYTES = 128 << 20
+ROW_SPLIT_SPLITS = (1, 2, 3, 4, 6)
+
+
+def runs_wide(M: int, N: int, K: int) -> bool:
+    return M > 64 or math.ceil(N / 256) * 16 * math.ceil(K / 256) * 8 * FRAG < WIDE_WEIGHT_BYTES
+
+
+def row_split_splits(M: int, N: int, K: int) -> int:
+    """K splits of a row-split tile on the wide kernel with the least modelled time (us): a CU's K steps at
+    0.075 us or its loads' 82 KiB per us, whichever is longer, and for the partial sums' round trip 0.8 us,
+    0.3 per split and 0.87 per MB. Measured at M = 56: 2048x2048 7.8 / 7.5 us with 1 / 2 splits,
+    6144x2048 9.6 / 11.1, 2048x8192 23.6 / 16.8 / 14.1 / 16.1 with 1 / 2 / 4 / 6."""
+    steps = math.ceil(K / 32)
+
+    def cost(split: int) -> float:
+        work = min(math.ceil(math.ceil(N / (64 * nf)) * math.ceil(M / (16 * mt)) * split / CU_COUNT)
+                   * max(0.075, (4 * nf + mt) / 82) for nf, mt in WIDE_TILES)
+        join = 0.8 + 0.3 * split + 0.87e-6 * 4 * split * M * N if split > 1 else 0.0
+        return math.ceil(steps / split) * work + join
+
+    return min((s for s in ROW_SPLIT_SPLITS if s == 1 or steps // s >= 16), key=cost)
+
+
 def heuristic_tile(M: int, N: int, K: int, supported=None) -> dict:
-    """A reasonable tile without measurement (what the MI355X measurements of the round shapes
-    favour): 32 rows per wavefront with a two-stage pipeline; rows split across the wavefronts
-    (128-row tiles) when that alone gives every compute unit a tile (the LM head: one round of
-    tiles instead of three and a fraction), else K split across 8 wavefronts (4 where 8 is not
-    compiled), and K splitting until about three quarters of the compute units have an item,
-    keeping at least two K steps per wavefront."""
+    """A reasonable tile without measurement: rows split across the wavefronts (the wide kernel's
+    linears, with ``row_split_splits``'s K splits; the row-split kernel itself for weights past
+    ``WIDE_WEIGHT_BYTES`` at up to 64 rows), else ``k_split_tile``."""
+    for nf in (2, 1, 4):
+        cfg = _first_compiled(M, nf, (1,), supported)
+        if cfg is None:
+            continue
+        if runs_wide(M, N, K):
+            return dict(cfg, split_k=row_split_splits(M, N, K))
+        if math.ceil(N / 16) // (K_WAVES * nf) >= CU_COUNT:
+            return cfg
+    return k_split_tile(M, N, K, supported)
+
+
+def k_split_tile(M: int, N: int, K: int, supported=None) -> dict:
+    """A tile of the K-split layouts without measurement (what the gated-LoRA launch runs where the
+    linear's own tile is a row-split one): 32 rows per wavefront with a two-stage pipeline, K split across 8
+    wavefronts (4 where 8 is not compiled), and K splitting until about three quarters of the compute
+    units have an item, keeping at least two K steps per wavefront."""
     for nf in (2, 4, 1):
-        layouts = (1,) if math.ceil(N / 16) // (K_WAVES * nf) >= CU_COUNT else (8, 4)
-        cfg = _first_compiled(M, nf, layouts, supported)
+        cfg = _first_compiled(M, nf, (8, 4), supported)
         if cfg is None:
             continue
         split = 1

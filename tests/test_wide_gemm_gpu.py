@@ -1,6 +1,7 @@
 """plm_gemm_wide: every output is one MFMA chain over K in ascending order, so it equals the packed
-row-split kernel without K splits (its own parity against the oracle: tests/test_gemm_gpu.py) bit for
-bit, at the edges of its tiles (32 to 160 rows of X by 64 to 256 of W) and of its 64-wide K stages. The
+row-split kernel without K splits, as a one-link chain runs it (its own parity against the oracle:
+tests/test_chain_gpu.py), bit for bit, at the edges of its tiles (16 to 160 rows of X by 64 to 256 of W)
+and of its 64-wide K stages; and with K splits, which single linears on row-split tiles run with. The
 activation epilogue equals torch's silu and multiply on the rounded projection up to one output step
 where the two exponentials' last bits part."""
 
@@ -11,7 +12,8 @@ import torch
 import torch.nn.functional as F
 
 from plm_amd import _lib, fast_gemm
-from plm_amd.fast_gemm import launch_packed, pack_weight, release, released_linear
+from plm_amd.chain import Link, LinearChain
+from plm_amd.fast_gemm import hip_linear, hip_linear_f32, pack_weight, release, released_linear
 from test_gemm_gpu import _inputs_on_gpu
 
 pytestmark = pytest.mark.gpu
@@ -26,9 +28,13 @@ def _wide(x, wp, N, kind, y):
     return y
 
 
-def _chain(x, wp, N):
-    parts = [launch_packed(x[m:m + 64], wp, N, ROW_SPLIT, torch.empty(min(64, x.shape[0] - m), N, device=x.device),
-                           f32_out=True) for m in range(0, x.shape[0], 64)]
+def _chain(x, w, split=1):
+    """fp32 ``x @ w^T`` on the packed row-split kernel, 128 rows of X at a time."""
+    parts = []
+    for m in range(0, x.shape[0], 128):
+        rows = x[m:m + 128]
+        parts.append(torch.empty(rows.shape[0], w.shape[0], device=x.device))
+        LinearChain([Link(rows, w, parts[-1], split_k=split)], dict(ROW_SPLIT, split_k=1)).run()
     return torch.cat(parts)
 
 
@@ -44,7 +50,7 @@ def test_matches_the_row_split_chain_bit_for_bit(device, M, N, K, dtype):
     print(f"wide M={M} N={N} K={K} {dtype}", flush=True)
     x, w = (t.to(dtype) for t in _inputs_on_gpu(M, N, K, 3 * M + N, device))
     wp = pack_weight(w)
-    ref = _chain(x, wp, N)
+    ref = _chain(x, w)
     pad = torch.full((M, N + 5), float("nan"), device=device, dtype=dtype)   # rows that no 16-byte store fits
     assert torch.equal(_wide(x, wp, N, _lib.PLM_OUT_F32, torch.empty(M, N, device=device)), ref)
     assert torch.equal(_wide(x, wp, N, _lib.PLM_OUT_MODEL, torch.empty(M, N, device=device, dtype=dtype)), ref.to(dtype))
@@ -55,7 +61,7 @@ def test_matches_the_row_split_chain_bit_for_bit(device, M, N, K, dtype):
 @pytest.mark.parametrize("M,N,K", [(129, 32, 8), (150, 1024, 1000), (640, 11264, 2048), (200, 2816, 512)])
 def test_silu_mul_of_a_released_gate_up_weight(device, M, N, K):
     x, w = _inputs_on_gpu(M, N, K, N + K, device)
-    y = _chain(x, pack_weight(w), N).to(x.dtype)
+    y = _chain(x, w).to(x.dtype)
     want = F.silu(y[:, : N // 2]) * y[:, N // 2:]
     release(w)
     out = torch.empty(M, N // 2, device=device, dtype=x.dtype)
@@ -64,6 +70,29 @@ def test_silu_mul_of_a_released_gate_up_weight(device, M, N, K):
     # expf of the two sides may round apart: one step of the silu (2^-8 relative) and one of the product.
     assert int((got != want).sum()) <= max(1, got.numel() // 1000)
     torch.testing.assert_close(got.float(), want.float(), rtol=2 * 2.0 ** -7, atol=1e-30)
+
+
+# Rounds on row-split tiles: one row, a tile's edge and past it, the widest; ranges of K steps that
+# start inside a group of packed steps, of odd length, and shorter than the loads in flight.
+@pytest.mark.parametrize("M,N,K", [(1, 64, 96), (17, 1003, 1416), (56, 2048, 8192), (65, 4608, 3072), (128, 777, 1000)])
+@pytest.mark.parametrize("split", [1, 2, 3, 6])
+def test_row_split_tiles_with_k_splits(device, M, N, K, split):
+    print(f"row split M={M} N={N} K={K} split={split}", flush=True)
+    x, w = _inputs_on_gpu(M, N, K, M + N + split, device)
+    cfg = dict(ROW_SPLIT, split_k=split)
+    ref = _chain(x, w, split)
+    for _ in range(2):   # the second launch finds the first one's counters and partials
+        assert torch.equal(hip_linear_f32(x, w, cfg), ref)
+    assert torch.equal(hip_linear(x, w, cfg), ref.bfloat16())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 32, 64), (42, 2816, 512), (110, 11264, 2048)])
+@pytest.mark.parametrize("split", [1, 2])
+def test_silu_mul_on_row_split_tiles(device, M, N, K, split):
+    x, w = _inputs_on_gpu(M, N, K, M + K, device)
+    want = torch.empty(M, N // 2, device=device, dtype=x.dtype)
+    LinearChain([Link(x, w, want, split_k=split, act=True)], dict(ROW_SPLIT, split_k=1)).run()
+    assert torch.equal(fast_gemm.gate_up_silu(x, w, dict(ROW_SPLIT, split_k=split)), want)
 
 
 def test_calls_that_need_more_than_a_product_go_to_f_linear(device):
