@@ -12,15 +12,13 @@
 // The floor rule (plm/decoder.py:78-82), accept = l_own - logsumexp(l) > log(eps), reads the same
 // row state: logsumexp(l) = mx + log(sum_j e_j).
 //
-// Two launches:
-//   1. own_logit_kernel: one workgroup per row r recomputes the single logit l[r, pending[r]] with
-//      the same tile geometry, K partition and reduction order as the main pass, so the value is
-//      bit-identical to the one the main pass forms for that column.
-//   2. verify_main_kernel: G workgroups, each streaming tiles b, b+G, b+2G, ... of W. For every
-//      tile it forms the [TN x R] logits in LDS, then each row's tile max / argmax / sum of
-//      exponentials / sum above l_own, merged into a running per-row state (online rescaling).
-//      The states go to the workspace; the last workgroup to finish (integer counter) merges them
-//      in a fixed tree and writes accept[] and argmax[]. No float atomics; bitwise reproducible.
+// One launch, over packed weights (verify_packed_main_kernel) or row-major ones (verify_rows_kernel):
+// the first workgroups recompute each row's proposal logit l[r, pending[r]] with the main pass's K
+// partition and order, so that the value is bit-identical to the one the main pass forms for that column;
+// the others stream tiles of W, fold the logits into running per-row states (maximum, argmax, sum of
+// exponentials, sum above l_own; online rescaling) and publish them; the last workgroups to finish
+// (integer counters) merge the states in a fixed tree and write accept[] and argmax[]. No float atomics;
+// bitwise reproducible.
 #include <hip/hip_runtime.h>
 
 #include <climits>
@@ -47,22 +45,17 @@ struct VerifyArgs {
   int64_t* argmax;
   int* counter;      // [1], zero between launches
   float* own;        // [R]
-  float* state;      // [G][R][3]: row max, sum of exp, sum of exp above own
-  int* state_idx;    // [G][R]: argmax
-  int* group_counter;  // packed verify: [G / kVerifyGroupSize], zero between launches
-  float* gstate;       // packed verify: [groups][R][3], the merged state of each group
-  int* gstate_idx;     // packed verify: [groups][R]
-  // Packed verify: the row states as 16-byte records {max, sum, sum above own, argmax bits}, one
-  // coherent store each and one coherent load each per merge: rec[G][R] over the state and
-  // state_idx areas, grec[groups][R] over gstate and gstate_idx.
+  int* group_counter;  // [G / kVerifyGroupSize], zero between launches
+  // The row states as 16-byte records {max, sum, sum above own, argmax bits}, one coherent store each
+  // and one coherent load each per merge: rec[G][R], and grec[groups][R] the merged state of each group.
   f32x4* rec;
   f32x4* grec;
   RoundEpilogue round;  // packed verify: k > 0 runs the round's epilogue after the last merge
   uint16_t* logits;     // packed verify: rows [0, logit_rows) of the logits in the model dtype, or null
   int64_t ld_logits;
   int logit_rows;
-  // packed verify: the first own_groups workgroups compute the proposals' own logits (four rows
-  // each) and count themselves into *own_done; the others wait for that count before their first
+  // The first own_groups workgroups compute the proposals' own logits (four rows each over packed
+  // weights, one over row-major ones) and count themselves into *own_done; the others wait for that count before their first
   // fold (bounded; a wait that gives up sets *error).
   int own_groups;
   int* own_done;
@@ -112,238 +105,15 @@ __device__ __forceinline__ RowState merge(RowState a, RowState b) {
 }
 #pragma clang fp contract(on)
 
-__device__ __forceinline__ RowState shfl_xor_state(const RowState& s, int off) {
-  return RowState{__shfl_xor(s.mx, off, 64), __shfl_xor(s.se, off, 64), __shfl_xor(s.ab, off, 64),
-                  __shfl_xor(s.ai, off, 64)};
-}
-
-__device__ __forceinline__ RowState wave_merge(RowState s) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) s = merge(s, shfl_xor_state(s, off));
-  return s;
-}
-
-template <int DT, int MT, int NF, int U, bool PIPE, int KW>
-__global__ __launch_bounds__(64 * KW) void own_logit_kernel(VerifyArgs a) {
-  extern __shared__ float red[];
-  constexpr int TN = 16 * NF;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r = blockIdx.x;
-  const int64_t pid64 = r < a.pending_rows ? a.pending[r] : -1;
-  if (pid64 < 0 || pid64 >= a.V) {  // not a vocabulary id: no logit, and the row accepts nothing
-    if (threadIdx.x == 0) a.own[r] = NAN;
-    return;
-  }
-  const int pid = static_cast<int>(pid64);
-  const int n0 = (pid / TN) * TN;
-  const int tn = min(TN, a.V - n0);
-  const auto xr = make_rsrc(a.x, static_cast<uint32_t>(a.R * a.ldx * 2));
-  const auto wr = make_rsrc(a.w + static_cast<int64_t>(n0) * a.ldw, static_cast<uint32_t>(tn * a.ldw * 2));
-  uint32_t xoff[MT], woff[NF];
-  row_offsets<MT>(a.ldx, r, r + 1, lane, xoff);
-  row_offsets<NF>(a.ldw, pid - n0, pid - n0 + 1, lane, woff);
-  int st0, st1;
-  k_slice(a.K, wave, KW, st0, st1);
-  f32x4 acc[NF][MT];
-#pragma unroll
-  for (int f = 0; f < NF; ++f)
-#pragma unroll
-    for (int t = 0; t < MT; ++t) acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  wave_mma<DT, MT, NF, U, PIPE>(xr, xoff, wr, woff, a.K, st0, st1, lane, acc);
-  wave_spill<MT, NF>(red, wave, lane, acc);
-  __syncthreads();
-  if (threadIdx.x == 0) a.own[r] = round_through(wg_sum<MT, NF>(red, KW, red_offset<MT, NF>(pid - n0, r)), a.round_mode);
-}
-
-template <int DT, int MT, int NF, int U, bool PIPE, int KW>
-__global__ __launch_bounds__(64 * KW) void verify_main_kernel(VerifyArgs a) {
-  extern __shared__ float red[];
-  constexpr int TN = 16 * NF;
-  static_assert(TN <= 64, "one lane per tile column");
-  constexpr int RPW = (16 * MT + KW - 1) / KW;  // rows of X per wavefront in the epilogue
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n_tiles = (a.V + TN - 1) / TN;
-
-  const auto xr = make_rsrc(a.x, static_cast<uint32_t>(a.R * a.ldx * 2));
-  uint32_t xoff[MT];
-  row_offsets<MT>(a.ldx, 0, a.R, lane, xoff);
-  int st0, st1;
-  k_slice(a.K, wave, KW, st0, st1);
-
-  RowState rs[RPW];
-  float own_l[RPW];
-#pragma unroll
-  for (int j = 0; j < RPW; ++j) {
-    rs[j] = empty_state();
-    const int m = wave + KW * j;
-    own_l[j] = m < a.R ? a.own[m] : 0.f;
-  }
-
-  for (int tile = blockIdx.x; tile < n_tiles; tile += a.G) {
-    const int n0 = tile * TN;
-    const int tn = min(TN, a.V - n0);
-    const auto wr = make_rsrc(a.w + static_cast<int64_t>(n0) * a.ldw, static_cast<uint32_t>(tn * a.ldw * 2));
-    uint32_t woff[NF];
-    row_offsets<NF>(a.ldw, 0, tn, lane, woff);
-    f32x4 acc[NF][MT];
-#pragma unroll
-    for (int f = 0; f < NF; ++f)
-#pragma unroll
-      for (int t = 0; t < MT; ++t) acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    wave_mma<DT, MT, NF, U, PIPE>(xr, xoff, wr, woff, a.K, st0, st1, lane, acc);
-    __syncthreads();  // the previous tile's epilogue has finished reading LDS
-    wave_spill<MT, NF>(red, wave, lane, acc);
-    __syncthreads();
-    const bool valid = lane < tn;
-    const int col = valid ? lane : 0;  // lanes past the tile read column 0 and discard it
-#pragma unroll
-    for (int j = 0; j < RPW; ++j) {
-      const int m = wave + KW * j;
-      if (m < a.R) {
-        const float lv = round_through(wg_sum<MT, NF>(red, KW, red_offset<MT, NF>(col, m)), a.round_mode);
-        const float l = valid ? lv : -INFINITY;
-        // Tile maximum with lowest-index tie-break, then the two exponential sums against it.
-        RowState t{l, 0.f, 0.f, valid ? n0 + lane : INT_MAX};
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) {
-          const float omx = __shfl_xor(t.mx, off, 64);
-          const int oai = __shfl_xor(t.ai, off, 64);
-          if (omx > t.mx || (omx == t.mx && oai < t.ai)) {
-            t.mx = omx;
-            t.ai = oai;
-          }
-        }
-        float e = valid ? exp_below_max(l - t.mx) : 0.f;
-        float ab = (valid && l > own_l[j]) ? e : 0.f;
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) {
-          e += __shfl_xor(e, off, 64);
-          ab += __shfl_xor(ab, off, 64);
-        }
-        t.se = e;
-        t.ab = ab;
-        rs[j] = merge(rs[j], t);
-      }
-    }
-  }
-
-  // Publish this workgroup's row states.
-  if (lane == 0) {
-#pragma unroll
-    for (int j = 0; j < RPW; ++j) {
-      const int m = wave + KW * j;
-      if (m < a.R) {
-        const int64_t slot = static_cast<int64_t>(blockIdx.x) * a.R + m;
-        publish(a.state + slot * 3 + 0, rs[j].mx);
-        publish(a.state + slot * 3 + 1, rs[j].se);
-        publish(a.state + slot * 3 + 2, rs[j].ab);
-        publish(a.state_idx + slot, rs[j].ai);
-      }
-    }
-  }
-  if (!arrive_last(a.counter, a.G)) return;
-
-  // Last workgroup: merge the G states of every row (lane-strided, then a butterfly).
-  for (int j = 0; j < RPW; ++j) {
-    const int m = wave + KW * j;
-    if (m >= a.R) continue;
-    RowState s = empty_state();
-    for (int g = lane; g < a.G; g += 64) {
-      const int64_t slot = static_cast<int64_t>(g) * a.R + m;
-      s = merge(s, RowState{collect(a.state + slot * 3 + 0), collect(a.state + slot * 3 + 1),
-                            collect(a.state + slot * 3 + 2), collect(a.state_idx + slot)});
-    }
-    s = wave_merge(s);
-    if (lane == 0) {
-      a.accept[m] = accept_proposal(a, a.own[m], s) ? 1 : 0;
-      a.argmax[m] = s.ai;
-    }
-  }
-}
-
-template <int MT, int NF, int U, bool PIPE, int KW>
-constexpr bool verify_compiled() {
-  if (KW != 4) return false;  // the K partition of the streaming GEMM (plm_gemm_f32out gives the same logits)
-  if (NF != 2 && NF != 4) return false;
-  if (MT < 1 || MT > 4) return false;
-  const bool u_ok = PIPE ? (U == 2 || U == 4) : (U == 4 || U == 8);
-  if (!u_ok) return false;
-  const int operand_vgprs = (PIPE ? 2 : 1) * U * (NF + MT) * 4;
-  const int budget = KW == 8 ? 256 : 512;
-  return operand_vgprs + NF * MT * 4 + 80 <= budget;
+// Whether the row-major verify takes this tile at mt X fragments, `pipe`: a K quarter is longer than the
+// tile's unroll.
+inline bool verify_tile_known(int mt, const plm_tile& t, bool pipe) {
+  if (t.wave_frags != 2 && t.wave_frags != 4) return false;
+  if (pipe ? t.unroll != 2 && t.unroll != 4 : t.unroll != 4 && t.unroll != 8) return false;
+  return (pipe ? 2 : 1) * t.unroll * (t.wave_frags + mt) * 4 + t.wave_frags * mt * 4 + 80 <= 512;
 }
 
 constexpr int kMaxVerifyGroups = 1024;
-
-template <int DT, int MT, int NF, int U, bool PIPE, int KW>
-hipError_t launch_verify(VerifyArgs a, int cu_count, hipStream_t stream, bool dry) {
-  if constexpr (!verify_compiled<MT, NF, U, PIPE, KW>()) {
-    return hipErrorInvalidConfiguration;
-  } else {
-    if (dry) return hipSuccess;
-    auto own_kern = own_logit_kernel<DT, MT, NF, U, PIPE, KW>;
-    auto main_kern = verify_main_kernel<DT, MT, NF, U, PIPE, KW>;
-    constexpr size_t lds = static_cast<size_t>(KW) * NF * MT * 256 * sizeof(float);
-    if constexpr (lds > 65536) {
-      static const hipError_t attr1 =
-          hipFuncSetAttribute(reinterpret_cast<const void*>(own_kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-      static const hipError_t attr2 =
-          hipFuncSetAttribute(reinterpret_cast<const void*>(main_kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-      if (attr1 != hipSuccess) return attr1;
-      if (attr2 != hipSuccess) return attr2;
-    }
-    static int per_cu = 0;
-    if (per_cu == 0) {
-      int blocks = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(main_kern), 64 * KW, lds) !=
-              hipSuccess ||
-          blocks < 1)
-        blocks = 1;
-      per_cu = blocks;
-    }
-    const int n_tiles = (a.V + 16 * NF - 1) / (16 * NF);
-    a.G = min(n_tiles, min(kMaxVerifyGroups, cu_count * per_cu));
-    hipLaunchKernelGGL(own_kern, dim3(a.R), dim3(64 * KW), lds, stream, a);
-    hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(main_kern, dim3(a.G), dim3(64 * KW), lds, stream, a);
-    return hipGetLastError();
-  }
-}
-
-template <int DT, int MT, int NF>
-hipError_t verify_pick_u(const VerifyArgs& a, const plm_tile& t, bool pipe, int cu, hipStream_t s, bool dry) {
-#define PLM_VERIFY_KW(U_, P_)                                                        \
-  if (t.unroll == U_ && pipe == P_) {                                                \
-    if (t.k_waves == 4) return launch_verify<DT, MT, NF, U_, P_, 4>(a, cu, s, dry);  \
-  }
-  PLM_VERIFY_KW(2, true)
-  PLM_VERIFY_KW(4, true)
-  PLM_VERIFY_KW(4, false)
-  PLM_VERIFY_KW(8, false)
-#undef PLM_VERIFY_KW
-  return hipErrorInvalidConfiguration;
-}
-
-template <int DT>
-hipError_t verify_dispatch(const VerifyArgs& a, const plm_tile& t, int cu, hipStream_t s, bool dry) {
-  const int64_t steps = (a.K + 31) / 32;
-  const bool pipe = (steps + t.k_waves - 1) / t.k_waves > t.unroll;
-  const int mt = (a.R + 15) / 16;
-#define PLM_VERIFY_NF(MT_)                                                  \
-  if (mt == MT_) {                                                          \
-    if (t.wave_frags == 2) return verify_pick_u<DT, MT_, 2>(a, t, pipe, cu, s, dry); \
-    if (t.wave_frags == 4) return verify_pick_u<DT, MT_, 4>(a, t, pipe, cu, s, dry); \
-  }
-  PLM_VERIFY_NF(1)
-  PLM_VERIFY_NF(2)
-  PLM_VERIFY_NF(3)
-  PLM_VERIFY_NF(4)
-#undef PLM_VERIFY_NF
-  return hipErrorInvalidConfiguration;
-}
 
 // ---------------------------------------------------------------------------------------------
 // The same step over packed weights (plm_pack_weight), on the packed GEMM's row-split pipeline
@@ -594,6 +364,72 @@ __device__ __forceinline__ void store_logits(const f32x4 (&acc)[NF][MT], int n0,
   }
 }
 
+// LDS of the merges: the wavefronts' row states, and the members of the group being merged.
+struct VerifyMergeLds {
+  float mx[kPackedWaves][64], se[kPackedWaves][64], ab[kPackedWaves][64];
+  int ai[kPackedWaves][64];
+};
+
+// The end of a main workgroup `b`: its wavefronts' states merged and published, then the two-level merge
+// over the workgroups; the last one decides every row (and runs the round's epilogue). rs[t]: this
+// wavefront's state of row 16t + lane%16, the same in the row's four lanes. `grid`: kVerifyGroupSize * 64
+// records.
+template <int MT>
+__device__ __forceinline__ void verify_merge(const VerifyArgs& a, int b, int wave, int lane, const RowState (&rs)[MT],
+                                             VerifyMergeLds& st, f32x4* grid) {
+  // The workgroup's state of each row: its four wavefronts merged in wavefront order.
+  if (lane < 16) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      const int m = 16 * t + lane;
+      st.mx[wave][m] = rs[t].mx;
+      st.se[wave][m] = rs[t].se;
+      st.ab[wave][m] = rs[t].ab;
+      st.ai[wave][m] = rs[t].ai;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < a.R) {
+    const int m = threadIdx.x;
+    RowState s0 = RowState{st.mx[0][m], st.se[0][m], st.ab[0][m], st.ai[0][m]};
+#pragma unroll
+    for (int w = 1; w < kPackedWaves; ++w) s0 = merge(s0, RowState{st.mx[w][m], st.se[w][m], st.ab[w][m], st.ai[w][m]});
+    publish_record(a.rec, b * a.R + m, a.G * a.R, s0);
+  }
+  // Two-level merge: the last workgroup of each group of kVerifyGroupSize merges the group's
+  // states, the last group to finish merges the group states. Each level is one batch of
+  // device-coherent loads into LDS and a fixed-order merge with one lane per row.
+  const int group = b / kVerifyGroupSize;
+  const int gsize = min(kVerifyGroupSize, a.G - group * kVerifyGroupSize);
+  if (!arrive_last(a.group_counter + group, gsize)) return;
+  gather_records(a.rec, group * kVerifyGroupSize, gsize, a.R, grid);
+  {
+    const RowState t = merge_rows(grid, gsize, wave, lane, st.mx, st.se, st.ab, st.ai);
+    if (wave == 0 && lane < a.R) publish_record(a.grec, group * a.R + lane, (group + 1) * a.R, t);
+  }
+  const int groups = (a.G + kVerifyGroupSize - 1) / kVerifyGroupSize;
+  if (!arrive_last(a.counter, groups)) return;
+  // The proposals' own logits (complete before any workgroup's first fold) load with the records.
+  const float own_v = (wave == 0 && lane < a.R) ? collect(a.own + lane) : 0.f;
+  gather_records(a.grec, 0, groups, a.R, grid);
+  const RowState t = merge_rows(grid, groups, wave, lane, st.mx, st.se, st.ab, st.ai);
+  if (wave == 0) {
+    if (lane == 0 && a.own_groups > 0) publish(a.own_done, 0);  // every workgroup has counted in and read it
+    const bool acc = lane < a.R && accept_proposal(a, own_v, t);
+    if (lane < a.R) {
+      if (a.accept != nullptr) a.accept[lane] = acc ? 1 : 0;
+      if (a.argmax != nullptr) a.argmax[lane] = t.ai;
+    }
+    if (a.round.k > 0) {
+      // Rows 0..k-1 verify, rows k.. are the proposal blocks: lane i holds row i's decision and
+      // argmax, so hypothesis j is lane k + j's argmax.
+      const int ai = t.ai;
+      const int k = a.round.k;
+      round_epilogue_wave(a.round, lane, acc, [&](int j) { return static_cast<int64_t>(__shfl(ai, k + j)); });
+    }
+  }
+}
+
 template <int MT, int NF, int D>
 constexpr bool verify_packed_compiled() {
   return MT >= 1 && MT <= 4 && (NF == 2 || NF == 4) && (D == 2 || D == 4 || D == 8) && packed_compiled<MT, NF, D, 1>();
@@ -609,8 +445,7 @@ __global__ __launch_bounds__(64 * kPackedWaves, (packed_waves_per_simd<MT, NF, D
   const int b = static_cast<int>(blockIdx.x) - a.own_groups;  // this workgroup among the main ones
   constexpr int KW = 1;
   constexpr int XN = x_per_wave<MT, KW>();
-  __shared__ float st_mx[kPackedWaves][64], st_se[kPackedWaves][64], st_ab[kPackedWaves][64];
-  __shared__ int st_ai[kPackedWaves][64];
+  __shared__ VerifyMergeLds st;
   __shared__ f32x4 grid[kVerifyGroupSize * 64];  // final merges: [member][row]
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -717,58 +552,7 @@ __global__ __launch_bounds__(64 * kPackedWaves, (packed_waves_per_simd<MT, NF, D
     }
   }
   __builtin_amdgcn_s_waitcnt(0);
-
-  // The workgroup's state of each row: its four wavefronts merged in wavefront order.
-  if (lane < 16) {
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      const int m = 16 * t + lane;
-      st_mx[wave][m] = rs[t].mx;
-      st_se[wave][m] = rs[t].se;
-      st_ab[wave][m] = rs[t].ab;
-      st_ai[wave][m] = rs[t].ai;
-    }
-  }
-  __syncthreads();
-  if (threadIdx.x < a.R) {
-    const int m = threadIdx.x;
-    RowState s0 = RowState{st_mx[0][m], st_se[0][m], st_ab[0][m], st_ai[0][m]};
-#pragma unroll
-    for (int w = 1; w < kPackedWaves; ++w) s0 = merge(s0, RowState{st_mx[w][m], st_se[w][m], st_ab[w][m], st_ai[w][m]});
-    publish_record(a.rec, b * a.R + m, a.G * a.R, s0);
-  }
-  // Two-level merge: the last workgroup of each group of kVerifyGroupSize merges the group's
-  // states, the last group to finish merges the group states. Each level is one batch of
-  // device-coherent loads into LDS and a fixed-order merge with one lane per row.
-  const int group = b / kVerifyGroupSize;
-  const int gsize = min(kVerifyGroupSize, a.G - group * kVerifyGroupSize);
-  if (!arrive_last(a.group_counter + group, gsize)) return;
-  gather_records(a.rec, group * kVerifyGroupSize, gsize, a.R, grid);
-  {
-    const RowState t = merge_rows(grid, gsize, wave, lane, st_mx, st_se, st_ab, st_ai);
-    if (wave == 0 && lane < a.R) publish_record(a.grec, group * a.R + lane, (group + 1) * a.R, t);
-  }
-  const int groups = (a.G + kVerifyGroupSize - 1) / kVerifyGroupSize;
-  if (!arrive_last(a.counter, groups)) return;
-  // The proposals' own logits (complete before any workgroup's first fold) load with the records.
-  const float own_v = (wave == 0 && lane < a.R) ? collect(a.own + lane) : 0.f;
-  gather_records(a.grec, 0, groups, a.R, grid);
-  const RowState t = merge_rows(grid, groups, wave, lane, st_mx, st_se, st_ab, st_ai);
-  if (wave == 0) {
-    if (lane == 0 && a.own_groups > 0) publish(a.own_done, 0);  // every workgroup has counted in and read it
-    const bool acc = lane < a.R && accept_proposal(a, own_v, t);
-    if (lane < a.R) {
-      if (a.accept != nullptr) a.accept[lane] = acc ? 1 : 0;
-      if (a.argmax != nullptr) a.argmax[lane] = t.ai;
-    }
-    if (a.round.k > 0) {
-      // Rows 0..k-1 verify, rows k.. are the proposal blocks: lane i holds row i's decision and
-      // argmax, so hypothesis j is lane k + j's argmax.
-      const int ai = t.ai;
-      const int k = a.round.k;
-      round_epilogue_wave(a.round, lane, acc, [&](int j) { return static_cast<int64_t>(__shfl(ai, k + j)); });
-    }
-  }
+  verify_merge<MT>(a, b, wave, lane, rs, st, grid);
 }
 
 template <int DT, int MT, int NF, int D>
@@ -819,14 +603,272 @@ hipError_t verify_packed_dispatch(const VerifyArgs& a, const plm_tile& t, int cu
   return hipErrorInvalidConfiguration;
 }
 
+// ---------------------------------------------------------------------------------------------
+// The step over row-major weights. Every logit is the sum, in order, of four MFMA chains over the four
+// quarters of the K steps (k_slice): the packed GEMM's four-wavefront K split, which returns the same
+// logits bit for bit (plm_gemm_packed_f32out, k_waves = 4).
+//
+// What bounds it: HBM, once W is loaded in whole cache lines. An MFMA operand loaded straight from a
+// row-major W takes 16 bytes of 16 rows per 16 lanes, 64 requests per instruction, and a wavefront per
+// K quarter loads all of X itself: that kernel ran at 0.79 TB/s (259 us at R = 56, V = 50257, K = 2048).
+// Here a wavefront owns 32 (or 16) vocabulary rows over all of K and adds its accumulator into the sum at the
+// quarters' ends, so that the workgroup's four wavefronts share one copy of X; W and X are loaded as
+// rows of 128 B (two K steps), eight lanes each, and turned into operands through LDS with 16-byte chunk
+// c of row r at slot c ^ (r % 8) (conflict-free). A stage is two K steps with one barrier in its middle,
+// loads run D stages ahead, as in csrc/wide_gemm.hip.
+//
+// Measured (R = 56, K = 2048, V = 50257; the same call 259.7 us before): 59.8 us, 3.45 TB/s. One weight
+// fragment per wavefront (64-row tiles) takes 68.7 us there but 25.2 against 30.3 us at V = 8000, whose
+// 63 tiles of 128 rows leave most CUs idle; four take 65.0.
+
+// Stages of loads in flight (two where more would not fit 256 registers: 69.5 us at R = 56).
+template <int MT, int NF>
+constexpr int rows_depth() {
+  return MT <= 2 || NF == 1 ? 4 : 2;
+}
+
+// One workgroup per proposal: wavefront q's chain over quarter q of the one logit, summed in order.
+template <int DT>
+__device__ __forceinline__ void own_logit_rows(const VerifyArgs& a) {
+  __shared__ float part[kPackedWaves];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = blockIdx.x;
+  const int64_t pid64 = r < a.pending_rows ? a.pending[r] : -1;
+  const bool valid = pid64 >= 0 && pid64 < a.V;
+  if (valid) {
+    const int pid = __builtin_amdgcn_readfirstlane(static_cast<int>(pid64));
+    const int n0 = pid & ~15, m0 = r & ~15;
+    const auto xr = make_rsrc(a.x, static_cast<uint32_t>(a.R * a.ldx * 2));
+    const auto wr = make_rsrc(a.w + static_cast<int64_t>(n0) * a.ldw,
+                              static_cast<uint32_t>(min(16, a.V - n0) * a.ldw * 2));
+    // The one row of each operand, in its place in the main pass's fragments.
+    const uint32_t xoff[1] = {(lane & 15) == r - m0 ? static_cast<uint32_t>((r * a.ldx + 8 * (lane >> 4)) * 2) : kOutOfRange};
+    const uint32_t woff[1] = {(lane & 15) == pid - n0 ? static_cast<uint32_t>(((pid - n0) * a.ldw + 8 * (lane >> 4)) * 2)
+                                                      : kOutOfRange};
+    int st0, st1;
+    k_slice(a.K, wave, kPackedWaves, st0, st1);
+    f32x4 acc[1][1] = {{f32x4{0.f, 0.f, 0.f, 0.f}}};
+    wave_mma<DT, 1, 1, 8, true>(xr, xoff, wr, woff, a.K, st0, st1, lane, acc);
+    const int v = pid - n0;
+    if (lane == (r & 15) + 16 * (v >> 2)) part[wave] = acc[0][0][v & 3];
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float s = NAN;
+    if (valid) {
+      s = part[0];
+      for (int w = 1; w < kPackedWaves; ++w) s += part[w];
+      s = round_through(s, a.round_mode);
+    }
+    publish(a.own + r, s);
+    __builtin_amdgcn_s_waitcnt(0);
+    __hip_atomic_fetch_add(a.own_done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+template <int DT, int MT, int NF>
+__global__ __launch_bounds__(64 * kPackedWaves, 2) void verify_rows_kernel(VerifyArgs a) {
+  if (static_cast<int>(blockIdx.x) < a.own_groups) {
+    own_logit_rows<DT>(a);
+    return;
+  }
+  constexpr int D = rows_depth<MT, NF>(), WN = 2 * NF, XN = (MT + 1) / 2;
+  constexpr int kXWords = 2 * MT * 64, kWWords = kPackedWaves * WN * 64;  // u32x4 of a stage
+  constexpr int kLds = 2 * (kXWords + kWWords), kGrid = kVerifyGroupSize * 64;
+  __shared__ __attribute__((aligned(16))) u32x4 lds[kLds > kGrid ? kLds : kGrid];
+  __shared__ VerifyMergeLds st;
+  const int b = static_cast<int>(blockIdx.x) - a.own_groups;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int steps = (a.K + 31) >> 5, tiles = (a.V + 64 * NF - 1) / (64 * NF);
+  // Quarter q of the K steps ends with stage end[q] (exclusive).
+  int end[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int lo = static_cast<int>(static_cast<int64_t>(q) * steps >> 2), hi = static_cast<int>(static_cast<int64_t>(q + 1) * steps >> 2);
+    end[q] = (q > 0 ? end[q - 1] : 0) + ((hi - lo + 1) >> 1);
+  }
+  const int stages = end[3];
+  const auto xr = make_rsrc(a.x, static_cast<uint32_t>(a.R * a.ldx * 2));
+  const int chunk = (lane & 7) ^ (lane >> 3);  // of the 128-byte row segments this lane loads
+  uint32_t xo[XN], wo[WN];
+#pragma unroll
+  for (int j = 0; j < XN; ++j) {
+    const int row = 8 * (wave + 4 * j) + (lane >> 3);
+    xo[j] = row < a.R ? static_cast<uint32_t>(row * a.ldx * 2) + 16u * chunk : kOutOfRange;
+  }
+#pragma unroll
+  for (int j = 0; j < WN; ++j) wo[j] = static_cast<uint32_t>((8 * j + (lane >> 3)) * a.ldw * 2) + 16u * chunk;
+  const int rd0 = (lane & 15) * 8 + ((lane >> 4) ^ (lane & 7)), rd1 = rd0 ^ 4;
+  u32x4* const wlds = lds + 2 * kXWords + wave * WN * 64;  // this wavefront's weights, kWWords apart
+
+  RowState rs[MT];
+  float own_l[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    rs[t] = empty_state();
+    own_l[t] = 0.f;
+  }
+  bool own_ready = false;
+  for (int tile = b; tile < tiles; tile += a.G) {
+    const int n_wave = tile * 64 * NF + wave * 16 * NF;
+    const int rows = max(0, min(16 * NF, a.V - n_wave));
+    const auto wr = make_rsrc(a.w + (rows > 0 ? static_cast<int64_t>(n_wave) * a.ldw : 0),
+                              static_cast<uint32_t>(rows * a.ldw * 2));
+    u32x4 X[D][XN], W[D][WN];
+    // The next stage to load: K steps [kb, kb + 2) up to the end of quarter q.
+    int kb = 0, q = 0;
+    auto cut = [&](int i) __attribute__((always_inline)) { return static_cast<int>(static_cast<int64_t>(i) * steps >> 2); };
+    while (q < 3 && cut(q + 1) == 0) ++q;
+    auto load = [&](u32x4 (&x)[XN], u32x4 (&w)[WN]) __attribute__((always_inline)) {
+      const int hi = cut(q + 1);
+      // Bytes of the row from the stage's start that belong to it: 128, or fewer at a quarter's or K's
+      // end (none past the last stage).
+      const int left = min(2 * a.K, 64 * hi) - 64 * kb;
+      const int so = __builtin_amdgcn_readfirstlane(64 * kb);
+      const bool in = 16 * chunk < left;
+      kb = min(kb + 2, hi);
+      while (q < 3 && kb == cut(q + 1)) ++q;
+#pragma unroll
+      for (int j = 0; j < XN; ++j) x[j] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, static_cast<int>(in ? xo[j] : kOutOfRange), so, 0));
+#pragma unroll
+      for (int j = 0; j < WN; ++j) w[j] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, static_cast<int>(in ? wo[j] : kOutOfRange), so, 0));
+    };
+    auto put = [&](int slot, const u32x4 (&x)[XN], const u32x4 (&w)[WN]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < XN; ++j)
+        if (4 * j + 3 < 2 * MT || wave + 4 * j < 2 * MT) lds[slot * kXWords + (wave + 4 * j) * 64 + lane] = x[j];
+#pragma unroll
+      for (int j = 0; j < WN; ++j) wlds[slot * kWWords + j * 64 + lane] = w[j];
+    };
+    f32x4 acc[NF][MT], sum[NF][MT];
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) acc[f][t] = sum[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    u32x4 A0[NF], A1[NF], B0[MT], B1[MT];
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      load(X[j], W[j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    lds_sync();  // the tile before: no wavefront reads its X any more
+    put(0, X[0], W[0]);
+    load(X[0], W[0]);
+    lds_sync();
+#pragma unroll
+    for (int t = 0; t < MT; ++t) B0[t] = lds[t * 128 + rd0];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) A0[f] = wlds[f * 128 + rd0];
+    auto stage = [&](int j, int i) __attribute__((always_inline)) {
+      const int slot = j & 1, jn = (j + 1) % D;
+#pragma unroll
+      for (int t = 0; t < MT; ++t) B1[t] = lds[slot * kXWords + t * 128 + rd1];
+#pragma unroll
+      for (int f = 0; f < NF; ++f) A1[f] = wlds[slot * kWWords + f * 128 + rd1];
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[f][t] = mfma_16x16x32<DT>(A0[f], B0[t], acc[f][t]);
+      put(slot ^ 1, X[jn], W[jn]);
+      load(X[jn], W[jn]);
+      lds_sync();
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) B0[t] = lds[(slot ^ 1) * kXWords + t * 128 + rd0];
+#pragma unroll
+      for (int f = 0; f < NF; ++f) A0[f] = wlds[(slot ^ 1) * kWWords + f * 128 + rd0];
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[f][t] = mfma_16x16x32<DT>(A1[f], B1[t], acc[f][t]);
+      if (i + 1 == end[0] || i + 1 == end[1] || i + 1 == end[2] || i + 1 == end[3]) {
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+          for (int t = 0; t < MT; ++t) {
+            sum[f][t] += acc[f][t];
+            acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int j = 0; j < D; ++j) stage(j, j);
+    for (int i = D; i < stages; i += D) {
+#pragma unroll
+      for (int j = 0; j < D; ++j) stage(j, i + j);
+    }
+    if (!own_ready) {
+      wait_own_logits(a);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const int m = 16 * t + (lane & 15);
+        own_l[t] = m < a.R ? collect(a.own + m) : 0.f;
+      }
+      own_ready = true;
+    }
+    const int n0 = n_wave + 4 * (lane >> 4);
+    const bool full = n_wave + 16 * NF <= a.V;
+    if (a.round_mode == PLM_ROUND_BF16) {
+      if (full) fold_columns<MT, NF, PLM_ROUND_BF16, false>(sum, n0, a.V, own_l, rs);
+      else fold_columns<MT, NF, PLM_ROUND_BF16, true>(sum, n0, a.V, own_l, rs);
+    } else if (a.round_mode == PLM_ROUND_F16) {
+      if (full) fold_columns<MT, NF, PLM_ROUND_F16, false>(sum, n0, a.V, own_l, rs);
+      else fold_columns<MT, NF, PLM_ROUND_F16, true>(sum, n0, a.V, own_l, rs);
+    } else {
+      if (full) fold_columns<MT, NF, PLM_ROUND_F32, false>(sum, n0, a.V, own_l, rs);
+      else fold_columns<MT, NF, PLM_ROUND_F32, true>(sum, n0, a.V, own_l, rs);
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0);
+  lds_sync();  // the stages' LDS becomes the merge's
+  verify_merge<MT>(a, b, wave, lane, rs, st, reinterpret_cast<f32x4*>(lds));
+}
+
+template <int DT, int MT, int NF>
+hipError_t launch_verify_rows(VerifyArgs a, int cu_count, hipStream_t stream) {
+  auto kern = verify_rows_kernel<DT, MT, NF>;
+  static int per_cu = 0;
+  if (per_cu == 0) {
+    per_cu = resident_per_cu(reinterpret_cast<const void*>(kern), 64 * kPackedWaves, 0);
+    if (per_cu < 1) return hipErrorInvalidConfiguration;
+  }
+  const int tiles = (a.V + 64 * NF - 1) / (64 * NF);
+  a.own_groups = a.R;
+  a.G = min(tiles, min(kMaxVerifyGroups, cu_count * per_cu));
+  hipLaunchKernelGGL(kern, dim3(a.own_groups + a.G), dim3(64 * kPackedWaves), 0, stream, a);
+  return hipGetLastError();
+}
+
+// 64-row tiles while they do not outnumber the CUs, else 128-row ones.
+template <int DT, int MT>
+hipError_t verify_rows_pick(const VerifyArgs& a, int cu, hipStream_t s) {
+  return a.V <= 64 * cu ? launch_verify_rows<DT, MT, 1>(a, cu, s) : launch_verify_rows<DT, MT, 2>(a, cu, s);
+}
+
+// A tile is checked as it always was; the kernel has its own.
+template <int DT>
+hipError_t verify_dispatch(const VerifyArgs& a, const plm_tile& t, int cu, hipStream_t s, bool dry) {
+  const int64_t steps = (a.K + 31) / 32;
+  if (t.k_waves != 4 || !verify_tile_known((a.R + 15) / 16, t, (steps + 3) / 4 > t.unroll)) return hipErrorInvalidConfiguration;
+  if (dry) return hipSuccess;
+  switch ((a.R + 15) / 16) {
+    case 1: return verify_rows_pick<DT, 1>(a, cu, s);
+    case 2: return verify_rows_pick<DT, 2>(a, cu, s);
+    case 3: return verify_rows_pick<DT, 3>(a, cu, s);
+    default: return verify_rows_pick<DT, 4>(a, cu, s);
+  }
+}
+
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
 // Workspace layout: counter area (ints kVerifyCounter, kVerifyOwnDone, kPkErrorSlot and
-// [kVerifyGroupBase, +groups) used) |
-// own[R] | state[kMaxVerifyGroups][R][3] | state_idx[kMaxVerifyGroups][R] | gstate[groups][R][3] |
-// gstate_idx[groups][R], groups = kMaxVerifyGroups / kVerifyGroupSize. The packed verify keeps its
-// 16-byte records over the same bytes: rec[kMaxVerifyGroups][R] from state, grec[groups][R] from
-// gstate (each pair of areas holds 12 + 4 bytes per entry).
+// [kVerifyGroupBase, +groups) used) | own[R] | rec[kMaxVerifyGroups][R] | grec[groups][R],
+// groups = kMaxVerifyGroups / kVerifyGroupSize; a record takes the 12 + 4 bytes of its two areas.
 constexpr int kMaxVerifyGroupSets = kMaxVerifyGroups / kVerifyGroupSize;
 static_assert(kVerifyGroupBase + kMaxVerifyGroupSets <= 64, "group counters fit before the streaming counters");
 void verify_layout(int64_t R, size_t& own_off, size_t& state_off, size_t& idx_off, size_t& gstate_off,
@@ -901,11 +943,11 @@ int plm_lm_head_verify(int32_t dtype, const void* x, int64_t ldx, const void* w,
   char* ws = static_cast<char*>(workspace);
   a.counter = reinterpret_cast<int*>(ws) + plm::kVerifyCounter;
   a.own = reinterpret_cast<float*>(ws + own_off);
-  a.state = reinterpret_cast<float*>(ws + state_off);
-  a.state_idx = reinterpret_cast<int*>(ws + idx_off);
   a.group_counter = reinterpret_cast<int*>(ws) + plm::kVerifyGroupBase;
-  a.gstate = reinterpret_cast<float*>(ws + gstate_off);
-  a.gstate_idx = reinterpret_cast<int*>(ws + gidx_off);
+  a.rec = reinterpret_cast<plm::f32x4*>(ws + state_off);
+  a.grec = reinterpret_cast<plm::f32x4*>(ws + gstate_off);
+  a.own_done = reinterpret_cast<int*>(ws) + plm::kVerifyOwnDone;
+  a.error = reinterpret_cast<int*>(ws) + plm::kPkErrorSlot;
 
   const int cu = plm::device_cu_count();
   if (cu <= 0) return PLM_ERR_LAUNCH;
@@ -972,11 +1014,7 @@ int packed_verify_entry(int32_t dtype, const void* x, int64_t ldx, const void* p
   char* ws = static_cast<char*>(workspace);
   a.counter = reinterpret_cast<int*>(ws) + plm::kVerifyCounter;
   a.own = reinterpret_cast<float*>(ws + own_off);
-  a.state = reinterpret_cast<float*>(ws + state_off);
-  a.state_idx = reinterpret_cast<int*>(ws + idx_off);
   a.group_counter = reinterpret_cast<int*>(ws) + plm::kVerifyGroupBase;
-  a.gstate = reinterpret_cast<float*>(ws + gstate_off);
-  a.gstate_idx = reinterpret_cast<int*>(ws + gidx_off);
   a.rec = reinterpret_cast<plm::f32x4*>(ws + state_off);
   a.grec = reinterpret_cast<plm::f32x4*>(ws + gstate_off);
   a.own_done = reinterpret_cast<int*>(ws) + plm::kVerifyOwnDone;

@@ -142,7 +142,8 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
     const uint32_t last = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(~((left | -left) >> 31))) & kOutOfRange;
 #pragma unroll
     for (int j = 0; j < XN; ++j)
-      x[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, xo[j] | (xl[j] & last), so, 0));
+      x[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                     xr, (xl[j] & last) != 0 ? kOutOfRange : xo[j], so, 0));
   };
   auto put_x = [&](int slot, const u32x4 (&x)[XN]) __attribute__((always_inline)) {
 #pragma unroll

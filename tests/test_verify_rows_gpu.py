@@ -1,0 +1,28 @@
+"""The row-major verify at the edges of its K quarters and vocabulary tiles: fewer K steps than quarters,
+cuts inside a two-step stage, K off the 32-wide step, one vocabulary row, a tile's edge and past it, more
+tiles than workgroups fit at once. Decisions and the proposals' own logits bit for bit on the four-quarter
+logits of the packed GEMM (test_verify_gpu.run_case)."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from test_verify_gpu import run_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("R,V,K", [(1, 1, 8), (5, 127, 40), (16, 128, 96), (17, 129, 232), (33, 1000, 1064),
+                                   (48, 4097, 1416), (64, 3000, 2056), (56, 140000, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_quarters_and_tiles(device, R, V, K, dtype):
+    print(f"row-major verify R={R} V={V} K={K} {dtype}", flush=True)
+    g = torch.Generator(device=device).manual_seed(R + V + K)
+    x = torch.randn(R, K, generator=g, device=device).to(dtype)
+    w = (torch.randn(V, K + 8, generator=g, device=device) / K ** 0.5).to(dtype)[:, :K]   # rows K + 8 apart
+    pending = torch.randint(-1, V + 1, (R,), generator=g, device=device, dtype=torch.int64)
+    mode = "bf16" if dtype == torch.bfloat16 else "fp16"
+    for m in ("fp32", mode):
+        for _ in range(2):   # the second launch finds the first one's counters
+            run_case(x, w, pending, 0.7, m, device, check_cpu=False, packed=False)
