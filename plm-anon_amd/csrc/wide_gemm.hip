@@ -21,7 +21,12 @@
 //
 // A stage is two K steps with one barrier, in its middle: the first step's MFMAs run while the second
 // step's X is read and the next stage's X written, then the barrier, then the second step's MFMAs
-// while the next stage's first X is read; memory instructions are spread between the MFMAs
+// while the next stage's first X is read. The 16-row tile, whose MFMAs cover none of those LDS round
+// trips, takes four K steps per stage and reads the next stage whole during a stage. Where the ranges of
+// K steps allow it a stage's offsets come from one multiply: a wavefront alone on its SIMD is bound by the
+// instructions it issues (512x1408 at M = 42: 5.6 -> 4.7 us; 2048x8192 at M = 256: 22.7 -> 20.5, at M = 7
+// unsplit 19.3 -> 16.2; four K steps per stage on 32-row tiles too: 6144x2048 at M = 56 9.45 -> 9.74, as
+// their loads then go out in bursts). Memory instructions are spread between the MFMAs
 // (sched_group_barrier), since a burst of them stalls a wavefront's MFMAs behind it (M = 640,
 // 8192 x 2048: 26.0 us without the spreading, 24.9 with). Global loads run D stages ahead. The
 // 16-bit outputs go through LDS so that a row's stores are whole 128*NF-byte segments.
@@ -75,21 +80,28 @@ __device__ __forceinline__ void wide_sync() { asm volatile("s_waitcnt lgkmcnt(0)
 // Masks of sched_group_barrier.
 constexpr int kMfma = 0x8, kVmemRead = 0x20, kDsRead = 0x100, kDsWrite = 0x200;
 
-// Stages of global loads in flight: four where a stage's MFMAs are short (2048x8192 at M = 256 on
-// 64 x 32 tiles: 29.6 us with two, 23.0 with four), two where they are long and the registers are
-// taken (128 x 128 tiles: no difference).
+// K steps of a stage, and stages of global loads in flight: eight K steps, or four where they are long and
+// the registers are taken (2048x8192 at M = 256 on 64 x 32 tiles: 29.6 us with four in flight, 23.0 with
+// eight, no better with sixteen; 128 x 128 tiles: no difference).
+template <int NF, int MT>
+constexpr int wide_steps() {
+  return NF * MT == 1 ? 4 : 2;
+}
 template <int NF, int MT>
 constexpr int wide_depth() {
-  return NF * MT <= 8 ? 4 : 2;
+  return wide_steps<NF, MT>() == 4 ? 2 : NF * MT <= 8 ? 4 : 2;
 }
 
-template <int DT, int NF, int MT, bool ACT>
+template <int DT, int NF, int MT, bool ACT, bool ALIGNED>
 __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) {
-  constexpr int D = wide_depth<NF, MT>();
-  constexpr int XN = (2 * MT + 3) / 4;                     // X loads of a wavefront per stage (8 rows each)
+  constexpr int D = wide_depth<NF, MT>(), S = wide_steps<NF, MT>();
+  constexpr int CH = 4 * S;                                // 16-byte chunks of an X row of a stage
+  constexpr int GR = 64 / CH;                              // rows of one load instruction
+  constexpr int GROUPS = 16 * MT / GR;                     // load instructions of a stage, over the workgroup
+  constexpr int XN = (GROUPS + 3) / 4;                     // and of a wavefront
   constexpr int OF = ACT ? NF / 2 : NF;                    // output fragments per wavefront
   constexpr int OC = 8 * OF;                               // 16-byte chunks of a row of the output tile
-  constexpr int kStageWords = 2 * MT * 64;                 // u32x4 of one stage of X
+  constexpr int kStageWords = GROUPS * 64;                 // u32x4 of one stage of X
   constexpr int kOutWords = 16 * MT * OC;                  // u32x4 of the 16-bit output tile
   __shared__ __attribute__((aligned(16))) u32x4 lds[2 * kStageWords > kOutWords ? 2 * kStageWords : kOutWords];
   const int lane = threadIdx.x & 63;
@@ -100,12 +112,12 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
   if (item >= a.tiles * a.split) return;
   const int ns = item / a.mtiles, mt = item - ns * a.mtiles;
   const int nt = a.split == 1 ? ns : ns / a.split, sp = ns - nt * a.split;
-  // K steps [lo, hi), stages of two from lo; k_tail of the last stage's 64 K elements are real.
+  // K steps [lo, hi), stages of S from lo; k_tail of the last stage's 32 S K elements are real.
   const int lo = a.split == 1 ? 0 : static_cast<int>(static_cast<uint32_t>(sp * a.Ks) / static_cast<uint32_t>(a.split));
   const int hi = a.split == 1 ? a.Ks
                               : static_cast<int>(static_cast<uint32_t>((sp + 1) * a.Ks) / static_cast<uint32_t>(a.split));
-  const int stages = (hi - lo + 1) >> 1;
-  const int k_tail = min(a.K, 32 * hi) - 32 * lo - 64 * (stages - 1);
+  const int stages = (hi - lo + S - 1) / S;
+  const int k_tail = min(a.K, 32 * hi) - 32 * lo - 32 * S * (stages - 1);
   const auto wr = make_rsrc(a.w, a.wbytes);
   const auto xr = make_rsrc(a.x, static_cast<uint32_t>(static_cast<int64_t>(a.M) * a.ldx * 2));
   const int of0 = (nt * kWideWaves + wave) * OF;           // this wavefront's first output fragment
@@ -117,38 +129,54 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
   }
 #pragma unroll
   for (int j = 0; j < XN; ++j) {
-    const int g = wave + 4 * j;                            // rows 8g .. 8g+7 of the tile, a row's 128 B per 8 lanes
-    const int row = mt * 16 * MT + 8 * g + (lane >> 3);
-    const int chunk = (lane & 7) ^ (lane >> 3);
-    xo[j] = (g < 2 * MT && row < a.M) ? static_cast<uint32_t>(static_cast<int64_t>(row) * a.ldx * 2) + 16u * chunk
+    const int g = wave + 4 * j;                            // rows GR g ... of the tile, CH lanes each
+    const int row = mt * 16 * MT + GR * g + lane / CH;
+    const int chunk = (lane % CH) ^ ((GR * wave + lane / CH) % CH);
+    xo[j] = (g < GROUPS && row < a.M) ? static_cast<uint32_t>(static_cast<int64_t>(row) * a.ldx * 2) + 16u * chunk
                                       : kOutOfRange;
     xl[j] = 8 * chunk < k_tail ? 0u : kOutOfRange;
   }
-  const int rd0 = (lane & 15) * 8 + ((lane >> 4) ^ (lane & 7));  // K step 0 of a stage, row lane % 16
-  const int rd1 = rd0 ^ 4;                                       // K step 1
-  u32x4 W[2 * D][NF], X[D][XN], B0[MT], B1[MT];
-  // Past the last step the sign bit puts the whole load out of range (zeros, no traffic).
-  auto w_off = [&](int s) __attribute__((always_inline)) {
-    return __builtin_amdgcn_readfirstlane(static_cast<int>(
-        pack_step_offset(lo + s, a.wgroup) | (static_cast<uint32_t>(hi - lo - 1 - s) & kWideNoLoad)));
+  const int rd0 = (lane & 15) * CH + ((lane >> 4) ^ (lane & 15) % CH);  // K step h of a stage: rd0 ^ 4h
+  u32x4 W[S * D][NF], X[D][XN];
+  // A stage's scalar offsets, with the sign bit set past the last stage: it puts the whole load out of
+  // range (zeros, no traffic). With ALIGNED ranges eight K steps lie in one group of the packed weight, a
+  // D-stage block apart: one multiply per stage and the steps as instruction offsets. A wavefront alone
+  // on its SIMD issues about one instruction per four clocks, so these counts are what short tiles run at.
+  struct StageOffsets {
+    int w[S], x;
+    uint32_t tail;  // in the last stage, the bit that takes lanes past K out of range
   };
-  auto load_w = [&](int so, int f, u32x4& w) __attribute__((always_inline)) {
-    w = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, wo[f], so, 0));
+  auto offsets = [&](int i, int jw) __attribute__((always_inline)) {
+    StageOffsets o;
+    const uint32_t gone = i < stages ? 0u : kWideNoLoad;
+    if constexpr (ALIGNED) {
+      const uint32_t base = (static_cast<uint32_t>(lo + S * i) >> 3) * a.wgroup + static_cast<uint32_t>(jw * S) * kPackFragBytes;
+      o.w[0] = static_cast<int>(base | gone);
+    } else {
+#pragma unroll
+      for (int h = 0; h < S; ++h)
+        o.w[h] = __builtin_amdgcn_readfirstlane(static_cast<int>(
+            pack_step_offset(lo + S * i + h, a.wgroup) | (static_cast<uint32_t>(hi - lo - 1 - S * i - h) & kWideNoLoad)));
+    }
+    o.x = static_cast<int>((static_cast<uint32_t>(lo + S * i) * 64u) | gone);
+    o.tail = i == stages - 1 ? kOutOfRange : 0u;
+    return o;
   };
-  auto load_x = [&](int i, u32x4 (&x)[XN]) __attribute__((always_inline)) {
-    const int left = stages - 1 - i;
-    const int so = __builtin_amdgcn_readfirstlane(
-        static_cast<int>((static_cast<uint32_t>(i) * 128u + static_cast<uint32_t>(lo) * 64u) | (static_cast<uint32_t>(left) & kWideNoLoad)));
-    const uint32_t last = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(~((left | -left) >> 31))) & kOutOfRange;
+  auto load_w = [&](const StageOffsets& o, int h, int f, u32x4& w) __attribute__((always_inline)) {
+    if constexpr (ALIGNED)
+      w = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, wo[f] + h * kPackFragBytes, o.w[0], 0));
+    else
+      w = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, wo[f], o.w[h], 0));
+  };
+  auto load_x = [&](const StageOffsets& o, u32x4 (&x)[XN]) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < XN; ++j)
-      x[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                     xr, (xl[j] & last) != 0 ? kOutOfRange : xo[j], so, 0));
+      x[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, xo[j] | (xl[j] & o.tail), o.x, 0));
   };
   auto put_x = [&](int slot, const u32x4 (&x)[XN]) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < XN; ++j)
-      if (4 * j + 3 < 2 * MT || wave + 4 * j < 2 * MT) lds[slot * kStageWords + (wave + 4 * j) * 64 + lane] = x[j];
+      if (4 * j + 3 < GROUPS || wave + 4 * j < GROUPS) lds[slot * kStageWords + (wave + 4 * j) * 64 + lane] = x[j];
   };
   f32x4 acc[NF][MT];
 #pragma unroll
@@ -157,82 +185,125 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
     for (int t = 0; t < MT; ++t) acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int j = 0; j < D; ++j) {
-    load_x(j, X[j]);
+    const StageOffsets o = offsets(j, j);
+    load_x(o, X[j]);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int so = w_off(2 * j + h);
+    for (int h = 0; h < S; ++h)
 #pragma unroll
-      for (int f = 0; f < NF; ++f) load_w(so, f, W[2 * j + h][f]);
-    }
+      for (int f = 0; f < NF; ++f) load_w(o, h, f, W[S * j + h][f]);
     __builtin_amdgcn_sched_barrier(0);
   }
   put_x(0, X[0]);
-  load_x(D, X[0]);
-  wide_sync();
+  load_x(offsets(D, 0), X[0]);
+  if constexpr (S == 4) {
+    // Two buffers of operands: while a stage's MFMAs run, the next stage's X is read whole and the one
+    // after it written, so a stage waits for one LDS round trip.
+    u32x4 B[2][S][MT];
+    wide_sync();
 #pragma unroll
-  for (int t = 0; t < MT; ++t) B0[t] = lds[t * 128 + rd0];
-  // Stage i in register slot j = i % D. B0 holds its first K step's X operands.
-  auto stage = [&](int j, int i) __attribute__((always_inline)) {
-    const int slot = j & 1, jn = (j + 1) % D;
-    const int w0 = w_off(2 * (i + D)), w1 = w_off(2 * (i + D) + 1);
+    for (int h = 0; h < S; ++h)
 #pragma unroll
-    for (int t = 0; t < MT; ++t) B1[t] = lds[slot * kStageWords + t * 128 + rd1];
-#pragma unroll
-    for (int f = 0; f < NF; ++f) {
-#pragma unroll
-      for (int t = 0; t < MT; ++t) acc[f][t] = mfma_16x16x32<DT>(W[2 * j][f], B0[t], acc[f][t]);
-      load_w(w0, f, W[2 * j][f]);
-    }
-    put_x(slot ^ 1, X[jn]);
-    load_x(i + 1 + D, X[jn]);
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
-      if (NF == 1 && t < XN) {
-        __builtin_amdgcn_sched_group_barrier(kDsWrite, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(kVmemRead, 1, 0);
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < (NF - 1) * MT; ++t) {
-      if ((t & 1) == 0 && t / 2 < XN)
-        __builtin_amdgcn_sched_group_barrier(kDsWrite, 1, 0);
-      else
-        __builtin_amdgcn_sched_group_barrier(kVmemRead, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
-    }
-    // Every wavefront has read this stage's X and written the next one's.
+      for (int t = 0; t < MT; ++t) B[0][h][t] = lds[t * 16 * CH + (rd0 ^ (4 * h))];
+    put_x(1, X[1]);
+    load_x(offsets(D + 1, 1), X[1]);
     wide_sync();
     __builtin_amdgcn_sched_barrier(0);
+    // Stage i in register slot j = i % D (D = 2), which is also its LDS slot.
+    auto stage = [&](int j, int i) __attribute__((always_inline)) {
+      const StageOffsets o = offsets(i + D, j);
 #pragma unroll
-    for (int t = 0; t < MT; ++t) B0[t] = lds[(slot ^ 1) * kStageWords + t * 128 + rd0];
+      for (int h = 0; h < S; ++h)
 #pragma unroll
-    for (int f = 0; f < NF; ++f) {
+        for (int t = 0; t < MT; ++t) B[j ^ 1][h][t] = lds[(j ^ 1) * kStageWords + t * 16 * CH + (rd0 ^ (4 * h))];
 #pragma unroll
-      for (int t = 0; t < MT; ++t) acc[f][t] = mfma_16x16x32<DT>(W[2 * j + 1][f], B1[t], acc[f][t]);
-      load_w(w1, f, W[2 * j + 1][f]);
+      for (int h = 0; h < S; ++h) {
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+#pragma unroll
+          for (int t = 0; t < MT; ++t) acc[f][t] = mfma_16x16x32<DT>(W[S * j + h][f], B[j][h][t], acc[f][t]);
+          load_w(o, h, f, W[S * j + h][f]);
+        }
+      }
+      put_x(j, X[j]);  // stage i + 2: every wavefront read stage i's X before the last barrier
+      load_x(offsets(i + 2 + D, j), X[j]);
+      wide_sync();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int j = 0; j < D; ++j) stage(j, j);
+    for (int i = D; i < stages; i += D) {
+#pragma unroll
+      for (int j = 0; j < D; ++j) stage(j, i + j);
     }
+  } else {
+    u32x4 B0[MT], B1[MT];
+    const int rd1 = rd0 ^ 4;
+    wide_sync();
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+    for (int t = 0; t < MT; ++t) B0[t] = lds[t * 128 + rd0];
+    // Stage i in register slot j = i % D. B0 holds its first K step's X operands.
+    auto stage = [&](int j, int i) __attribute__((always_inline)) {
+      const int slot = j & 1, jn = (j + 1) % D;
+      const StageOffsets o = offsets(i + D, j), ox = offsets(i + 1 + D, jn);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) B1[t] = lds[slot * kStageWords + t * 128 + rd1];
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[f][t] = mfma_16x16x32<DT>(W[2 * j][f], B0[t], acc[f][t]);
+        load_w(o, 0, f, W[2 * j][f]);
+      }
+      put_x(slot ^ 1, X[jn]);
+      load_x(ox, X[jn]);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+        if (NF == 1 && t < XN) {
+          __builtin_amdgcn_sched_group_barrier(kDsWrite, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(kVmemRead, 1, 0);
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < (NF - 1) * MT; ++t) {
+        if ((t & 1) == 0 && t / 2 < XN)
+          __builtin_amdgcn_sched_group_barrier(kDsWrite, 1, 0);
+        else
+          __builtin_amdgcn_sched_group_barrier(kVmemRead, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+      }
+      // Every wavefront has read this stage's X and written the next one's.
+      wide_sync();
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) B0[t] = lds[(slot ^ 1) * kStageWords + t * 128 + rd0];
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[f][t] = mfma_16x16x32<DT>(W[2 * j + 1][f], B1[t], acc[f][t]);
+        load_w(o, 1, f, W[2 * j + 1][f]);
+      }
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+      }
+#pragma unroll
+      for (int f = 1; f < NF; ++f) {
+        __builtin_amdgcn_sched_group_barrier(kVmemRead, 1, 0);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // The first D stages peeled off: the loop is entered only with its own load order in flight, so the
+    // compiler's load-count waits stay exact. Stages past the last multiply zeros.
+#pragma unroll
+    for (int j = 0; j < D; ++j) stage(j, j);
+    for (int i = D; i < stages; i += D) {
+#pragma unroll
+      for (int j = 0; j < D; ++j) stage(j, i + j);
     }
-#pragma unroll
-    for (int f = 1; f < NF; ++f) {
-      __builtin_amdgcn_sched_group_barrier(kVmemRead, 1, 0);
-#pragma unroll
-      for (int t = 0; t < MT; ++t) __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  // The first D stages peeled off: the loop is entered only with its own load order in flight, so the
-  // compiler's load-count waits stay exact. Stages past the last multiply zeros.
-#pragma unroll
-  for (int j = 0; j < D; ++j) stage(j, j);
-  for (int i = D; i < stages; i += D) {
-#pragma unroll
-    for (int j = 0; j < D; ++j) stage(j, i + j);
   }
 
   if (a.split > 1) {
@@ -392,8 +463,13 @@ hipError_t wide_go(WideArgs a, hipStream_t stream) {
   a.mtiles = static_cast<int>(mtiles);
   a.tiles = static_cast<int>(mtiles * ntiles);
   a.per_xcd = (a.tiles * a.split + 7) / 8;
-  hipLaunchKernelGGL((wide_gemm_kernel<DT, NF, MT, ACT>), dim3(static_cast<unsigned>(8 * a.per_xcd)), dim3(kWideThreads),
-                     0, stream, a);
+  // Every range of K steps starts at a group of the packed weight and, but for K's end (zero fragments
+  // follow), ends at one.
+  constexpr bool block = wide_steps<NF, MT>() * wide_depth<NF, MT>() == kPackGroup;
+  auto kern = wide_gemm_kernel<DT, NF, MT, ACT, false>;
+  if constexpr (block)
+    if (a.split == 1 || a.Ks % (kPackGroup * a.split) == 0) kern = wide_gemm_kernel<DT, NF, MT, ACT, true>;
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(8 * a.per_xcd)), dim3(kWideThreads), 0, stream, a);
   return hipGetLastError();
 }
 
