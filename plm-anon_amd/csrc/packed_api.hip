@@ -589,6 +589,28 @@ int plm_gemm_packed_lora(int32_t dtype, const void* x, int64_t ldx, const void* 
   status = plm::packed_check_linear(dtype, gh, M);
   if (status != PLM_OK) return status;
   if (base_tiles + l.h_tiles > plm::kPackedBarrierBase - plm::kPackedArriveBase) return PLM_ERR_ARGUMENT;
+  if (plm::wide_preferred(M, N, K, t)) {
+    plm::PackedArgs dry{};
+    dry.M = static_cast<int>(M);
+    if (plm::packed_dispatch_dt(dtype, dry, t, 1, nullptr, true, plm::kEpiLora) != hipSuccess) return PLM_ERR_TILE;
+    plm::WideLoraCall c{};
+    c.packed_a = packed_a;
+    c.b = static_cast<const uint16_t*>(lora_b);
+    c.width = static_cast<int>(width);
+    c.rank = static_cast<int>(rank);
+    c.gated_from = static_cast<int>(gated_from);
+    for (int i = 0; i < 3; ++i) c.shard_end[i] = z.shard_end[i];
+    // h is to be written before the base tiles' K steps end: unsplit it takes their whole K range (M = 110,
+    // 4608x3072, rank 64: 18.1 us against 16.2 with four splits), but up to 1024 K elements that is
+    // shorter than a split's round trip (M = 42, 768x512: 6.1 against 7.3).
+    c.h_split = plm::ksteps(K) <= 32 ? 1 : static_cast<int>(std::min<int64_t>(l.h_split, 4));
+    c.h_partial = l.h_partial;
+    c.h_offset = l.h_offset;
+    c.spin_limit = plm::kPackedSpinLimit;
+    c.workspace = workspace;
+    const int ran = plm::wide_lora(dtype, x, ldx, packed_w, y, ldy, M, N, K, t.split_k, c, static_cast<hipStream_t>(stream));
+    if (ran != PLM_ERR_ARGUMENT) return ran;
+  }
   z.pre = gh;
   z.b = static_cast<const uint16_t*>(lora_b);
   z.rank = static_cast<int>(rank);

@@ -24,4 +24,19 @@ enum class WideOut { kModel, kF32, kActPlain, kActInterleaved };
 int wide_gemm(int32_t dtype, const void* x, int64_t ldx, const void* wp, void* y, int64_t ldy, int64_t M, int64_t N,
               int64_t K, hipStream_t stream, WideOut out, int split = 1, void* workspace = nullptr);
 
+// The gated-LoRA launch's second half: h = X A^T and the correction (plm_gemm_packed_lora).
+struct WideLoraCall {
+  const void* packed_a;
+  const uint16_t* b;          // [N][rank]
+  int width, rank, gated_from;
+  int shard_end[3];
+  int h_split;                // K splits of the h linear
+  int64_t h_partial;          // its partials' float offset behind the counter area
+  int64_t h_offset;           // h's byte offset in the workspace
+  int spin_limit;
+  void* workspace;
+};
+int wide_lora(int32_t dtype, const void* x, int64_t ldx, const void* wp, void* y, int64_t ldy, int64_t M, int64_t N,
+              int64_t K, int split, const WideLoraCall& c, hipStream_t stream);
+
 }  // namespace plm

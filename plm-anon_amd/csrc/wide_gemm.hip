@@ -2,7 +2,8 @@
 // reference hands to F.linear, plm/rounds.py:16, plm/fast_gemm.py:108-111), so that a caller that
 // keeps only the packed copy of a weight has a compute-bound kernel for them; for single linears of a
 // round on row-split tiles (packed_api.hip, wide_preferred), where its X, read once per workgroup, beats
-// the packed kernel's; and both with a fused gate/up projection's SiLU-and-multiply as the epilogue.
+// the packed kernel's; both with a fused gate/up projection's SiLU-and-multiply as the epilogue; and the
+// gated-LoRA launch on such tiles.
 //
 // Every output is one MFMA chain over the K steps in ascending order (v_mfma_f32_16x16x32), the
 // order of a row-split packed tile without K splits; it is also what torch's F.linear returned bit for
@@ -38,6 +39,7 @@
 // 7.9 / 12.0 / 16.6. Rows past N or M and K past K load zeros (buffer range checks, per-lane masks) and are never stored.
 #include <hip/hip_runtime.h>
 
+#include "packed_gemm.h"
 #include "plm_amd.h"
 #include "tile.h"
 #include "wide_gemm.h"
@@ -48,6 +50,30 @@ namespace {
 constexpr int kWideWaves = 4;
 constexpr int kWideThreads = 64 * kWideWaves;
 constexpr uint32_t kWideNoLoad = 0x80000000u;
+
+// What the kernel's stores are: the product, a fused gate/up projection's activation, or the gated-LoRA
+// launch's base linear (with the h linear's workgroups ahead of it).
+constexpr int kWidePlain = 0, kWideAct = 1, kWideLora = 2;
+
+// The gated-LoRA launch (plm_gemm_packed_lora): workgroups [0, items) form h = X A^T in the model dtype,
+// the base linear's workgroups follow, wait for h once their own sums are formed, and add the rank-r
+// correction as MFMAs. Against the packed kernel's launch, which adds it as scalar products (us, base
+// linear alone in brackets): 3072x2048, rank 16, M = 56 13.6 [9.9] -> 11.1 [7.3]; 11264x2048 38.2 [23.1] ->
+// 15.2 [12.2]; 4608x3072, rank 64, M = 110 61.5 [29.6] -> 16.2 [11.9]. What is left over the base linear is
+// h's chain: X, the partial sums' round trip, h's own.
+struct WideLora {
+  const void* w;     // A, packed
+  uint16_t* h;       // [M][width]
+  const uint16_t* b; // [N][rank]
+  uint32_t wbytes, wgroup;
+  int width, split, tiles, items, rank, gated_from;
+  int base_tiles;
+  int shard_end[3];  // exclusive column ends of the first three shards (N past the last)
+  float* partial;
+  int* arrive;
+  int* counters;     // the workspace's: h tiles written, base tiles past their wait, the error flag
+  int spin_limit;
+};
 
 struct WideArgs {
   const void* x;
@@ -62,6 +88,7 @@ struct WideArgs {
   int* arrive;             // split > 1: one arrival counter per tile
   int gate_step, up_step;  // activation: fragment g's gate rows lie in weight fragment g * gate_step,
                            // its up rows up_step fragments further
+  WideLora lora;           // kWideLora only
 };
 
 template <int DT>
@@ -92,8 +119,24 @@ constexpr int wide_depth() {
   return wide_steps<NF, MT>() == 4 ? 2 : NF * MT <= 8 ? 4 : 2;
 }
 
-template <int DT, int NF, int MT, bool ACT, bool ALIGNED>
+// The base linear's wait (bounded) until every h tile is written.
+__device__ __forceinline__ void wide_wait_h(const WideLora& z) {
+  for (int i = 0;; ++i) {
+    if (__builtin_amdgcn_readfirstlane(collect(z.counters + kPkLoraHDone)) >= z.tiles) return;
+    if (i >= z.spin_limit) {
+      if ((threadIdx.x & 63) == 0) publish(z.counters + kPkErrorSlot, 1);
+      return;
+    }
+    if (i % kErrorCheckPolls == kErrorCheckPolls - 1 &&
+        __builtin_amdgcn_readfirstlane(collect(z.counters + kPkErrorSlot)) != 0)
+      return;
+    __builtin_amdgcn_s_sleep(1);
+  }
+}
+
+template <int DT, int NF, int MT, int EPI, bool ALIGNED>
 __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) {
+  constexpr bool ACT = EPI == kWideAct;
   constexpr int D = wide_depth<NF, MT>(), S = wide_steps<NF, MT>();
   constexpr int CH = 4 * S;                                // 16-byte chunks of an X row of a stage
   constexpr int GR = 64 / CH;                              // rows of one load instruction
@@ -108,7 +151,23 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // Workgroups go round the 8 XCDs; each XCD takes a run of items, X tiles fastest, then splits, so
   // that a weight tile is read into one XCD's L2 only.
-  const int item = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
+  int block = blockIdx.x;
+  bool forms_h = false;
+  if constexpr (EPI == kWideLora) {
+    forms_h = block < a.lora.items;
+    block -= a.lora.items;
+    if (forms_h) {
+      a.w = a.lora.w;
+      a.N = a.lora.width;
+      a.wbytes = a.lora.wbytes;
+      a.wgroup = a.lora.wgroup;
+      a.split = a.lora.split;
+      a.tiles = a.lora.tiles;
+      a.partial = a.lora.partial;
+      a.arrive = a.lora.arrive;
+    }
+  }
+  const int item = forms_h ? static_cast<int>(blockIdx.x) : (block & 7) * a.per_xcd + (block >> 3);
   if (item >= a.tiles * a.split) return;
   const int ns = item / a.mtiles, mt = item - ns * a.mtiles;
   const int nt = a.split == 1 ? ns : ns / a.split, sp = ns - nt * a.split;
@@ -135,6 +194,22 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
     xo[j] = (g < GROUPS && row < a.M) ? static_cast<uint32_t>(static_cast<int64_t>(row) * a.ldx * 2) + 16u * chunk
                                       : kOutOfRange;
     xl[j] = 8 * chunk < k_tail ? 0u : kOutOfRange;
+  }
+  // Gated LoRA: the first 32 rank elements of this wavefront's rows of B, as MFMA operands (row lane % 16,
+  // elements 8 * (lane / 16) ..), requested ahead of everything else.
+  [[maybe_unused]] u32x4 b_first[NF];
+  [[maybe_unused]] __amdgpu_buffer_rsrc_t br;
+  [[maybe_unused]] auto load_b = [&](int f, int j) __attribute__((always_inline)) {
+    const int n = 16 * (of0 + f) + (lane & 15), e = 32 * j + 8 * (lane >> 4);
+    const uint32_t off = n < a.N && e < a.lora.rank ? static_cast<uint32_t>((n * a.lora.rank + e) * 2) : kOutOfRange;
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(br, static_cast<int>(off), 0, 0));
+  };
+  if constexpr (EPI == kWideLora) {
+    if (!forms_h) {
+      br = make_rsrc(a.lora.b, static_cast<uint32_t>(a.N * a.lora.rank * 2));
+#pragma unroll
+      for (int f = 0; f < NF; ++f) b_first[f] = load_b(f, 0);
+    }
   }
   const int rd0 = (lane & 15) * CH + ((lane >> 4) ^ (lane & 15) % CH);  // K step h of a stage: rd0 ^ 4h
   u32x4 W[S * D][NF], X[D][XN];
@@ -368,6 +443,74 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
     }
   }
 
+  if constexpr (EPI == kWideLora) {
+    const WideLora& z = a.lora;
+    if (forms_h) {
+      // Written through for the base workgroups of every XCD, then counted in.
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          const int m = mt * 16 * MT + 16 * t + (lane & 15), n = 16 * (of0 + f) + 4 * (lane >> 4);
+          if (m >= a.M || n >= a.N) continue;  // the width is a multiple of 8: all four columns are in range
+          const f32x4 v = acc[f][t];
+          const uint64_t lo2 = static_cast<uint64_t>(to_bits16<DT>(v[0])) | (static_cast<uint64_t>(to_bits16<DT>(v[1])) << 16);
+          const uint64_t hi2 = static_cast<uint64_t>(to_bits16<DT>(v[2])) | (static_cast<uint64_t>(to_bits16<DT>(v[3])) << 16);
+          publish(reinterpret_cast<uint64_t*>(z.h + static_cast<int64_t>(m) * z.width + n), lo2 | (hi2 << 32));
+        }
+      __builtin_amdgcn_s_waitcnt(0);
+      wide_sync();
+      if (threadIdx.x == 0)
+        __hip_atomic_fetch_add(z.counters + kPkLoraHDone, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
+    }
+    wide_wait_h(z);
+    // Rows m >= gated_from: the base value rounded to the model dtype plus sum_j h[m, s rank + j] B[n, j],
+    // s the shard of column n, as MFMAs over 32 rank elements; a fragment's columns of other shards than
+    // the one at hand are zero rows of B.
+    const auto hr = make_rsrc(z.h, static_cast<uint32_t>(a.M * z.width * 2));
+    auto shard_of = [&](int n) { return (n >= z.shard_end[0]) + (n >= z.shard_end[1]) + (n >= z.shard_end[2]); };
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const int nf = __builtin_amdgcn_readfirstlane(16 * (of0 + f));
+      const int s_lo = shard_of(nf), s_hi = shard_of(min(nf + 15, a.N - 1));
+      const int s_own = shard_of(nf + (lane & 15));
+      f32x4 corr[MT];
+#pragma unroll
+      for (int t = 0; t < MT; ++t) corr[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; 32 * j < z.rank; ++j) {
+        const u32x4 row = j == 0 ? b_first[f] : load_b(f, j);
+        const int e = 32 * j + 8 * (lane >> 4);
+        for (int s = s_lo; s <= s_hi; ++s) {
+          const u32x4 bs = s_own == s ? row : u32x4{0u, 0u, 0u, 0u};
+          u32x4 hv[MT];
+#pragma unroll
+          for (int t = 0; t < MT; ++t) {
+            const int m = mt * 16 * MT + 16 * t + (lane & 15);
+            const uint32_t off = m < a.M && e < z.rank ? static_cast<uint32_t>((m * z.width + s * z.rank + e) * 2) : kOutOfRange;
+            hv[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(hr, static_cast<int>(off), 0, kCoherent));
+          }
+#pragma unroll
+          for (int t = 0; t < MT; ++t) corr[t] = mfma_16x16x32<DT>(bs, hv[t], corr[t]);
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const bool gated = mt * 16 * MT + 16 * t + (lane & 15) >= z.gated_from;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          acc[f][t][r] = gated ? from_bits16<DT>(to_bits16<DT>(acc[f][t][r])) + corr[t][r] : acc[f][t][r];
+      }
+    }
+    // The last base tile to pass its wait leaves both counters ready for the next launch.
+    wide_sync();
+    if (threadIdx.x == 0 && __hip_atomic_fetch_add(z.counters + kPkLoraPast, 1, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT) == z.base_tiles - 1) {
+      publish(z.counters + kPkLoraHDone, 0);
+      publish(z.counters + kPkLoraPast, 0);
+    }
+  }
+
   // Fragment (f, t): output columns n0 + 16f + 4*(lane/16) + r, row m0 + 16t + lane%16.
   const int m0 = mt * 16 * MT;
   if constexpr (!ACT) {
@@ -405,7 +548,6 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
   wide_sync();
   uint16_t* y = static_cast<uint16_t*>(a.y);
   const bool wide16 = (reinterpret_cast<uintptr_t>(y) & 15) == 0 && (a.ldy & 7) == 0;
-#pragma unroll
   for (int i = threadIdx.x; i < kOutWords; i += kWideThreads) {
     const int row = i / OC, c = i - row * OC;
     const int m = m0 + row, n = 16 * (nt * kWideWaves * OF) + 8 * c;
@@ -454,68 +596,72 @@ WideTile wide_pick(int64_t M, int64_t N, int64_t split, bool act) {
   return best;
 }
 
-template <int DT, int NF, int MT, bool ACT>
+template <int DT, int NF, int MT, int EPI>
 hipError_t wide_go(WideArgs a, hipStream_t stream) {
-  constexpr int tn = 64 * NF / (ACT ? 2 : 1), tm = 16 * MT;
+  constexpr int tn = 64 * NF / (EPI == kWideAct ? 2 : 1), tm = 16 * MT;
   const int64_t mtiles = (a.M + tm - 1) / tm, ntiles = (static_cast<int64_t>(a.N) + tn - 1) / tn;
+  int64_t counters = a.split > 1 ? mtiles * ntiles : 0;
   if (mtiles * ntiles * a.split > (int64_t(1) << 28)) return hipErrorInvalidConfiguration;
-  if (a.split > 1 && mtiles * ntiles > kPackedBarrierBase - kPackedArriveBase) return hipErrorInvalidConfiguration;
   a.mtiles = static_cast<int>(mtiles);
   a.tiles = static_cast<int>(mtiles * ntiles);
   a.per_xcd = (a.tiles * a.split + 7) / 8;
+  unsigned grid = static_cast<unsigned>(8 * a.per_xcd);
+  if constexpr (EPI == kWideLora) {
+    a.lora.base_tiles = a.tiles;
+    a.lora.tiles = static_cast<int>(mtiles * ((a.lora.width + tn - 1) / tn));
+    a.lora.items = a.lora.tiles * a.lora.split;
+    a.lora.arrive = a.lora.counters + kPackedArriveBase + counters;
+    counters += a.lora.split > 1 ? a.lora.tiles : 0;
+    grid += static_cast<unsigned>(a.lora.items);
+  }
+  if (counters > kPackedBarrierBase - kPackedArriveBase) return hipErrorInvalidConfiguration;
   // Every range of K steps starts at a group of the packed weight and, but for K's end (zero fragments
   // follow), ends at one.
+  auto aligned = [&](int split) { return split == 1 || a.Ks % (kPackGroup * split) == 0; };
   constexpr bool block = wide_steps<NF, MT>() * wide_depth<NF, MT>() == kPackGroup;
-  auto kern = wide_gemm_kernel<DT, NF, MT, ACT, false>;
+  auto kern = wide_gemm_kernel<DT, NF, MT, EPI, false>;
   if constexpr (block)
-    if (a.split == 1 || a.Ks % (kPackGroup * a.split) == 0) kern = wide_gemm_kernel<DT, NF, MT, ACT, true>;
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(8 * a.per_xcd)), dim3(kWideThreads), 0, stream, a);
+    if (aligned(a.split) && (EPI != kWideLora || aligned(a.lora.split))) kern = wide_gemm_kernel<DT, NF, MT, EPI, true>;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(kWideThreads), 0, stream, a);
   return hipGetLastError();
 }
 
-template <int DT, bool ACT>
+template <int DT, int EPI>
 hipError_t wide_dispatch(const WideArgs& a, WideTile t, hipStream_t s) {
   switch (16 * t.nf + t.mt) {
-    case 16 * 2 + 1: return wide_go<DT, 2, 1, ACT>(a, s);
-    case 16 * 2 + 2: return wide_go<DT, 2, 2, ACT>(a, s);
-    case 16 * 2 + 3: return wide_go<DT, 2, 3, ACT>(a, s);
-    case 16 * 2 + 4: return wide_go<DT, 2, 4, ACT>(a, s);
-    case 16 * 2 + 5: return wide_go<DT, 2, 5, ACT>(a, s);
-    case 16 * 2 + 6: return wide_go<DT, 2, 6, ACT>(a, s);
-    case 16 * 2 + 8: return wide_go<DT, 2, 8, ACT>(a, s);
-    case 16 * 2 + 10: return wide_go<DT, 2, 10, ACT>(a, s);
-    case 16 * 4 + 8: return wide_go<DT, 4, 8, ACT>(a, s);
+    case 16 * 2 + 1: return wide_go<DT, 2, 1, EPI>(a, s);
+    case 16 * 2 + 2: return wide_go<DT, 2, 2, EPI>(a, s);
+    case 16 * 2 + 3: return wide_go<DT, 2, 3, EPI>(a, s);
+    case 16 * 2 + 4: return wide_go<DT, 2, 4, EPI>(a, s);
+    case 16 * 2 + 5: return wide_go<DT, 2, 5, EPI>(a, s);
+    case 16 * 2 + 6: return wide_go<DT, 2, 6, EPI>(a, s);
+    case 16 * 2 + 8: return wide_go<DT, 2, 8, EPI>(a, s);
     default: break;
   }
-  if constexpr (!ACT) {
+  if constexpr (EPI != kWideLora) {  // past 128 rows, or more than 256 tiles of 128 x 128
     switch (16 * t.nf + t.mt) {
-      case 16 + 1: return wide_go<DT, 1, 1, ACT>(a, s);
-      case 16 + 2: return wide_go<DT, 1, 2, ACT>(a, s);
-      case 16 + 3: return wide_go<DT, 1, 3, ACT>(a, s);
-      case 16 + 4: return wide_go<DT, 1, 4, ACT>(a, s);
-      case 16 + 5: return wide_go<DT, 1, 5, ACT>(a, s);
-      case 16 + 8: return wide_go<DT, 1, 8, ACT>(a, s);
+      case 16 * 2 + 10: return wide_go<DT, 2, 10, EPI>(a, s);
+      case 16 * 4 + 8: return wide_go<DT, 4, 8, EPI>(a, s);
+      default: break;
+    }
+  }
+  if constexpr (EPI != kWideAct) {
+    switch (16 * t.nf + t.mt) {
+      case 16 + 1: return wide_go<DT, 1, 1, EPI>(a, s);
+      case 16 + 2: return wide_go<DT, 1, 2, EPI>(a, s);
+      case 16 + 3: return wide_go<DT, 1, 3, EPI>(a, s);
+      case 16 + 4: return wide_go<DT, 1, 4, EPI>(a, s);
+      case 16 + 5: return wide_go<DT, 1, 5, EPI>(a, s);
+      case 16 + 8: return wide_go<DT, 1, 8, EPI>(a, s);
       default: break;
     }
   }
   return hipErrorInvalidConfiguration;
 }
 
-}  // namespace
-
-// The scratch a caller of plm_gemm_packed provides above 128 rows. The kernel itself needs none (a K
-// split would change the sums' order); the sizes callers reserve and the refusal of a smaller
-// workspace are the interface's and stay.
-int64_t wide_workspace(int64_t M, int64_t N, int64_t K, int64_t cap) {
-  const int64_t tiles = ((N + 127) / 128) * ((M + 127) / 128), ks = (K + 31) / 32;
-  const auto bytes = [&](int64_t s) { return static_cast<int64_t>(kCounterBytes) + tiles * s * 64 * 1024; };
-  int64_t split = 1;
-  while (tiles * split * 2 <= 320 && ks / (split * 2) >= 16 && split < 8 && bytes(split * 2) <= cap) split *= 2;
-  return split == 1 ? 0 : bytes(split);
-}
-
-int wide_gemm(int32_t dtype, const void* x, int64_t ldx, const void* wp, void* y, int64_t ldy, int64_t M, int64_t N,
-              int64_t K, hipStream_t stream, WideOut out, int split, void* workspace) {
+// Fills what every launch needs; N: the weight's rows.
+WideArgs wide_args(const void* x, int64_t ldx, const void* wp, void* y, int64_t ldy, int64_t M, int64_t N, int64_t K,
+                   WideOut out, int split, void* workspace) {
   const bool act = out == WideOut::kActPlain || out == WideOut::kActInterleaved;
   WideArgs a{};
   a.x = x;
@@ -537,13 +683,57 @@ int wide_gemm(int32_t dtype, const void* x, int64_t ldx, const void* wp, void* y
     a.arrive = static_cast<int*>(workspace) + kPackedArriveBase;
     a.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes);
   }
-  const WideTile t = wide_pick(M, a.N, split, act);
-  hipError_t err;
-  if (dtype == PLM_BF16)
-    err = act ? wide_dispatch<DT_BF16, true>(a, t, stream) : wide_dispatch<DT_BF16, false>(a, t, stream);
-  else
-    err = act ? wide_dispatch<DT_F16, true>(a, t, stream) : wide_dispatch<DT_F16, false>(a, t, stream);
+  return a;
+}
+
+int wide_status(hipError_t err) {
   return err == hipSuccess ? PLM_OK : err == hipErrorInvalidConfiguration ? PLM_ERR_ARGUMENT : PLM_ERR_LAUNCH;
+}
+
+}  // namespace
+
+// The scratch a caller of plm_gemm_packed provides above 128 rows. The kernel itself needs none (a K
+// split would change the sums' order); the sizes callers reserve and the refusal of a smaller
+// workspace are the interface's and stay.
+int64_t wide_workspace(int64_t M, int64_t N, int64_t K, int64_t cap) {
+  const int64_t tiles = ((N + 127) / 128) * ((M + 127) / 128), ks = (K + 31) / 32;
+  const auto bytes = [&](int64_t s) { return static_cast<int64_t>(kCounterBytes) + tiles * s * 64 * 1024; };
+  int64_t split = 1;
+  while (tiles * split * 2 <= 320 && ks / (split * 2) >= 16 && split < 8 && bytes(split * 2) <= cap) split *= 2;
+  return split == 1 ? 0 : bytes(split);
+}
+
+int wide_gemm(int32_t dtype, const void* x, int64_t ldx, const void* wp, void* y, int64_t ldy, int64_t M, int64_t N,
+              int64_t K, hipStream_t stream, WideOut out, int split, void* workspace) {
+  const WideArgs a = wide_args(x, ldx, wp, y, ldy, M, N, K, out, split, workspace);
+  const bool act = out == WideOut::kActPlain || out == WideOut::kActInterleaved;
+  const WideTile t = wide_pick(M, a.N, split, act);
+  if (dtype == PLM_BF16)
+    return wide_status(act ? wide_dispatch<DT_BF16, kWideAct>(a, t, stream) : wide_dispatch<DT_BF16, kWidePlain>(a, t, stream));
+  return wide_status(act ? wide_dispatch<DT_F16, kWideAct>(a, t, stream) : wide_dispatch<DT_F16, kWidePlain>(a, t, stream));
+}
+
+int wide_lora(int32_t dtype, const void* x, int64_t ldx, const void* wp, void* y, int64_t ldy, int64_t M, int64_t N,
+              int64_t K, int split, const WideLoraCall& c, hipStream_t stream) {
+  WideArgs a = wide_args(x, ldx, wp, y, ldy, M, N, K, WideOut::kModel, split, c.workspace);
+  char* ws = static_cast<char*>(c.workspace);
+  WideLora& z = a.lora;
+  z.w = c.packed_a;
+  z.h = reinterpret_cast<uint16_t*>(ws + c.h_offset);
+  z.b = c.b;
+  z.width = c.width;
+  z.wbytes = static_cast<uint32_t>(pack_bytes(c.width, a.Ks));
+  z.wgroup = pack_group_bytes(c.width);
+  z.split = c.h_split;
+  z.rank = c.rank;
+  z.gated_from = c.gated_from;
+  for (int i = 0; i < 3; ++i) z.shard_end[i] = c.shard_end[i];
+  z.partial = reinterpret_cast<float*>(ws + kCounterBytes) + c.h_partial;
+  z.counters = reinterpret_cast<int*>(ws);
+  z.spin_limit = c.spin_limit;
+  const WideTile t = wide_pick(M, N, split, false);
+  return wide_status(dtype == PLM_BF16 ? wide_dispatch<DT_BF16, kWideLora>(a, t, stream)
+                                       : wide_dispatch<DT_F16, kWideLora>(a, t, stream));
 }
 
 }  // namespace plm

@@ -16,7 +16,6 @@ linear method (plm/gated_lora.py:60-89).
 from __future__ import annotations
 
 import ctypes
-import functools
 from collections.abc import Iterator
 from contextlib import contextmanager
 
@@ -51,13 +50,6 @@ def stack_b(lora_bs: list[torch.Tensor]) -> torch.Tensor:
     ``plm_gemm_packed_lora`` reads. A new tensor; callers that apply the same adapter repeatedly
     (``GatedLoraMethod``) stack once and pass it as ``lora_b``."""
     return torch.cat([b.contiguous() for b in lora_bs], dim=0).contiguous()
-
-
-@functools.lru_cache(maxsize=4096)
-def _lora_tile(M: int, N: int, K: int) -> Config:
-    from .fast_gemm import tile_supported
-
-    return tiles.k_split_tile(M, N, K, supported=lambda cfg: tile_supported(M, K, cfg))
 
 
 def _eligible(x, weight, lora_a, lora_bs, first_gated_row, bias, cfg) -> bool:
@@ -105,10 +97,7 @@ def gated_linear(x: torch.Tensor, weight: torch.Tensor, lora_a: torch.Tensor, lo
     if first_gated_row is None or first_gated_row >= M:
         return dispatch_unquantized_gemm()(None, x, weight, bias)
     first_gated_row = max(int(first_gated_row), 0)
-    if cfg is None:
-        cfg = CONFIGS.get((M, weight.shape[0], weight.shape[1]))
-        if cfg is not None and cfg["k_waves"] == 1:   # the linear's own tile runs on the wide kernel
-            cfg = _lora_tile(M, weight.shape[0], weight.shape[1])
+    cfg = cfg if cfg is not None else CONFIGS.get((M, weight.shape[0], weight.shape[1]))
     shards = len(lora_bs)
     rank = lora_a.shape[0] // shards
     if not _eligible(x, weight, lora_a, lora_bs, first_gated_row, bias, cfg):

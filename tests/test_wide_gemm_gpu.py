@@ -14,6 +14,7 @@ import torch.nn.functional as F
 from plm_amd import _lib, fast_gemm
 from plm_amd.chain import Link, LinearChain
 from plm_amd.fast_gemm import hip_linear, hip_linear_f32, pack_weight, release, released_linear
+from plm_amd.gated_lora import gated_linear
 from test_gemm_gpu import _inputs_on_gpu
 
 pytestmark = pytest.mark.gpu
@@ -93,6 +94,30 @@ def test_silu_mul_on_row_split_tiles(device, M, N, K, split):
     want = torch.empty(M, N // 2, device=device, dtype=x.dtype)
     LinearChain([Link(x, w, want, split_k=split, act=True)], dict(ROW_SPLIT, split_k=1)).run()
     assert torch.equal(fast_gemm.gate_up_silu(x, w, dict(ROW_SPLIT, split_k=split)), want)
+
+
+# Shards that end inside a 16-column fragment, ranks past one MFMA's 32 elements and below them, gates at the
+# first and last row, with and without K splits of the base linear (h: one range up to K = 1024, else four).
+@pytest.mark.parametrize("M,shards,K,rank,gate,split", [
+    (1, (24,), 64, 8, 0, 1), (56, (2048, 512, 512), 2048, 16, 7, 1), (42, (520, 136, 100), 1000, 40, 41, 2),
+    (110, (1000, 1048), 3072, 72, 10, 3), (65, (7, 8, 9), 1416, 32, 3, 1)])
+def test_gated_lora_on_row_split_tiles(device, M, shards, K, rank, gate, split):
+    g = torch.Generator(device=device).manual_seed(M + K)
+    N, cfg = sum(shards), dict(ROW_SPLIT, split_k=split)
+    x, w = _inputs_on_gpu(M, N, K, M + N, device)
+    a = (torch.randn(len(shards) * rank, K, generator=g, device=device) / K ** 0.5).bfloat16()
+    bs = [torch.randn(n, rank, generator=g, device=device).bfloat16() for n in shards]
+    got = [gated_linear(x, w, a, bs, gate, cfg=cfg) for _ in range(3)]
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+    base = hip_linear(x, w, cfg)
+    assert torch.equal(got[0][:gate], base[:gate])
+    h = x[gate:].double() @ a.double().t()
+    delta = torch.cat([h[:, i * rank:(i + 1) * rank] @ b.double().t() for i, b in enumerate(bs)], dim=1)
+    want = x[gate:].double() @ w.double().t() + delta
+    # Roundings to bf16: the base (2^-9 of it), h (2^-9 of each of its products with B), the sum.
+    hb = torch.cat([h[:, i * rank:(i + 1) * rank].abs() @ b.double().abs().t() for i, b in enumerate(bs)], dim=1)
+    bound = 2.0 ** -8 * ((want - delta).abs() + hb + want.abs()) + 1e-4
+    assert bool(((got[0][gate:].double() - want).abs() <= bound).all())
 
 
 def test_calls_that_need_more_than_a_product_go_to_f_linear(device):
