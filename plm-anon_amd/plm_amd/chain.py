@@ -92,7 +92,8 @@ class LinearChain:
         entry = lib.plm_gemm_chain_packed if self.packed else lib.plm_gemm_chain
         status = entry(_lib.DTYPE_CODES[self.dtype], self.host, self.table.data_ptr(), len(self.links), self.M,
                        self._tile, self.ws.data_ptr(), self.ws.numel(), _lib.stream_handle(self.device))
-        _lib.check(status, f"plm_gemm_chain({len(self.links)} linears, M={self.M}, cfg={self.cfg})")
+        if status:
+            _lib.check(status, f"plm_gemm_chain({len(self.links)} linears, M={self.M}, cfg={self.cfg})")
 
     @property
     def sync_mode(self) -> int:

@@ -129,7 +129,8 @@ def pack_weight(w: torch.Tensor) -> torch.Tensor:
     out = torch.empty(nbytes, dtype=torch.uint8, device=w.device)
     status = lib.plm_pack_weight(_lib.DTYPE_CODES[w.dtype], w.data_ptr(), w.stride(0), N, K, out.data_ptr(), nbytes,
                                  _lib.stream_handle(w.device))
-    _lib.check(status, f"plm_pack_weight(N={N}, K={K})")
+    if status:
+        _lib.check(status, f"plm_pack_weight(N={N}, K={K})")
     return out
 
 
@@ -182,7 +183,8 @@ def unpack_weight(p: torch.Tensor, N: int, K: int, dtype: torch.dtype) -> torch.
     out = torch.empty(N, K, dtype=dtype, device=p.device)
     status = _lib.lib().plm_unpack_weight(_lib.DTYPE_CODES[dtype], p.data_ptr(), p.numel(), N, K, out.data_ptr(), K,
                                           _lib.stream_handle(p.device))
-    _lib.check(status, f"plm_unpack_weight(N={N}, K={K})")
+    if status:
+        _lib.check(status, f"plm_unpack_weight(N={N}, K={K})")
     return out
 
 
@@ -259,8 +261,9 @@ def gate_up_silu(x: torch.Tensor, w: torch.Tensor, cfg: Config | None = None,
     N = w.shape[0]
     half = N // 2
     if M > 128:
-        if w in _released and N % 32 == 0:
-            act = _wide(x, w, _lib.PLM_OUT_SILU_MUL)
+        packed = _released.get(w) if N % 32 == 0 else None
+        if packed is not None:
+            act = _wide(x, w, packed, _lib.PLM_OUT_SILU_MUL)
             if act is not None:
                 return act if out is None else out.copy_(act)
         y = released_linear(x, w) if w in _released else F.linear(x, w)
@@ -288,7 +291,8 @@ def gate_up_silu(x: torch.Tensor, w: torch.Tensor, cfg: Config | None = None,
     status = lib.plm_gemm_packed_silu_mul(_lib.DTYPE_CODES[x.dtype], x.data_ptr(), x.stride(0),
                                           packed_gate_up(w).data_ptr(), out.data_ptr(), out.stride(0), M, N, K,
                                           tile, ws_ptr, ws_bytes, _lib.stream_handle(x.device))
-    _lib.check(status, f"plm_gemm_packed_silu_mul(M={M}, N={N}, K={K}, cfg={cfg})")
+    if status:
+        _lib.check(status, f"plm_gemm_packed_silu_mul(M={M}, N={N}, K={K}, cfg={cfg})")
     return out
 
 
@@ -355,7 +359,8 @@ def launch_packed(a: torch.Tensor, wp: torch.Tensor, N: int, cfg: Config, out: t
     entry = lib.plm_gemm_packed_f32out if f32_out else lib.plm_gemm_packed
     status = entry(_lib.DTYPE_CODES[a.dtype], a.data_ptr(), a.stride(0), wp.data_ptr(), out.data_ptr(), out.stride(0),
                    M, N, K, tile, ws_ptr, ws_bytes, _lib.stream_handle(a.device))
-    _lib.check(status, f"plm_gemm_packed(M={M}, N={N}, K={K}, cfg={cfg})")
+    if status:
+        _lib.check(status, f"plm_gemm_packed(M={M}, N={N}, K={K}, cfg={cfg})")
     return out
 
 
@@ -384,7 +389,8 @@ def hip_linear_rowmajor(a: torch.Tensor, w: torch.Tensor, cfg: Config, out: torc
     entry = lib.plm_gemm_f32out if f32_out else lib.plm_gemm
     status = entry(_lib.DTYPE_CODES[a.dtype], a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(),
                    out.stride(0), M, N, K, tile, ws_ptr, ws_bytes, _lib.stream_handle(a.device))
-    _lib.check(status, f"plm_gemm(M={M}, N={N}, K={K}, cfg={cfg})")
+    if status:
+        _lib.check(status, f"plm_gemm(M={M}, N={N}, K={K}, cfg={cfg})")
     return out
 
 
@@ -436,11 +442,11 @@ def _plain(x: torch.Tensor) -> bool:
             and torch.autograd.forward_ad.unpack_dual(x).tangent is None)
 
 
-def _wide(x: torch.Tensor, weight: torch.Tensor, out_kind: int) -> torch.Tensor | None:
-    """``x[M, K] @ weight^T`` of a released weight on the wide kernel (``out_kind`` as plm_gemm_wide's), or
-    None for a call that ``F.linear`` on the unpacked weight has to take. The two have the same sums in
-    the same order where F.linear's library does not split K; measured (M = 640, 1.3B block): 137 us with
-    F.linear, 97 us here."""
+def _wide(x: torch.Tensor, weight: torch.Tensor, packed: torch.Tensor, out_kind: int) -> torch.Tensor | None:
+    """``x[M, K] @ weight^T`` of a released weight, whose copy is ``packed``, on the wide kernel
+    (``out_kind`` as plm_gemm_wide's), or None for a call that ``F.linear`` on the unpacked weight has to
+    take. The two have the same sums in the same order where F.linear's library does not split K;
+    measured (M = 640, 1.3B block): 137 us with F.linear, 97 us here."""
     if not _plain(x) or x.device != weight.device:
         return None
     x = _row_major(x)
@@ -448,9 +454,10 @@ def _wide(x: torch.Tensor, weight: torch.Tensor, out_kind: int) -> torch.Tensor 
     if M * x.stride(0) * 2 >= 1 << 31:
         return None
     y = torch.empty(M, N // 2 if out_kind == _lib.PLM_OUT_SILU_MUL else N, device=x.device, dtype=x.dtype)
-    status = _lib.lib().plm_gemm_wide(_lib.DTYPE_CODES[x.dtype], x.data_ptr(), x.stride(0), _released[weight].data_ptr(),
+    status = _lib.lib().plm_gemm_wide(_lib.DTYPE_CODES[x.dtype], x.data_ptr(), x.stride(0), packed.data_ptr(),
                                       y.data_ptr(), y.stride(0), M, N, K, out_kind, _lib.stream_handle(x.device))
-    _lib.check(status, f"plm_gemm_wide(M={M}, N={N}, K={K}, out_kind={out_kind})")
+    if status:
+        _lib.check(status, f"plm_gemm_wide(M={M}, N={N}, K={K}, out_kind={out_kind})")
     return y
 
 
@@ -460,31 +467,42 @@ def released_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | 
     ``(M, N, K)``, else ``default_config``; a bias added after), wider on the wide kernel, or with a bias
     (one rounding for the sum) and in the cases ``_plain`` names as ``F.linear`` on the weight unpacked
     into a transient buffer."""
+    return _released_linear(x, weight, _released.get(weight), bias)
+
+
+def _released_linear(x: torch.Tensor, weight: torch.Tensor, packed: torch.Tensor | None,
+                     bias: torch.Tensor | None) -> torch.Tensor:
+    """``released_linear`` with the packed copy already looked up (a weak-key lookup costs 0.6 us)."""
     if x.dtype != weight.dtype:
         raise TypeError(f"released weight is {weight.dtype}, input is {x.dtype}")
     N, K = weight.shape
-    lead = x.shape[:-1]
-    x2 = x.reshape(-1, K)
+    flat = x.dim() == 2 and x.shape[1] == K
+    x2 = x if flat else x.reshape(-1, K)
     M = x2.shape[0]
     if M > WIDE_ROWS:
-        y = _wide(x2, weight, _lib.PLM_OUT_MODEL) if bias is None else None
-        return F.linear(x, unpacked(weight), bias) if y is None else y.reshape(*lead, N)
+        y = _wide(x2, weight, packed, _lib.PLM_OUT_MODEL) if bias is None and packed is not None else None
+        if y is None:
+            return F.linear(x, unpacked(weight), bias)
+        return y if flat else y.reshape(*x.shape[:-1], N)
     if M == 0:
         out = x2.new_empty(0, N)
     else:
-        cfg = CONFIGS.get((M, N, K)) or default_config(M, N, K)
-        out = hip_linear(x2, weight, cfg)
+        _check_operands(x2, weight)
+        out = x2.new_empty(M, N)
+        launch_packed(x2, packed_weight(weight) if packed is None else packed, N,
+                      CONFIGS.get((M, N, K)) or default_config(M, N, K), out)
     if bias is not None:
         out += bias
-    return out.reshape(*lead, N)
+    return out if flat else out.reshape(*x.shape[:-1], N)
 
 
 def fast_gemm(layer, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """vLLM ``default_unquantized_gemm`` signature; tuned 2-D half-precision calls without bias go to
     the HIP kernel, everything else to ``F.linear`` (plm/fast_gemm.py:106-111). A released weight
     has no row-major data: every call with it runs on its packed copy (``released_linear``)."""
-    if weight in _released:
-        return released_linear(x, weight, bias)
+    packed = _released.get(weight)
+    if packed is not None:
+        return _released_linear(x, weight, packed, bias)
     if bias is None and x.dim() == 2 and x.dtype in HALF_DTYPES:
         cfg = CONFIGS.get((x.shape[0], weight.shape[0], weight.shape[1]))
         if cfg is not None:

@@ -22,7 +22,7 @@ from contextlib import contextmanager
 import torch
 
 from . import _lib, tiles
-from .fast_gemm import CONFIGS, HALF_DTYPES, Config, dispatch_unquantized_gemm, packed_weight, workspace
+from .fast_gemm import CONFIGS, HALF_DTYPES, Config, _tile, dispatch_unquantized_gemm, packed_weight, workspace
 
 _rows_from: int | None = None
 
@@ -117,7 +117,7 @@ def gated_linear(x: torch.Tensor, weight: torch.Tensor, lora_a: torch.Tensor, lo
         lora_b = stack_b(lora_bs)
     elif lora_b.shape != (N, rank) or lora_b.stride() != (rank, 1) or lora_b.data_ptr() % 16:
         raise ValueError(f"lora_b must be the shards' B's stacked row-major as [{N}, {rank}]")
-    tile = _lib.Tile.from_config(cfg)
+    tile = _tile(cfg)
     lib = _lib.lib()
     g = first_gated_row
     ws = workspace(x.device, int(lib.plm_gemm_packed_lora_workspace_bytes(M, N, K, g, rank, shards, tile)))
@@ -126,7 +126,8 @@ def gated_linear(x: torch.Tensor, weight: torch.Tensor, lora_a: torch.Tensor, lo
                                       packed_weight(weight).data_ptr(), out.data_ptr(), out.stride(0), M, N, K, g,
                                       packed_weight(lora_a).data_ptr(), lora_b.data_ptr(), rank, shards, sizes, tile,
                                       ws.data_ptr(), ws.numel(), _lib.stream_handle(x.device))
-    _lib.check(status, f"plm_gemm_packed_lora(M={M}, N={N}, K={K}, rank={rank}, shards={shards})")
+    if status:
+        _lib.check(status, f"plm_gemm_packed_lora(M={M}, N={N}, K={K}, rank={rank}, shards={shards})")
     return out
 
 

@@ -14,7 +14,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .fast_gemm import HALF_DTYPES, Config, packed_weight, row_major_weight, workspace
+from .fast_gemm import HALF_DTYPES, Config, _tile, packed_weight, row_major_weight, workspace
 
 ROUND_MODES = {"fp32": _lib.PLM_ROUND_F32, "bf16": _lib.PLM_ROUND_BF16, "fp16": _lib.PLM_ROUND_F16}
 RULES = {"nucleus": _lib.PLM_RULE_NUCLEUS, "floor": _lib.PLM_RULE_FLOOR}
@@ -65,7 +65,7 @@ def lm_head_verify(x: torch.Tensor, w: torch.Tensor, pending: torch.Tensor, p: f
     if not (x.is_cuda and w.is_cuda):
         raise RuntimeError("lm_head_verify runs on the GPU only; got a CPU tensor")
     cfg = (VERIFY_CONFIG if packed else ROWMAJOR_VERIFY_CONFIG) if cfg is None else cfg
-    tile = _lib.Tile.from_config(cfg)
+    tile = _tile(cfg)
     x = x if (x.stride(1) == 1 and x.stride(0) % 8 == 0) else x.contiguous()
     if not packed:  # the packed path reads packed_weight(w), which handles any layout of w itself
         w = row_major_weight(w)
@@ -84,11 +84,13 @@ def lm_head_verify(x: torch.Tensor, w: torch.Tensor, pending: torch.Tensor, p: f
     if packed:
         status = lib.plm_lm_head_verify_packed(_lib.DTYPE_CODES[x.dtype], x.data_ptr(), x.stride(0),
                                                packed_weight(w).data_ptr(), R, V, K, *common)
-        _lib.check(status, f"plm_lm_head_verify_packed(R={R}, V={V}, K={K}, cfg={cfg})")
+        if status:
+            _lib.check(status, f"plm_lm_head_verify_packed(R={R}, V={V}, K={K}, cfg={cfg})")
     else:
         status = lib.plm_lm_head_verify(_lib.DTYPE_CODES[x.dtype], x.data_ptr(), x.stride(0), w.data_ptr(),
                                         w.stride(0), R, V, K, *common)
-        _lib.check(status, f"plm_lm_head_verify(R={R}, V={V}, K={K}, cfg={cfg})")
+        if status:
+            _lib.check(status, f"plm_lm_head_verify(R={R}, V={V}, K={K}, cfg={cfg})")
     if accept is not None and not direct:
         accept.copy_(accept_out)
         return accept, argmax
@@ -143,7 +145,8 @@ def round_epilogue(k: int, widened: torch.Tensor, hypotheses: torch.Tensor, veri
             *_state_args(k, verify, pending, anchor, out, base_t, offset_t, round_sequence, sequence_step, dev),
             _ptr(accepted, "accepted", k - 1, _U8, dev), _ptr(num_correct, "num_correct", 1, _I64, dev))
     status = _lib.lib().plm_round_epilogue(k, *args, _lib.stream_handle(dev))
-    _lib.check(status, f"plm_round_epilogue(k={k})")
+    if status:
+        _lib.check(status, f"plm_round_epilogue(k={k})")
 
 
 class RoundVerify:
@@ -199,7 +202,7 @@ class RoundVerify:
         dev = hidden.device
         x = hidden if (hidden.stride(1) == 1 and hidden.stride(0) % 8 == 0) else hidden.contiguous()
         V, K = w.shape
-        tile = _lib.Tile.from_config(VERIFY_CONFIG if self.cfg is None else self.cfg)
+        tile = _tile(VERIFY_CONFIG if self.cfg is None else self.cfg)
         lib = _lib.lib()
         ws = workspace(dev, int(lib.plm_lm_head_verify_workspace_bytes(W, V, K, tile)))
         status = lib.plm_round_verify_packed(
@@ -208,7 +211,8 @@ class RoundVerify:
             *_state_args(k, verify_tokens, pending, anchor, out, base_t, offset_t, round_sequence, sequence_step, dev),
             self.accept.data_ptr(), self.argmax.data_ptr(), _ptr(accepted, "accepted", k - 1, _U8, dev),
             _ptr(num_correct, "num_correct", 1, _I64, dev), tile, ws.data_ptr(), ws.numel(), _lib.stream_handle(dev))
-        _lib.check(status, f"plm_round_verify_packed(k={k}, V={V}, K={K})")
+        if status:
+            _lib.check(status, f"plm_round_verify_packed(k={k}, V={V}, K={K})")
 
 
 def lm_head_verify_logits(x: torch.Tensor, w: torch.Tensor, pending: torch.Tensor, pending_rows: int, p: float,
@@ -238,7 +242,7 @@ def lm_head_verify_logits(x: torch.Tensor, w: torch.Tensor, pending: torch.Tenso
     if not (x.is_cuda and w.is_cuda and logits.is_cuda):
         raise RuntimeError("lm_head_verify_logits runs on the GPU only; got a CPU tensor")
     cfg = VERIFY_CONFIG if cfg is None else cfg
-    tile = _lib.Tile.from_config(cfg)
+    tile = _tile(cfg)
     x = x if (x.stride(1) == 1 and x.stride(0) % 8 == 0) else x.contiguous()
     accept = torch.empty(R, dtype=torch.bool, device=x.device) if accept is None else accept
     argmax = torch.empty(R, dtype=torch.int64, device=x.device) if argmax is None else argmax
@@ -252,7 +256,8 @@ def lm_head_verify_logits(x: torch.Tensor, w: torch.Tensor, pending: torch.Tenso
         pending.data_ptr() if pending_rows > 0 else 0, pending_rows, RULES[rule], float(p), mode, accept.data_ptr(),
         argmax.data_ptr(), logits.data_ptr(), logits.stride(0), logit_rows, tile, ws.data_ptr(), ws.numel(),
         _lib.stream_handle(x.device))
-    _lib.check(status, f"plm_lm_head_verify_packed_logits(R={R}, V={V}, K={K}, logit_rows={logit_rows})")
+    if status:
+        _lib.check(status, f"plm_lm_head_verify_packed_logits(R={R}, V={V}, K={K}, logit_rows={logit_rows})")
     return accept, argmax
 
 
