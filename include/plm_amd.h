@@ -215,7 +215,9 @@ typedef struct plm_chain_gemm {
  * wave_frags, k_waves and unroll for every linear; each linear's split_k is its own. The launch
  * (one kernel; its last workgroup to finish advances the workspace's launch epoch) needs
  * every workgroup resident at once (the device to itself while it runs); a barrier that does not
- * complete in about a second sets the int at PLM_WORKSPACE_ERROR_INDEX to 1.
+ * complete in about a second sets the int at PLM_WORKSPACE_ERROR_INDEX to 1. With a row-split tile
+ * (k_waves 1) linears that read one another run one after the other on the stream instead, a launch
+ * each, with the same results and the same workspace; nothing then waits on another workgroup.
  * plm_gemm_chain_packed_prepare fills the derived fields and returns the workspace bytes.
  */
 int64_t plm_gemm_chain_packed_prepare(plm_chain_gemm* gemms, int32_t count, int64_t M, const plm_tile* tile);
@@ -229,7 +231,8 @@ int plm_gemm_chain_packed(int32_t dtype, const plm_chain_gemm* host_gemms, const
  * no device needed): 0 none reads another; 2 per-wavefront waits on the producer's tile-done flags
  * (every linear after the first reads the one before it and every Y that is read starts on a
  * 128-byte boundary with ldy a multiple of 64 elements); 1 a grid barrier after every linear that
- * is read (any other pattern). A negative status for an invalid chain or tile. */
+ * is read (any other pattern); with a row-split tile the launches' order takes the place of both, and
+ * the value only tells the pattern. A negative status for an invalid chain or tile. */
 int plm_gemm_chain_packed_sync_mode(const plm_chain_gemm* gemms, int32_t count, const plm_tile* tile);
 
 /*

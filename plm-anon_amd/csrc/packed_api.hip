@@ -512,6 +512,30 @@ int plm_gemm_chain_packed(int32_t dtype, const plm_chain_gemm* host_gemms, const
       if (ys[i].overlaps(ws[j])) return PLM_ERR_ARGUMENT;
       if (ys[i].overlaps(xs[j]) && host_gemms[j].dep != i) return PLM_ERR_ARGUMENT;
     }
+  if (sync && tile->k_waves == 1) {
+    // Linears that read one another on a row-split tile run one after the other on the current stream,
+    // each as its own launch would (mostly the wide kernel). A launch costs about what the chain's wait
+    // for tile flags does, and the wide kernel stages X once per workgroup, where the chained kernel's
+    // wavefronts each load their own X fragments. us per linear, captured, the best chained tile / here:
+    // GPT-style blocks of hidden 2048 at M = 28 9.3 / 9.8, M = 42 10.3 / 9.7, M = 56 10.5 / 10.2,
+    // M = 110 15.3 / 12.0; of hidden 2560 at M = 56 17.0 / 13.9; Llama-style of hidden 3072 at M = 42
+    // 16.8 / 13.9, M = 56 18.2 / 14.8, M = 110 27.5 / 17.9.
+    if (workspace == nullptr || static_cast<int64_t>(workspace_bytes) < need ||
+        (reinterpret_cast<uintptr_t>(workspace) & 15) != 0)
+      return PLM_ERR_WORKSPACE;
+    for (int32_t i = 0; i < count; ++i) {
+      const plm_chain_gemm& g = host_gemms[i];
+      plm_tile ti = *tile;
+      ti.split_k = g.split_k;
+      const int status =
+          g.out_f32 == PLM_OUT_SILU_MUL
+              ? plm_gemm_packed_silu_mul(dtype, g.x, g.ldx, g.w, g.y, g.ldy, M, g.N, g.K, &ti, workspace, workspace_bytes, stream)
+              : plm::packed_entry(dtype, g.x, g.ldx, g.w, g.y, g.ldy, M, g.N, g.K, &ti, workspace, workspace_bytes, stream,
+                                  g.out_f32);
+      if (status != PLM_OK) return status;
+    }
+    return PLM_OK;
+  }
   plm::PackedArgs a{};
   a.chain = device_gemms;
   a.single = host_gemms[0];

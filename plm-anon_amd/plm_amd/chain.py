@@ -7,7 +7,8 @@ of start-up and tail in which HBM idles; a chain keeps one persistent grid strea
 across the linears. With packed weights (the default) the workgroups meet at a grid barrier after
 each linear another one reads, with the next linear's first weights already requested; the
 streaming kernel on row-major weights (``packed=False``) starts each tile of a linear as soon as
-the producer tiles it reads are written.
+the producer tiles it reads are written. On a row-split tile (``k_waves`` 1, what rounds of more than 48
+rows run on) a chain of linears that read one another is a launch per linear, back to back on the stream.
 """
 
 from __future__ import annotations
@@ -98,7 +99,8 @@ class LinearChain:
     @property
     def sync_mode(self) -> int:
         """How the launch makes linears wait for the ones they read (packed chains): 0 none, 1 grid
-        barriers, 2 tile-done flags (``plm_gemm_chain_packed_sync_mode``)."""
+        barriers, 2 tile-done flags (``plm_gemm_chain_packed_sync_mode``). On a row-split tile the order
+        of the launches stands in for both."""
         if not self.packed:
             raise ValueError("sync_mode describes packed chains")
         mode = int(_lib.lib().plm_gemm_chain_packed_sync_mode(self.host, len(self.links), self._tile))

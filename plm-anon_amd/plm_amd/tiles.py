@@ -177,9 +177,11 @@ def packed_chain_split(N: int, K: int, cfg: dict, workgroups: int) -> int:
     is that of the busiest workgroup): the split with the least estimated busiest-workgroup time,
     counting each item's K steps per wavefront plus a fixed cost of a few steps for the item's end
     (reduction, stores; with split > 1 the partial round trip)."""
+    if cfg["k_waves"] == 1:   # linear by linear on the wide kernel; its splits hardly depend on the width
+        return row_split_splits(64, N, K)
     tiles_ = math.ceil(math.ceil(N / 16) / tile_frags(cfg))
     ks = math.ceil(K / 32)
-    kw = 1 if cfg["k_waves"] == 1 else cfg["k_waves"]
+    kw = cfg["k_waves"]
     best, best_cost = 1, None
     for split in SPLITS:
         if split > 1 and ks // split // kw < 2:
@@ -246,12 +248,17 @@ def chain_tile(M: int) -> dict:
 
 
 def packed_chain_tile(M: int) -> dict:
-    """Tile of a packed chained round at width M: 32-row tiles of eight wavefronts splitting K, one
-    workgroup per CU. At M > 48 (four X fragments) the two-stage pipeline has that residency; at
-    M <= 48 the two-stage kernel's smaller register count admits two workgroups per CU, which
-    measured slower (1167 against 1025 us for the 1.3B-shape round at M = 42), so the four-stage
-    pipeline is used."""
-    return {"wave_frags": 2, "k_waves": 8, "split_k": 1, "unroll": 2 if M > 48 else 4}
+    """Tile of a packed chained round at width M. At M <= 48, 32-row tiles of eight wavefronts
+    splitting K on a four-stage pipeline, one workgroup per CU (the two-stage kernel's smaller
+    register count admits two, which measured slower: 1167 against 1025 us for the 1.3B-shape round
+    at M = 42). Wider rounds take a row-split tile, whose linears run one after the other on the wide
+    kernel: the eight wavefronts each load every X fragment of their K range, seven of them at
+    M = 110, while the wide kernel stages X once per workgroup. Per linear, row-split against
+    eight-way: hidden 1024 6.4 / 6.9 us at M = 56 and 6.5 / 9.6 at 110 (but 6.4 / 5.6 at M = 30),
+    hidden 2048 10.2 / 10.5 and 12.0 / 15.3, hidden 2560 13.9 / 17.0 and 16.5 / 23.9."""
+    if M > 48:
+        return {"wave_frags": 2, "k_waves": 1, "split_k": 1, "unroll": 2}
+    return {"wave_frags": 2, "k_waves": 8, "split_k": 1, "unroll": 4}
 
 
 def chain_split(N: int, K: int, cfg: dict = CHAIN_TILE, workgroups: int = CU_COUNT) -> int:

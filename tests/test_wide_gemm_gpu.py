@@ -96,6 +96,34 @@ def test_silu_mul_on_row_split_tiles(device, M, N, K, split):
     assert torch.equal(fast_gemm.gate_up_silu(x, w, dict(ROW_SPLIT, split_k=split)), want)
 
 
+# One row, a tile's edge and past it, the widest; links that read the first columns of an earlier output, two
+# that read the same one, an activation link in between, an fp32 last link and one that reads none.
+@pytest.mark.parametrize("M", [1, 16, 49, 128])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_row_split_chains_equal_their_links_alone(device, M, dtype):
+    print(f"row split chain M={M} {dtype}", flush=True)
+    g = torch.Generator(device=device).manual_seed(M)
+    # (N, K, the link it reads, split, activation, fp32)
+    shapes = [(1003, 264, -1, 1, False, False), (704, 1000, 0, 3, True, False), (520, 352, 1, 1, False, False),
+              (136, 344, 1, 2, False, False), (777, 96, -1, 2, False, True), (2050, 520, 2, 1, False, True)]
+    outs = [torch.full((M, -(-n // 64) * 64), float("nan"), device=device, dtype=torch.float32 if f32 else dtype)
+            [:, :n // 2 if act else n] for n, _, _, _, act, f32 in shapes]
+    x = torch.randn(M, 264, generator=g, device=device).to(dtype)
+    links = []
+    for (n, k, dep, split, act, _), y in zip(shapes, outs):
+        w = (torch.randn(n, k, generator=g, device=device) / k ** 0.5).to(dtype)
+        links.append(Link(x[:, :k] if dep < 0 else outs[dep][:, :k], w, y, dep, split, act))
+    chain = LinearChain(links, ROW_SPLIT)
+    for _ in range(2):
+        x.copy_(torch.randn(M, 264, generator=g, device=device))
+        chain.run()
+        for i, ln in enumerate(links):
+            alone = torch.empty_like(ln.y)
+            LinearChain([Link(ln.x, ln.w, alone, split_k=ln.split_k, act=ln.act)], ROW_SPLIT).run()
+            assert torch.equal(ln.y, alone), i
+    chain.check()
+
+
 # Shards that end inside a 16-column fragment, ranks past one MFMA's 32 elements and below them, gates at the
 # first and last row, with and without K splits of the base linear (h: one range up to K = 1024, else four).
 @pytest.mark.parametrize("M,shards,K,rank,gate,split", [
