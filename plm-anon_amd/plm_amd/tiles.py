@@ -128,8 +128,10 @@ def row_split_splits(M: int, N: int, K: int) -> int:
     """K splits of a row-split tile on the wide kernel with the least modelled time (us): a CU's K steps at
     0.075 us or its loads' 82 KiB per us, whichever is longer, and for the partial sums' round trip 0.8 us,
     0.3 per split and 0.87 per MB. Measured at M = 56: 2048x2048 7.8 / 7.5 us with 1 / 2 splits,
-    6144x2048 9.6 / 11.1, 2048x8192 23.6 / 16.8 / 14.1 / 16.1 with 1 / 2 / 4 / 6."""
-    steps = math.ceil(K / 32)
+    6144x2048 9.6 / 11.1, 2048x8192 23.6 / 16.8 / 14.1 / 16.1 with 1 / 2 / 4 / 6. Fewer than 32 rows take
+    32 rows' splits: the join's latency does not fall with them as the modelled bytes do (6144x2048 at 2 to
+    30 rows 9.6 us with 1, 11.0 with 2; 7680x2560 11.1 with 1, 12.6 with 2, 13.9 with 4)."""
+    M, steps = max(M, 32), math.ceil(K / 32)
 
     def cost(split: int) -> float:
         work = min(math.ceil(math.ceil(N / (64 * nf)) * math.ceil(M / (16 * mt)) * split / CU_COUNT)
@@ -143,7 +145,15 @@ def row_split_splits(M: int, N: int, K: int) -> int:
 def heuristic_tile(M: int, N: int, K: int, supported=None) -> dict:
     """A reasonable tile without measurement: rows split across the wavefronts (the wide kernel's
     linears, with ``row_split_splits``'s K splits; the row-split kernel itself for weights past
-    ``WIDE_WEIGHT_BYTES`` at up to 64 rows), else ``k_split_tile``."""
+    ``WIDE_WEIGHT_BYTES`` at up to 64 rows), else ``k_split_tile``. Up to 16 rows a long K whose K-split
+    items fit the CUs one each keeps those: their join is a sum in LDS and fewer partials, or none.
+    Row-split against K-split, us at 2 to 16 rows: 1024x4096 8.6 / 7.7, 2048x8192 12.6 / 11.4, 2048x5632
+    10.5 / 9.6, 6144x2048 9.2 / 8.2, 8192x2048 9.8 / 9.4; but 2048x2048, which needs four splits, 7.2 / 7.5,
+    3072x1024 4.8 / 6.7 and 2560x10240, whose 320 items take two rounds, 15.4 / 18.1."""
+    if M <= 16 and K >= 2048 and _first_compiled(M, 2, (8, 4), supported):
+        cfg = k_split_tile(M, N, K, supported)
+        if items(N, cfg) <= CU_COUNT and (K >= 4096 or cfg["split_k"] == 1):
+            return cfg
     for nf in (2, 1, 4):
         cfg = _first_compiled(M, nf, (1,), supported)
         if cfg is None:
@@ -156,10 +166,9 @@ def heuristic_tile(M: int, N: int, K: int, supported=None) -> dict:
 
 
 def k_split_tile(M: int, N: int, K: int, supported=None) -> dict:
-    """A tile of the K-split layouts without measurement (what the gated-LoRA launch runs where the
-    linear's own tile is a row-split one): 32 rows per wavefront with a two-stage pipeline, K split across 8
-    wavefronts (4 where 8 is not compiled), and K splitting until about three quarters of the compute
-    units have an item, keeping at least two K steps per wavefront."""
+    """A tile of the K-split layouts without measurement: 32 rows per wavefront with a two-stage pipeline,
+    K split across 8 wavefronts (4 where 8 is not compiled), and K splitting until about three quarters
+    of the compute units have an item, keeping at least two K steps per wavefront."""
     for nf in (2, 4, 1):
         cfg = _first_compiled(M, nf, (8, 4), supported)
         if cfg is None:
