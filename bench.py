@@ -6,7 +6,8 @@ attention-out 2048->2048, MLP up 2048->8192, MLP down 8192->2048) plus the LM he
 (~N(0, 0.02^2)) resident in HBM. The round is recorded once as a HIP graph and replayed (the
 reference replays its round as a CUDA graph, plm/decoder.py:414-447), two ways, both over
 weights packed once into the MFMA fragment layout (as a served model keeps them):
-  * all 97 linears in one chained launch (plm_gemm_chain_packed), checked bit for bit against
+  * the block linears as a chain (plm_gemm_chain_packed; one persistent launch, or on a row-split
+    tile a launch of the wide kernel per linear) + the LM head, checked bit for bit against
   * the per-GEMM drop-in path: 97 fast_gemm launches (plm_gemm_packed, tuned tile per shape).
 
 Prints one JSON line: ``value`` is microseconds per round (lower is better) of the faster of the
@@ -138,12 +139,19 @@ def time_graph(graph, steps, warmup):
     return start.elapsed_time(end) / steps
 
 
-def kernel_class(M, K, cfg):
-    """The compiled kernel a GEMM launches: (MT, wave_frags, unroll, k_waves)."""
+def kernel_class(M, N, K, cfg):
+    """The compiled kernel a GEMM launches: (MT, wave_frags, unroll, k_waves), or the wide kernel, which
+    picks its tile itself, as (MT,)."""
+    from plm_amd.tiles import runs_wide
+
+    if cfg["k_waves"] == 1 and runs_wide(M, N, K):
+        return (math.ceil(M / 16),)
     return (math.ceil(M / 16), cfg["wave_frags"], cfg["unroll"], cfg["k_waves"])
 
 
 def kernel_name(cls):
+    if len(cls) == 1:
+        return f"wide_gemm_kernel<bf16> ({cls[0]} X fragments)"
     mt, nf, d, kw = cls
     return f"packed_gemm_kernel<bf16, MT={mt}, NF={nf}, D={d}, KW={kw}>"
 
@@ -152,7 +160,7 @@ def dominant_kernel_roofline(rnd, steps):
     """Per kernel class: graph of that class's launches only (in round order), HIP-event timed."""
     classes = {}
     for i, (g, cfg) in enumerate(zip(rnd.gemms, rnd.cfgs)):
-        classes.setdefault(kernel_class(rnd.M, g.K, cfg), []).append(i)
+        classes.setdefault(kernel_class(rnd.M, g.N, g.K, cfg), []).append(i)
     rows = []
     for cls, idx in classes.items():
         graph = rnd.capture(idx)
@@ -245,10 +253,11 @@ def capture_graph(fn):
 
 
 class ChainedRound:
-    """The round as two launches: its 96 block linears chained output-to-input in one persistent
-    launch over packed weights (plm_gemm_chain_packed, on the chain tile measured fastest for the
-    round's hidden size and width, each linear's K split chosen for the resident grid), then the LM head (read by no later linear) as its own launch with its tuned tile, which
-    streams a 206 MB weight faster than the chain's tile does."""
+    """The round's block linears chained output-to-input over packed weights (plm_gemm_chain_packed, on
+    the chain tile measured fastest for the round's hidden size and width, each linear's K split chosen
+    for it: one persistent launch, or a launch per linear on a row-split tile), then the LM head (read
+    by no later linear) as its own launch with its tuned tile, which streams a 206 MB weight faster
+    than the chain's tile does."""
 
     def __init__(self, rnd):
         from plm_amd import _lib, gemm_tables
@@ -266,6 +275,7 @@ class ChainedRound:
         self.chain = LinearChain(links, cfg, packed=True)
         self.head = (rnd.inputs[n], rnd.weights[n], rnd.cfgs[n], rnd.outs[n])
         self.chain_bytes = sum(g.bytes(rnd.M) for g in rnd.gemms[:n])
+        self.launches = (n if cfg["k_waves"] == 1 else 1) + 1
 
     def run(self):
         from plm_amd.fast_gemm import hip_linear
@@ -335,8 +345,8 @@ def main():
         print(f"[bench] eager chained round + per-GEMM round + verify x {max(1, args.steps)}", file=sys.stderr)
         return
 
-    # Headline: the round as the chained launch of its block linears + the LM-head launch, replayed
-    # as a HIP graph; the chained launch alone is timed too (its own roofline).
+    # Headline: the round as the chain of its block linears + the LM-head launch, replayed as a HIP
+    # graph; the chain alone is timed too (its own roofline).
     graph = capture_graph(chained.run)
     ms = time_graph(graph, args.steps, args.warmup)
     if chain.error_flag():
@@ -347,7 +357,7 @@ def main():
     graph = capture_graph(chain.run)
     us_chain = time_graph(graph, args.steps, args.warmup) * 1000.0
     del graph
-    # The chained launch computes what the single-linear kernel does with the same tiles, bit for
+    # The chain computes what the single-linear kernel does with the same tiles, bit for
     # bit, through all 96 block linears; the LM head is the per-GEMM path's own launch.
     for i, ln in enumerate(chain.links):
         hip_linear(ln.x, ln.w, dict(chain.cfg, split_k=ln.split_k), rnd.outs[i])
@@ -387,8 +397,8 @@ def main():
     us_value = us_round if chain_wins else us_graph
     gbps_value = rnd.bytes / (us_value * 1e-6) / 1e9
     n_lin = len(rnd.gemms)
-    timing = (f"HIP graph replay, HIP events; value = the round as one chained launch of its {n_lin - 1} block "
-              "linears over packed weights (plm_gemm_chain_packed) + the LM-head launch (plm_gemm_packed)"
+    timing = (f"HIP graph replay, HIP events; value = the round as one chain of its {n_lin - 1} block linears over "
+              f"packed weights (plm_gemm_chain_packed) + the LM head (plm_gemm_packed), {chained.launches} launches"
               if chain_wins else
               f"HIP graph replay, HIP events; value = the round as {n_lin} fast_gemm launches (plm_gemm_packed, "
               "tuned tile per shape) in one graph")
@@ -403,7 +413,7 @@ def main():
                    "vocab": GPT2_VOCAB, "gemm_launches": len(gemms), "bytes_per_round": rnd.bytes,
                    "timing": timing, "chain_tile": chain.cfg},
         "gbps": round(gbps_value, 1), "pct_of_hbm_peak": round(100.0 * gbps_value / HBM_PEAK_GBPS, 2),
-        "chained_round": {"us": round(us_round, 2), "gbps": round(gbps, 1), "launches": 2,
+        "chained_round": {"us": round(us_round, 2), "gbps": round(gbps, 1), "launches": chained.launches,
                           "chain_launch_us": round(us_chain, 2)},
         "per_gemm_graph": {"us": round(us_graph, 2), "gbps": round(rnd.bytes / (us_graph * 1e-6) / 1e9, 1),
                            "launches": len(gemms)},
@@ -417,15 +427,17 @@ def main():
         result["per_gemm_kernels"] = [{k: (round(v, 3) if isinstance(v, float) else v) for k, v in r.items()}
                                       for r in rows]
         if chain_wins:
-            # The chained launch is the round's dominant kernel: its HIP-event time per replay (a graph
-            # of that launch alone) is its duration.
-            kernel = "packed_gemm_kernel<bf16, MT=%d, NF=%d, D=%d, KW=%d> (chained block linears)" % (
-                math.ceil(args.M / 16), chain.cfg["wave_frags"], chain.cfg["unroll"], chain.cfg["k_waves"])
+            # The chain is the round's dominant work: its HIP-event time per replay (a graph of the chain
+            # alone) over its launches.
+            cls = kernel_class(args.M, rnd.gemms[0].N, rnd.gemms[0].K, chain.cfg)
+            kernel, parts = kernel_name(cls) + " (chained block linears)", chained.launches - 1
             achieved = chained.chain_bytes / (us_chain * 1e-6) / 1e9
             result["roofline"] = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBPS,
                                   "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBPS, 4),
-                                  "traffic": traffic_for("chain_round"), "kernel": kernel, "launches_per_round": 1,
-                                  "us_per_launch": round(us_chain, 2), "bytes_per_launch": chained.chain_bytes}
+                                  "traffic": traffic_for("chain_round" if parts == 1 else kernel_name(cls)),
+                                  "kernel": kernel, "launches_per_round": parts,
+                                  "us_per_launch": round(us_chain / parts, 3),
+                                  "bytes_per_launch": round(chained.chain_bytes / parts, 1)}
         else:
             # The kernel class with the most time in the round; its launches timed alone as a graph.
             top = rows[0]
@@ -657,11 +669,11 @@ def time_configs(args, device, rnd, chained, us_round, us_graph):
         cpu = layers * sum(per[:4]) + per[4]
     achieved = c4.chain_bytes / (us_c4_chain * 1e-6) / 1e9
     out["4_round_h2560"] = {
-        "chained": _line(us_c4, r4.bytes, cpu, launches=2, chain_matches_per_linear=bool(same)),
+        "chained": _line(us_c4, r4.bytes, cpu, launches=c4.launches, chain_matches_per_linear=bool(same)),
         "per_gemm": _line(us_g4, r4.bytes, cpu, launches=len(gemms)),
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
-                     "frac": round(achieved / HBM_PEAK_GBPS, 4), "kernel": "chained launch of the 128 block linears",
-                     "us_per_launch": round(us_c4_chain, 2), "bytes_per_launch": c4.chain_bytes},
+                     "frac": round(achieved / HBM_PEAK_GBPS, 4), "kernel": f"chain of the 128 block linears, {c4.launches - 1} launches",
+                     "us_per_chain": round(us_c4_chain, 2), "bytes_per_chain": c4.chain_bytes},
         "shape": f"{layers} GPT-style blocks of hidden {hidden} (QKV {3 * hidden}, MLP {mlp}) + LM head "
                  f"{hidden}->{GPT2_VOCAB}, M={rnd.M}",
         "cpu_note": "torch CPU F.linear: one block + LM head timed, round = 32 x block + LM head" if cpu else None}
@@ -701,7 +713,7 @@ def time_wide_round(args, device, rnd):
     graph = wide.capture()
     us_graph = time_graph(graph, max(5, args.steps // 2), 2) * 1000.0
     del graph
-    line = {"chained": _line(us_chain, wide.bytes, launches=2, chain_matches_per_linear=bool(same)),
+    line = {"chained": _line(us_chain, wide.bytes, launches=cw.launches, chain_matches_per_linear=bool(same)),
             "per_gemm": _line(us_graph, wide.bytes, launches=len(wide.gemms)),
             "shape": f"the headline round's {len(wide.gemms)} linears at M=110 (k=10)"}
     print(f"[bench] W=110 round: chained {us_chain:.1f} us, per-GEMM {us_graph:.1f} us", file=sys.stderr, flush=True)
@@ -765,7 +777,7 @@ def profile_lora(args, device):
 def profile_act(args, device):
     """The Llama-style 1.3B MLP (gate_up 2048 -> 2 x 5632, down 5632 -> 2048) at width M, eager,
     rotating over 8 weight sets (552 MB): the fused gate/up + SiLU-and-multiply launch, the gate/up
-    projection alone, and the MLP as one chained launch (gate/up with its activation, then down)."""
+    projection alone, and the MLP as one chain (gate/up with its activation, then down)."""
     import torch
 
     from plm_amd import _lib, gemm_tables
@@ -952,7 +964,7 @@ def time_gate_up_silu(args, device):
 def time_prefill(args, device, block_weights):
     """Prefill widths (M = 64 ... 640, plm/rounds.py:16; the reference hands them to F.linear) over
     the round's 96 block linears: the packed kernel on the packed copies (fast_gemm's path for a
-    released weight: the tuned tile or default_config, 128-row slices above 128 rows) against
+    released weight: the tuned tile or default_config, the wide kernel above 128 rows) against
     F.linear (hipBLASLt) on the row-major weights, each a graph of the 96 launches; per block."""
     import torch
     import torch.nn.functional as F
@@ -990,7 +1002,7 @@ def time_prefill(args, device, block_weights):
         print(f"[bench] prefill M={M}: {line}", file=sys.stderr, flush=True)
     return dict(out, note="96 block linears of the headline round per graph; packed = plm_gemm_packed "
                           "(its wide kernel above 128 rows), unpacked_f_linear = plm_unpack_weight into a "
-                          "transient buffer + F.linear (a released weight's path above 128 rows), f_linear = "
+                          "transient buffer + F.linear (a released weight's calls with a bias or a gradient), f_linear = "
                           "torch F.linear on a kept row-major weight")
 
 
@@ -1135,7 +1147,7 @@ def time_verify(w_lm, hidden, device, steps):
     from plm_amd.workloads import GPT2_VOCAB
 
     head_cfg = gemm_tables.read_table(hidden)[(56, GPT2_VOCAB, hidden)]
-    head = mfma_for(kernel_name(kernel_class(56, hidden, head_cfg))) or {}
+    head = mfma_for(kernel_name(kernel_class(56, GPT2_VOCAB, hidden, head_cfg))) or {}
     return {"us": round(ms * 1000.0, 2), "gbps": round(nbytes / (ms * 1e-3) / 1e9, 1),
             "pct_of_hbm_peak": round(100.0 * nbytes / (ms * 1e-3) / 1e9 / HBM_PEAK_GBPS, 2),
             "bytes": nbytes, "accepted": int(acc.sum().item()), "round_us": round(ms_round * 1000.0, 2),

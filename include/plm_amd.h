@@ -106,7 +106,7 @@ int plm_pack_weight(int32_t dtype, const void* w, int64_t ldw, int64_t N, int64_
  * ldw % 8 == 0) back from its packed copy, bit for bit. No counterpart in the reference, which
  * keeps only the row-major weight and hands the widths it does not tune (prefill chunks,
  * plm/rounds.py:16) to F.linear (plm/fast_gemm.py:108-111): a caller that keeps only the packed
- * copy unpacks a weight into a transient buffer for such a call.
+ * copy and needs the row-major one (a library product, a gradient) unpacks it into a transient buffer.
  */
 int plm_unpack_weight(int32_t dtype, const void* packed, size_t packed_bytes, int64_t N, int64_t K, void* w, int64_t ldw,
                       void* stream);
@@ -118,13 +118,13 @@ int plm_unpack_weight(int32_t dtype, const void* packed, size_t packed_bytes, in
  * wavefront (1, 2, 4); k_waves = 4: a workgroup tile is 16*wave_frags rows and its four
  * wavefronts split the tile's K range (summed in LDS in wavefront order), or k_waves = 1: a
  * workgroup tile is 64*wave_frags rows, each wavefront owns 16*wave_frags of them over the whole
- * K range, and the four share one copy of X through LDS; split_k = workgroups splitting K (1..64,
+ * K range, and the four share one copy of X through LDS (where M > 64 or the packed weight is under
+ * 128 MiB, such a call runs on the wide kernel, with the same sums in the same order); split_k = workgroups splitting K (1..64,
  * partials summed in split order); unroll = K steps of loads in flight per wavefront (2, 4, 6,
  * 8). Requirements as plm_gemm (K % 8 == 0, K <= 2^24, ldx % 8 == 0, x 16-byte aligned) except
  * that M may exceed 128: wider calls (prefill chunks, plm/rounds.py:16, which the reference hands to
- * F.linear) run on a compute-oriented wide kernel (128 x 128 tiles staged through LDS, K split in
- * fixed order for shapes with few tiles) whose tiling is its own: `tile` must be valid but is not
- * used. Workspace: plm_gemm_packed_workspace_bytes.
+ * F.linear) run on the wide kernel (X through LDS, weights straight to registers, no K split), whose
+ * tiling is its own: `tile` must be valid but is not used. Workspace: plm_gemm_packed_workspace_bytes.
  */
 int plm_gemm_packed(int32_t dtype, const void* x, int64_t ldx, const void* packed_w, void* y, int64_t ldy, int64_t M,
                     int64_t N, int64_t K, const plm_tile* tile, void* workspace, size_t workspace_bytes, void* stream);

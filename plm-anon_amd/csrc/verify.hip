@@ -55,8 +55,8 @@ struct VerifyArgs {
   int64_t ld_logits;
   int logit_rows;
   // The first own_groups workgroups compute the proposals' own logits (four rows each over packed
-  // weights, one over row-major ones) and count themselves into *own_done; the others wait for that count before their first
-  // fold (bounded; a wait that gives up sets *error).
+  // weights, one over row-major ones) and count themselves into *own_done; the others wait for that
+  // count before their first fold (bounded; a wait that gives up sets *error).
   int own_groups;
   int* own_done;
   int* error;
