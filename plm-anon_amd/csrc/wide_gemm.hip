@@ -466,8 +466,9 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
     }
     wide_wait_h(z);
     // Rows m >= gated_from: the base value rounded to the model dtype plus sum_j h[m, s rank + j] B[n, j],
-    // s the shard of column n, as MFMAs over 32 rank elements; a fragment's columns of other shards than
-    // the one at hand are zero rows of B.
+    // s the shard of column n, as MFMAs over 32 rank elements. A fragment that straddles shards forms the
+    // product with each shard's h by itself and takes a column's value from its own shard's (the other
+    // shards' columns are zero rows of B, but an overflowed h times zero is NaN).
     const auto hr = make_rsrc(z.h, static_cast<uint32_t>(a.M * z.width * 2));
     auto shard_of = [&](int n) { return (n >= z.shard_end[0]) + (n >= z.shard_end[1]) + (n >= z.shard_end[2]); };
 #pragma unroll
@@ -475,14 +476,13 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
       const int nf = __builtin_amdgcn_readfirstlane(16 * (of0 + f));
       const int s_lo = shard_of(nf), s_hi = shard_of(min(nf + 15, a.N - 1));
       const int s_own = shard_of(nf + (lane & 15));
-      f32x4 corr[MT];
+      auto product = [&](int s, f32x4 (&p)[MT]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int t = 0; t < MT; ++t) corr[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-      for (int j = 0; 32 * j < z.rank; ++j) {
-        const u32x4 row = j == 0 ? b_first[f] : load_b(f, j);
-        const int e = 32 * j + 8 * (lane >> 4);
-        for (int s = s_lo; s <= s_hi; ++s) {
+        for (int t = 0; t < MT; ++t) p[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; 32 * j < z.rank; ++j) {
+          const u32x4 row = j == 0 ? b_first[f] : load_b(f, j);
           const u32x4 bs = s_own == s ? row : u32x4{0u, 0u, 0u, 0u};
+          const int e = 32 * j + 8 * (lane >> 4);
           u32x4 hv[MT];
 #pragma unroll
           for (int t = 0; t < MT; ++t) {
@@ -491,8 +491,18 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
             hv[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(hr, static_cast<int>(off), 0, kCoherent));
           }
 #pragma unroll
-          for (int t = 0; t < MT; ++t) corr[t] = mfma_16x16x32<DT>(bs, hv[t], corr[t]);
+          for (int t = 0; t < MT; ++t) p[t] = mfma_16x16x32<DT>(bs, hv[t], p[t]);
         }
+      };
+      f32x4 corr[MT];
+      product(s_lo, corr);
+      for (int s = s_lo + 1; s <= s_hi; ++s) {
+        f32x4 part[MT];
+        product(s, part);
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) corr[t][r] = shard_of(nf + 4 * (lane >> 4) + r) == s ? part[t][r] : corr[t][r];
       }
 #pragma unroll
       for (int t = 0; t < MT; ++t) {

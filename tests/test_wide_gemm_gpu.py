@@ -148,6 +148,27 @@ def test_gated_lora_on_row_split_tiles(device, M, shards, K, rank, gate, split):
     assert bool(((got[0][gate:].double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("M,shards,K,rank,split", [
+    (7, (24, 30, 42), 64, 8, 1), (56, (520, 136, 100), 1000, 40, 2), (110, (5640, 5624), 256, 72, 1)])
+@pytest.mark.parametrize("over", [0, 1])
+def test_gated_lora_overflow_stays_in_its_shard(device, M, shards, K, rank, split, over):
+    """One shard's h past fp16's largest value: the other shards' columns, those of the fragments it shares
+    with them included, equal the run without the overflow."""
+    g = torch.Generator(device=device).manual_seed(M)
+    cfg = dict(ROW_SPLIT, split_k=split)
+    x = torch.rand(M, K, generator=g, device=device).half()
+    w = (torch.randn(sum(shards), K, generator=g, device=device) / K ** 0.5).half()
+    a = (torch.randn(len(shards) * rank, K, generator=g, device=device) / K ** 0.5).half()
+    bs = [torch.randn(n, rank, generator=g, device=device).half() for n in shards]
+    want = gated_linear(x, w, a, bs, 3, cfg=cfg)
+    a[over * rank:(over + 1) * rank] = 60000.0
+    got = gated_linear(x, w, a, bs, 3, cfg=cfg)
+    lo = sum(shards[:over])
+    hi = lo + shards[over]
+    assert torch.equal(got[:, :lo], want[:, :lo]) and torch.equal(got[:, hi:], want[:, hi:])
+    assert torch.equal(got[:3], want[:3]) and not bool(got[3:, lo:hi].isfinite().any())
+
+
 def test_calls_that_need_more_than_a_product_go_to_f_linear(device):
     """A bias, autograd, autocast and vmap of a released weight's wide calls act as F.linear's own."""
     x, w = _inputs_on_gpu(130, 256, 64, 9, device)
