@@ -87,8 +87,9 @@ __device__ __forceinline__ bool accept_proposal(const VerifyArgs& a, float own, 
 // for terms far below the row's largest.
 __device__ __forceinline__ float exp_below_max(float d) { return __builtin_amdgcn_exp2f(d * 1.4426950408889634f); }
 
-// An empty state (maximum -inf) leaves the other unchanged; selects rather than branches, as the
-// lanes of a wavefront merge states of different rows.
+// A state whose maximum is -inf adds nothing to the other's sums (its own may be NaN, -inf less -inf), and
+// its index counts only where the other's maximum is -inf too; selects rather than branches, as the lanes
+// of a wavefront merge states of different rows.
 #pragma clang fp contract(off)
 __device__ __forceinline__ RowState merge(RowState a, RowState b) {
   RowState r;
@@ -285,9 +286,11 @@ __device__ __forceinline__ float round_logit(float v) {
 }
 
 // Branch-free: a lane visits its columns in increasing order, so a strict comparison keeps the
-// lowest index among its equal maxima (NaN never wins). With CHECK (a wavefront whose columns run
-// past V: the last tile) columns past V read as -inf, which neither wins nor adds: e^(-inf - mx) = 0
-// once the row maximum is finite, and a row whose maximum is -inf is not merged.
+// lowest index among its equal maxima (NaN never wins), starting from its first column, so that a row of
+// -inf logits (16-bit roundings of large negative ones) has the index of the first. With CHECK (a wavefront
+// whose columns run past V: the last tile) columns past V read as -inf, which neither wins nor adds:
+// e^(-inf - mx) = 0 once the row maximum is finite, and merge() takes only the index of a tile whose
+// maximum is -inf; a lane with no column in range keeps INT_MAX.
 template <int MT, int NF, int MODE, bool CHECK>
 __device__ __forceinline__ void fold_columns(const f32x4 (&acc)[NF][MT], int n0, int V, const float (&own_l)[MT],
                                              RowState (&rs)[MT]) {
@@ -295,7 +298,7 @@ __device__ __forceinline__ void fold_columns(const f32x4 (&acc)[NF][MT], int n0,
   for (int t = 0; t < MT; ++t) {
     float lv[NF][4];
     float mx = -INFINITY;
-    int ai = INT_MAX;
+    int ai = CHECK && n0 >= V ? INT_MAX : n0;
 #pragma unroll
     for (int f = 0; f < NF; ++f)
 #pragma unroll
@@ -331,7 +334,7 @@ __device__ __forceinline__ void fold_columns(const f32x4 (&acc)[NF][MT], int n0,
       e += __shfl_xor(e, off, 64);
       ab += __shfl_xor(ab, off, 64);
     }
-    if (mx != -INFINITY) rs[t] = merge(rs[t], RowState{mx, e, ab, ai});
+    rs[t] = merge(rs[t], RowState{mx, e, ab, ai});
   }
 }
 

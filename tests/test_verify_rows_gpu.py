@@ -8,6 +8,9 @@ from __future__ import annotations
 import pytest
 import torch
 
+import oracle
+from plm_amd.fast_gemm import hip_linear_f32
+from plm_amd.verify import LOGITS_CONFIG, ROWMAJOR_LOGITS_CONFIG, lm_head_verify
 from test_verify_gpu import run_case
 
 pytestmark = pytest.mark.gpu
@@ -26,3 +29,21 @@ def test_quarters_and_tiles(device, R, V, K, dtype):
     for m in ("fp32", mode):
         for _ in range(2):   # the second launch finds the first one's counters
             run_case(x, w, pending, 0.7, m, device, check_cpu=False, packed=False)
+
+
+@pytest.mark.parametrize("packed", [True, False], ids=["packed", "rowmajor"])
+@pytest.mark.parametrize("R,V,K", [(3, 1, 8), (5, 129, 64), (16, 5003, 64), (42, 300, 2048), (64, 20000, 64)])
+def test_rows_of_minus_infinity_name_their_first_id(device, R, V, K, packed):
+    """Logits that round to -inf in fp16: a row of nothing else has argmax 0, a row with a finite logit
+    in a later tile that one's id."""
+    x = torch.zeros(R, K, device=device).half()
+    w = torch.full((V, K), -300.0, device=device).half()
+    w[V // 2, 1] = 1.0
+    x[0] = 300.0
+    x[1, 0] = 300.0
+    x[2, 1] = 300.0
+    pending = torch.zeros(R, dtype=torch.int64, device=device)
+    argmax = lm_head_verify(x, w, pending, 0.7, "fp16", packed=packed)[1]
+    logits = hip_linear_f32(x, w, LOGITS_CONFIG if packed else ROWMAJOR_LOGITS_CONFIG).half()
+    assert int(logits[:3].isfinite().sum()) == 1 and bool(logits[2, V // 2].isfinite())
+    assert torch.equal(argmax.cpu(), oracle.argmax(logits.float().cpu()))
