@@ -442,6 +442,12 @@ def _plain(x: torch.Tensor) -> bool:
             and torch.autograd.forward_ad.unpack_dual(x).tangent is None)
 
 
+def _wide_takes(M: int, ldx: int, packed_bytes: int) -> bool:
+    """Whether ``plm_gemm_wide`` takes these sizes: it reads X and the packed weight through 32-bit offsets
+    and takes up to 2^24 rows (``wide_rows`` in csrc/packed_api.hip; K is bounded by the weight's bytes)."""
+    return M <= 1 << 24 and 2 * M * ldx < 1 << 31 and packed_bytes < 1 << 31
+
+
 def _wide(x: torch.Tensor, weight: torch.Tensor, packed: torch.Tensor, out_kind: int) -> torch.Tensor | None:
     """``x[M, K] @ weight^T`` of a released weight, whose copy is ``packed``, on the wide kernel
     (``out_kind`` as plm_gemm_wide's), or None for a call that ``F.linear`` on the unpacked weight has to
@@ -451,7 +457,7 @@ def _wide(x: torch.Tensor, weight: torch.Tensor, packed: torch.Tensor, out_kind:
         return None
     x = _row_major(x)
     (M, K), N = x.shape, weight.shape[0]
-    if M * x.stride(0) * 2 >= 1 << 31:
+    if not _wide_takes(M, x.stride(0), packed.numel()):
         return None
     y = torch.empty(M, N // 2 if out_kind == _lib.PLM_OUT_SILU_MUL else N, device=x.device, dtype=x.dtype)
     status = _lib.lib().plm_gemm_wide(_lib.DTYPE_CODES[x.dtype], x.data_ptr(), x.stride(0), packed.data_ptr(),

@@ -86,6 +86,22 @@ def test_argument_validation_happens_before_launch():
                                              fake, 1 << 30, None) == -3
 
 
+@pytest.mark.parametrize("M,N,K", [(129, 262144, 4096), (129, 152064, 8192), (640, 64, (1 << 24) + 8),
+                                   ((1 << 24) + 1, 64, 8), (1 << 17, 64, 8192)])
+def test_released_calls_past_the_wide_kernels_limits_go_to_f_linear(M, N, K):
+    """Sizes plm_gemm_wide refuses (a packed weight or X of 2 GiB, M or K past 2^24) are not sent to it;
+    one row, row block or K step less is."""
+    lib = _lib.lib()
+    fake = 1 << 20
+    nbytes = int(lib.plm_packed_weight_bytes(N, K))
+    assert lib.plm_gemm_wide(0, fake, K, fake, fake, N, M, N, K, 0, None) == -1
+    assert not fast_gemm._wide_takes(M, K, nbytes)
+    if M > 640:
+        assert fast_gemm._wide_takes(M - 1, K, nbytes)
+    elif N > 64:
+        assert fast_gemm._wide_takes(M, K, int(lib.plm_packed_weight_bytes(N // 2, K)))
+
+
 def test_epilogue_argument_validation_happens_before_launch():
     lib = _lib.lib()
     fake = 1 << 20
