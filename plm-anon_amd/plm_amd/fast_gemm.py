@@ -457,7 +457,7 @@ def _wide(x: torch.Tensor, weight: torch.Tensor, packed: torch.Tensor, out_kind:
         return None
     x = _row_major(x)
     (M, K), N = x.shape, weight.shape[0]
-    if not _wide_takes(M, x.stride(0), packed.numel()):
+    if x.data_ptr() % 16 or not _wide_takes(M, x.stride(0), packed.numel()):
         return None
     y = torch.empty(M, N // 2 if out_kind == _lib.PLM_OUT_SILU_MUL else N, device=x.device, dtype=x.dtype)
     status = _lib.lib().plm_gemm_wide(_lib.DTYPE_CODES[x.dtype], x.data_ptr(), x.stride(0), packed.data_ptr(),

@@ -187,3 +187,15 @@ def test_calls_that_need_more_than_a_product_go_to_f_linear(device):
     assert torch.func.vmap(lambda t: released_linear(t, w))(stack).shape == (2, 130, 256)
     with torch.no_grad():
         assert torch.equal(released_linear(leaf, w), F.linear(x, ref_w))
+
+
+def test_rows_off_16_bytes_go_to_f_linear(device):
+    """A contiguous X that starts off a 16-byte boundary, which no 16-byte load reads."""
+    _, w = _inputs_on_gpu(130, 256, 64, 11, device)
+    ref_w = w.clone()
+    release(w)
+    x = torch.randn(130 * 64 + 8, device=device).bfloat16()[1:130 * 64 + 1].view(130, 64)
+    assert x.is_contiguous() and x.data_ptr() % 16
+    y = F.linear(x, ref_w)
+    assert torch.equal(released_linear(x, w), y)
+    assert torch.equal(fast_gemm.gate_up_silu(x, w), F.silu(y[:, :128]) * y[:, 128:])
