@@ -14,7 +14,7 @@ config go to ``F.linear``, exactly as in the reference.
 it runs from the packed copy: widths up to 128 rows (the round widths) on the packed kernel with
 their tuned tiles or ``default_config``'s; wider calls (prefill chunks, plm/rounds.py:16, which the
 reference hands to ``F.linear``) on the wide kernel (``plm_gemm_wide``), or, where the call needs more
-than a product (a bias, autograd, autocast, tracing), as ``F.linear`` on the weight unpacked into a
+than a product (a bias, autograd, autocast, tracing) or the library is faster (``_wide_pays``), as ``F.linear`` on the weight unpacked into a
 transient buffer (``unpacked``, bit for bit).
 """
 
@@ -448,6 +448,24 @@ def _wide_takes(M: int, ldx: int, packed_bytes: int) -> bool:
     return M <= 1 << 24 and 2 * M * ldx < 1 << 31 and packed_bytes < 1 << 31
 
 
+def _wide_pays(M: int, N: int, K: int, act: bool) -> bool:
+    """Whether a released weight's call above ``WIDE_ROWS`` rows is left to the wide kernel, or is ``F.linear``
+    on the unpacked weight (for ``act`` with the activation as launches of its own). Measured, us, unpack and
+    F.linear / wide kernel:
+
+    * up to 1536 rows the wide kernel (6144x2048: 640 rows 34 / 22, 1536 50 / 43; the closest, 8192x8192 at
+      1536, 200 / 195), since unpacking costs as much as the product. Above, the library's larger tiles
+      overtake it, wide weights first: 2048 rows 2048x2048 29 / 20, 6144x2048 57 / 50, but 8192x2048 68 / 70,
+      8192x8192 225 / 244; 4096 rows 8192x2048 117 / 150, 3072x8192 177 / 233. The activation's two launches
+      move that to 2048 rows (8192x8192 256 / 228; at 4096 447 / 510).
+    * not a few columns over a very long K, whose every output is one chain of K / 32 steps here and split
+      in the library: 128x8192 at 192 rows 14.7 / 15.8, 256x14336 22.3 / 25.1, but 256x8192 16.9 / 15.6,
+      384x14336 25.7 / 25.6."""
+    if K > 7168 and 48 * N <= K:
+        return False
+    return M <= 1536 or M <= 2048 and (act or N < 8192)
+
+
 def _wide(x: torch.Tensor, weight: torch.Tensor, packed: torch.Tensor, out_kind: int) -> torch.Tensor | None:
     """``x[M, K] @ weight^T`` of a released weight, whose copy is ``packed``, on the wide kernel
     (``out_kind`` as plm_gemm_wide's), or None for a call that ``F.linear`` on the unpacked weight has to
@@ -458,6 +476,8 @@ def _wide(x: torch.Tensor, weight: torch.Tensor, packed: torch.Tensor, out_kind:
     x = _row_major(x)
     (M, K), N = x.shape, weight.shape[0]
     if x.data_ptr() % 16 or not _wide_takes(M, x.stride(0), packed.numel()):
+        return None
+    if not _wide_pays(M, N, K, out_kind == _lib.PLM_OUT_SILU_MUL):
         return None
     y = torch.empty(M, N // 2 if out_kind == _lib.PLM_OUT_SILU_MUL else N, device=x.device, dtype=x.dtype)
     status = _lib.lib().plm_gemm_wide(_lib.DTYPE_CODES[x.dtype], x.data_ptr(), x.stride(0), packed.data_ptr(),
@@ -471,7 +491,7 @@ def released_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | 
     """``F.linear(x, weight, bias)`` for a released weight, any leading shape of ``x``: up to
     ``WIDE_ROWS`` rows on the packed kernel (the tuned tile where the tables have one for
     ``(M, N, K)``, else ``default_config``; a bias added after), wider on the wide kernel, or with a bias
-    (one rounding for the sum) and in the cases ``_plain`` names as ``F.linear`` on the weight unpacked
+    (one rounding for the sum) and in the cases ``_plain`` and ``_wide_pays`` name as ``F.linear`` on the weight unpacked
     into a transient buffer."""
     return _released_linear(x, weight, _released.get(weight), bias)
 

@@ -102,6 +102,15 @@ def test_released_calls_past_the_wide_kernels_limits_go_to_f_linear(M, N, K):
         assert fast_gemm._wide_takes(M, K, int(lib.plm_packed_weight_bytes(N // 2, K)))
 
 
+def test_released_calls_the_library_is_faster_at_go_to_f_linear():
+    """Shapes (M, N, K) on both sides of each line of ``_wide_pays``, as timed."""
+    wide = [(129, 64, 64), (640, 8192, 2048), (1536, 50304, 2048), (2048, 6144, 2048), (192, 256, 8192), (192, 384, 14336)]
+    library = [(1537, 8192, 2048), (2049, 2048, 2048), (8192, 768, 512), (192, 128, 8192), (192, 256, 14336)]
+    assert all(fast_gemm._wide_pays(*shape, False) for shape in wide)
+    assert not any(fast_gemm._wide_pays(*shape, False) for shape in library)
+    assert fast_gemm._wide_pays(2048, 16384, 3072, True) and not fast_gemm._wide_pays(2049, 16384, 3072, True)
+
+
 def test_epilogue_argument_validation_happens_before_launch():
     lib = _lib.lib()
     fake = 1 << 20

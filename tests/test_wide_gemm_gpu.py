@@ -199,3 +199,17 @@ def test_rows_off_16_bytes_go_to_f_linear(device):
     y = F.linear(x, ref_w)
     assert torch.equal(released_linear(x, w), y)
     assert torch.equal(fast_gemm.gate_up_silu(x, w), F.silu(y[:, :128]) * y[:, 128:])
+
+
+@pytest.mark.parametrize("M,N,K", [(2049, 64, 64), (1600, 8192, 64), (130, 64, 7176)])
+def test_calls_the_library_is_faster_at(device, M, N, K):
+    """Past the wide kernel's range the released calls are F.linear's, with the activation torch's."""
+    x, w = _inputs_on_gpu(M, N, K, M + K, device)
+    y = F.linear(x, w)
+    release(w)
+    assert torch.equal(released_linear(x, w), y)
+    got, want = fast_gemm.gate_up_silu(x, w), F.silu(y[:, :N // 2]) * y[:, N // 2:]
+    if M == 1600:   # the activation's own line is 2048 rows: the wide kernel, one step of each rounding
+        torch.testing.assert_close(got.float(), want.float(), rtol=2 * 2.0 ** -7, atol=1e-30)
+    else:
+        assert torch.equal(got, want)
