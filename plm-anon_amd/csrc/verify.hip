@@ -12,7 +12,8 @@
 // The floor rule (plm/decoder.py:78-82), accept = l_own - logsumexp(l) > log(eps), reads the same
 // row state: logsumexp(l) = mx + log(sum_j e_j).
 //
-// One launch, over packed weights (verify_packed_main_kernel) or row-major ones (verify_rows_kernel):
+// One launch, over packed weights (verify_packed_main_kernel) or row-major ones (verify_rows_kernel; at few
+// rows few_rows_kernel, two launches and one merge):
 // the first workgroups recompute each row's proposal logit l[r, pending[r]] with the main pass's K
 // partition and order, so that the value is bit-identical to the one the main pass forms for that column;
 // the others stream tiles of W, fold the logits into running per-row states (maximum, argmax, sum of
@@ -50,6 +51,8 @@ struct VerifyArgs {
   // and one coherent load each per merge: rec[G][R], and grec[groups][R] the merged state of each group.
   f32x4* rec;
   f32x4* grec;
+  float* state;    // row-major weights, few rows: [G][R][3], row max, sum of exp, sum of exp above own
+  int* state_idx;  // and [G][R], argmax
   RoundEpilogue round;  // packed verify: k > 0 runs the round's epilogue after the last merge
   uint16_t* logits;     // packed verify: rows [0, logit_rows) of the logits in the model dtype, or null
   int64_t ld_logits;
@@ -853,12 +856,195 @@ hipError_t verify_rows_pick(const VerifyArgs& a, int cu, hipStream_t s) {
   return a.V <= 64 * cu ? launch_verify_rows<DT, MT, 1>(a, cu, s) : launch_verify_rows<DT, MT, 2>(a, cu, s);
 }
 
-// A tile is checked as it always was; the kernel has its own.
+// ---------------------------------------------------------------------------------------------
+// Row-major weights at few rows: the same logits (wavefront q's MFMA chains over quarter q of the K steps,
+// summed in order), but every wavefront loads its operands straight from the rows of W and X, its quarter
+// only, and the four accumulators meet in LDS. Its loads waste most of each cache line, which caps it at
+// 0.8 TB/s over a large W; but a tile is 32 vocabulary rows by a quarter of K per wavefront, where
+// verify_rows_kernel's wavefronts each walk all of K, and with few rows that chain is the launch's time.
+// Two launches: the proposals' logits, then the tiles. us, this kernel / verify_rows_kernel:
+//   K = 512:  R = 1 V = 2000 12.3 / 14.5, R = 4 V = 4000 14.1 / 15.1, R = 6 V = 4000 16.3 / 14.9
+//   K = 2048: R = 1 V = 2000 16.5 / 22.2, R = 8 V = 2000 21.6 / 23.2, R = 4 V = 8000 22.7 / 24.1,
+//             R = 8 V = 8000 27.4 / 24.0, R = 1 V = 16500 31.7 / 28.4
+//   K = 4096: R = 1 V = 2000 24.6 / 34.6, R = 12 V = 4000 34.4 / 34.7, R = 16 V = 8000 44.2 / 35.2,
+//             R = 1 V = 12000 40.1 / 36.6, but R = 1 V = 32000 71.0 / 77.5
+constexpr int kFewNF = 2, kFewU = 4;  // weight fragments, and K steps per batch of loads, of a wavefront
+
+// Where it is the faster one: few rows against K over a vocabulary of up to 8192 (a line through the
+// figures above), and one or two rows over the largest weights.
+inline bool few_rows_faster(int64_t R, int64_t V, int64_t K) {
+  if (R <= 2 && V * K >= 125000000) return true;
+  return R <= 16 && V <= 8192 && 1500 * R + V <= 8250 + 7 * K / 2;
+}
+
+__device__ __forceinline__ RowState wave_merge(RowState s) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1)
+    s = merge(s, RowState{__shfl_xor(s.mx, off, 64), __shfl_xor(s.se, off, 64), __shfl_xor(s.ab, off, 64),
+                          __shfl_xor(s.ai, off, 64)});
+  return s;
+}
+
+// One workgroup per proposal.
+template <int DT, bool PIPE>
+__global__ __launch_bounds__(64 * kPackedWaves) void few_own_kernel(VerifyArgs a) {
+  __shared__ float red[kPackedWaves * kFewNF * 256];
+  constexpr int TN = 16 * kFewNF;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = blockIdx.x;
+  const int64_t pid64 = r < a.pending_rows ? a.pending[r] : -1;
+  if (pid64 < 0 || pid64 >= a.V) {  // not a vocabulary id: no logit, and the row accepts nothing
+    if (threadIdx.x == 0) a.own[r] = NAN;
+    return;
+  }
+  const int pid = static_cast<int>(pid64);
+  const int n0 = (pid / TN) * TN;
+  const int tn = min(TN, a.V - n0);
+  const auto xr = make_rsrc(a.x, static_cast<uint32_t>(a.R * a.ldx * 2));
+  const auto wr = make_rsrc(a.w + static_cast<int64_t>(n0) * a.ldw, static_cast<uint32_t>(tn * a.ldw * 2));
+  uint32_t xoff[1], woff[kFewNF];
+  row_offsets<1>(a.ldx, r, r + 1, lane, xoff);
+  row_offsets<kFewNF>(a.ldw, pid - n0, pid - n0 + 1, lane, woff);
+  int st0, st1;
+  k_slice(a.K, wave, kPackedWaves, st0, st1);
+  f32x4 acc[kFewNF][1];
+#pragma unroll
+  for (int f = 0; f < kFewNF; ++f) acc[f][0] = f32x4{0.f, 0.f, 0.f, 0.f};
+  wave_mma<DT, 1, kFewNF, kFewU, PIPE>(xr, xoff, wr, woff, a.K, st0, st1, lane, acc);
+  wave_spill<1, kFewNF>(red, wave, lane, acc);
+  __syncthreads();
+  if (threadIdx.x == 0)
+    a.own[r] = round_through(wg_sum<1, kFewNF>(red, kPackedWaves, red_offset<1, kFewNF>(pid - n0, r)), a.round_mode);
+}
+
+// G workgroups over the tiles; wavefront w folds rows w, w + 4, ... and the last workgroup merges the states.
+template <int DT, bool PIPE>
+__global__ __launch_bounds__(64 * kPackedWaves) void few_rows_kernel(VerifyArgs a) {
+  __shared__ float red[kPackedWaves * kFewNF * 256];
+  constexpr int TN = 16 * kFewNF, RPW = 16 / kPackedWaves;
+  static_assert(TN <= 64, "one lane per tile column");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n_tiles = (a.V + TN - 1) / TN;
+
+  const auto xr = make_rsrc(a.x, static_cast<uint32_t>(a.R * a.ldx * 2));
+  uint32_t xoff[1];
+  row_offsets<1>(a.ldx, 0, a.R, lane, xoff);
+  int st0, st1;
+  k_slice(a.K, wave, kPackedWaves, st0, st1);
+
+  RowState rs[RPW];
+  float own_l[RPW];
+#pragma unroll
+  for (int j = 0; j < RPW; ++j) {
+    rs[j] = empty_state();
+    const int m = wave + kPackedWaves * j;
+    own_l[j] = m < a.R ? a.own[m] : 0.f;
+  }
+
+  for (int tile = blockIdx.x; tile < n_tiles; tile += a.G) {
+    const int n0 = tile * TN;
+    const int tn = min(TN, a.V - n0);
+    const auto wr = make_rsrc(a.w + static_cast<int64_t>(n0) * a.ldw, static_cast<uint32_t>(tn * a.ldw * 2));
+    uint32_t woff[kFewNF];
+    row_offsets<kFewNF>(a.ldw, 0, tn, lane, woff);
+    f32x4 acc[kFewNF][1];
+#pragma unroll
+    for (int f = 0; f < kFewNF; ++f) acc[f][0] = f32x4{0.f, 0.f, 0.f, 0.f};
+    wave_mma<DT, 1, kFewNF, kFewU, PIPE>(xr, xoff, wr, woff, a.K, st0, st1, lane, acc);
+    __syncthreads();  // the tile before has been read
+    wave_spill<1, kFewNF>(red, wave, lane, acc);
+    __syncthreads();
+    const bool valid = lane < tn;
+    const int col = valid ? lane : 0;  // lanes past the tile read column 0 and discard it
+#pragma unroll
+    for (int j = 0; j < RPW; ++j) {
+      const int m = wave + kPackedWaves * j;
+      if (m < a.R) {
+        const float lv =
+            round_through(wg_sum<1, kFewNF>(red, kPackedWaves, red_offset<1, kFewNF>(col, m)), a.round_mode);
+        const float l = valid ? lv : -INFINITY;
+        // Tile maximum with lowest-index ties, then the two exponential sums against it.
+        RowState t{l, 0.f, 0.f, valid ? n0 + lane : INT_MAX};
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) {
+          const float omx = __shfl_xor(t.mx, off, 64);
+          const int oai = __shfl_xor(t.ai, off, 64);
+          if (omx > t.mx || (omx == t.mx && oai < t.ai)) {
+            t.mx = omx;
+            t.ai = oai;
+          }
+        }
+        float e = valid ? exp_below_max(l - t.mx) : 0.f;
+        float ab = (valid && l > own_l[j]) ? e : 0.f;
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) {
+          e += __shfl_xor(e, off, 64);
+          ab += __shfl_xor(ab, off, 64);
+        }
+        t.se = e;
+        t.ab = ab;
+        rs[j] = merge(rs[j], t);
+      }
+    }
+  }
+
+  if (lane == 0) {
+#pragma unroll
+    for (int j = 0; j < RPW; ++j) {
+      const int m = wave + kPackedWaves * j;
+      if (m < a.R) {
+        const int64_t slot = static_cast<int64_t>(blockIdx.x) * a.R + m;
+        publish(a.state + slot * 3 + 0, rs[j].mx);
+        publish(a.state + slot * 3 + 1, rs[j].se);
+        publish(a.state + slot * 3 + 2, rs[j].ab);
+        publish(a.state_idx + slot, rs[j].ai);
+      }
+    }
+  }
+  if (!arrive_last(a.counter, a.G)) return;
+
+  // Last workgroup: the G states of every row, strided over the lanes, then a butterfly.
+  for (int j = 0; j < RPW; ++j) {
+    const int m = wave + kPackedWaves * j;
+    if (m >= a.R) continue;
+    RowState s = empty_state();
+    for (int g = lane; g < a.G; g += 64) {
+      const int64_t slot = static_cast<int64_t>(g) * a.R + m;
+      s = merge(s, RowState{collect(a.state + slot * 3 + 0), collect(a.state + slot * 3 + 1),
+                            collect(a.state + slot * 3 + 2), collect(a.state_idx + slot)});
+    }
+    s = wave_merge(s);
+    if (lane == 0) {
+      a.accept[m] = accept_proposal(a, a.own[m], s) ? 1 : 0;
+      a.argmax[m] = s.ai;
+    }
+  }
+}
+
+template <int DT, bool PIPE>
+hipError_t launch_few_rows(VerifyArgs a, int cu_count, hipStream_t stream) {
+  auto kern = few_rows_kernel<DT, PIPE>;
+  static int per_cu = 0;
+  if (per_cu == 0) per_cu = std::max(1, resident_per_cu(reinterpret_cast<const void*>(kern), 64 * kPackedWaves, 0));
+  const int tiles = (a.V + 16 * kFewNF - 1) / (16 * kFewNF);
+  a.G = min(tiles, min(kMaxVerifyGroups, cu_count * per_cu));
+  hipLaunchKernelGGL((few_own_kernel<DT, PIPE>), dim3(a.R), dim3(64 * kPackedWaves), 0, stream, a);
+  const hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  hipLaunchKernelGGL(kern, dim3(a.G), dim3(64 * kPackedWaves), 0, stream, a);
+  return hipGetLastError();
+}
+
+// A tile is checked against the set of the launch it once chose; both kernels have their own.
 template <int DT>
 hipError_t verify_dispatch(const VerifyArgs& a, const plm_tile& t, int cu, hipStream_t s, bool dry) {
   const int64_t steps = (a.K + 31) / 32;
   if (t.k_waves != 4 || !verify_tile_known((a.R + 15) / 16, t, (steps + 3) / 4 > t.unroll)) return hipErrorInvalidConfiguration;
   if (dry) return hipSuccess;
+  if (few_rows_faster(a.R, a.V, a.K))
+    return steps > 4 * kFewU ? launch_few_rows<DT, true>(a, cu, s) : launch_few_rows<DT, false>(a, cu, s);
   switch ((a.R + 15) / 16) {
     case 1: return verify_rows_pick<DT, 1>(a, cu, s);
     case 2: return verify_rows_pick<DT, 2>(a, cu, s);
@@ -871,7 +1057,8 @@ size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
 // Workspace layout: counter area (ints kVerifyCounter, kVerifyOwnDone, kPkErrorSlot and
 // [kVerifyGroupBase, +groups) used) | own[R] | rec[kMaxVerifyGroups][R] | grec[groups][R],
-// groups = kMaxVerifyGroups / kVerifyGroupSize; a record takes the 12 + 4 bytes of its two areas.
+// groups = kMaxVerifyGroups / kVerifyGroupSize; a record takes the 12 + 4 bytes of its two areas (few_rows_kernel
+// keeps state and state_idx in rec's two).
 constexpr int kMaxVerifyGroupSets = kMaxVerifyGroups / kVerifyGroupSize;
 static_assert(kVerifyGroupBase + kMaxVerifyGroupSets <= 64, "group counters fit before the streaming counters");
 void verify_layout(int64_t R, size_t& own_off, size_t& state_off, size_t& idx_off, size_t& gstate_off,
@@ -947,6 +1134,8 @@ int plm_lm_head_verify(int32_t dtype, const void* x, int64_t ldx, const void* w,
   a.counter = reinterpret_cast<int*>(ws) + plm::kVerifyCounter;
   a.own = reinterpret_cast<float*>(ws + own_off);
   a.group_counter = reinterpret_cast<int*>(ws) + plm::kVerifyGroupBase;
+  a.state = reinterpret_cast<float*>(ws + state_off);
+  a.state_idx = reinterpret_cast<int*>(ws + idx_off);
   a.rec = reinterpret_cast<plm::f32x4*>(ws + state_off);
   a.grec = reinterpret_cast<plm::f32x4*>(ws + gstate_off);
   a.own_done = reinterpret_cast<int*>(ws) + plm::kVerifyOwnDone;

@@ -31,6 +31,15 @@ def test_quarters_and_tiles(device, R, V, K, dtype):
             run_case(x, w, pending, 0.7, m, device, check_cpu=False, packed=False)
 
 
+# few_rows_kernel: one row, both pipelines (K steps per wavefront up to four, and more), K off the step and
+# fewer steps than quarters, the last row of its range and the next one, more tiles than workgroups.
+@pytest.mark.parametrize("R,V,K", [(1, 8192, 512), (2, 33, 8), (4, 1001, 520), (7, 4097, 2056), (8, 4097, 2056),
+                                   (14, 300, 4096), (15, 300, 4096), (2, 31000, 4104)])
+def test_few_rows(device, R, V, K):
+    test_quarters_and_tiles(device, R, V, K, torch.bfloat16)
+    test_quarters_and_tiles(device, R, V, K, torch.float16)
+
+
 @pytest.mark.parametrize("packed", [True, False], ids=["packed", "rowmajor"])
 @pytest.mark.parametrize("R,V,K", [(3, 1, 8), (5, 129, 64), (16, 5003, 64), (42, 300, 2048), (64, 20000, 64)])
 def test_rows_of_minus_infinity_name_their_first_id(device, R, V, K, packed):
