@@ -118,8 +118,8 @@ int plm_unpack_weight(int32_t dtype, const void* packed, size_t packed_bytes, in
  * wavefront (1, 2, 4); k_waves = 4: a workgroup tile is 16*wave_frags rows and its four
  * wavefronts split the tile's K range (summed in LDS in wavefront order), or k_waves = 1: a
  * workgroup tile is 64*wave_frags rows, each wavefront owns 16*wave_frags of them over the whole
- * K range, and the four share one copy of X through LDS (where M > 64 or the packed weight is under
- * 128 MiB, such a call runs on the wide kernel, with the same sums in the same order); split_k = workgroups splitting K (1..64,
+ * K range, and the four share one copy of X through LDS (except at M <= 64 over a packed weight of 128 MiB
+ * and more with N > 32768, such a call runs on the wide kernel, with the same sums in the same order); split_k = workgroups splitting K (1..64,
  * partials summed in split order); unroll = K steps of loads in flight per wavefront (2, 4, 6,
  * 8). Requirements as plm_gemm (K % 8 == 0, K <= 2^24, ldx % 8 == 0, x 16-byte aligned) except
  * that M may exceed 128: wider calls (prefill chunks, plm/rounds.py:16, which the reference hands to

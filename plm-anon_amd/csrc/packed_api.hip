@@ -182,13 +182,19 @@ int packed_launch_args(int32_t dtype, PackedArgs& a, const plm_tile& t, void* wo
 }
 
 // Whether a single linear on a row-split tile (k_waves = 1) runs on the wide kernel, whose sums are the
-// row-split kernel's bit for bit: weights below 128 MiB, or widths above 64 rows. There the wide
-// kernel's X, read once per workgroup into LDS, and its smaller tiles win (us, best tile of the packed
-// kernel against it: M = 56, 6144x2048 11.9 / 8.8, 16384x3072 24.1 / 20.8; M = 110, 3072x3072 17.4 /
-// 11.0, 50257x2048 62.0 / 48.2); a longer stream at few rows is bound by HBM either way and the
-// row-split kernel's deeper pipeline is level or ahead (50257x2048: M = 7 40.2 / 41.4, M = 56 46.6 / 46.7).
+// row-split kernel's bit for bit: always, but for the long streams of a weight of 128 MiB and more with
+// over 256 tiles of 128 rows (with K splits, from 512 items on) at up to 64 rows of X. The wide kernel's X, read once per workgroup into LDS,
+// and its smaller tiles win (us, best row-split tile of the packed kernel against it: M = 56, 6144x2048
+// 11.9 / 8.8, 16384x3072 24.1 / 20.8; M = 110, 3072x3072 17.4 / 11.0, 50257x2048 62.0 / 48.2; weights of
+// 128 MiB and more at M = 7 16384x4096 46.7 / 26.1, 32768x2048 32.8 / 26.1, 28672x4096 56.1 / 43.0, at
+// M = 56 4096x16384 173 / 48, 8192x8192 93 / 33). The LM heads' streams are bound by HBM either way, and
+// the row-split kernel's deeper pipeline is level or ahead (50257x2048: M = 7 40.2 / 41.4, M = 56 46.6 /
+// 46.7; 40000x2048: M = 7 32.6 / 34.3), as it is where K splits make many items of such a weight (four
+// splits: 32768x2048 at M = 7 33.6 / 38.2, 28672x4096 50.0 / 54.0, but 16384x8192 54.3 / 52.9).
 bool wide_preferred(int64_t M, int64_t N, int64_t K, const plm_tile& t) {
-  if (t.k_waves != 1 || (M <= 64 && packed_bytes(N, K) >= (int64_t(128) << 20))) return false;
+  if (t.k_waves != 1) return false;
+  const bool many = t.split_k == 1 ? N > 128 * 256 : N * t.split_k >= 128 * 512;
+  if (M <= 64 && many && packed_bytes(N, K) >= (int64_t(128) << 20)) return false;
   // Split partials lie behind one 32-bit buffer range.
   return t.split_k == 1 || t.split_k * ((N + 15) / 16) * ((M + 15) / 16) * kFragBytes < (int64_t(1) << 31);
 }

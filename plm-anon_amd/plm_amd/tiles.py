@@ -112,8 +112,8 @@ def _first_compiled(M: int, nf: int, layouts, supported) -> dict | None:
 
 
 # The wide kernel (csrc/wide_gemm.hip), which runs single linears on row-split tiles: its tiles as
-# (64-row weight blocks, 16-row X fragments), and above this packed size at up to 64 rows the row-split
-# kernel proper (``wide_preferred`` in csrc/packed_api.hip).
+# (64-row weight blocks, 16-row X fragments). From this packed size on, with more 128-row tiles than compute
+# units and up to 64 rows, they run on the row-split kernel proper (``wide_preferred`` in csrc/packed_api.hip).
 WIDE_TILES = ((1, 1), (1, 2), (1, 3), (1, 4), (1, 5), (1, 8), (2, 1), (2, 2), (2, 3), (2, 4), (2, 5), (2, 6), (2, 8),
               (2, 10), (4, 8))
 WIDE_WEIGHT_BYTES = 128 << 20
@@ -121,7 +121,8 @@ ROW_SPLIT_SPLITS = (1, 2, 3, 4, 6)
 
 
 def runs_wide(M: int, N: int, K: int) -> bool:
-    return M > 64 or math.ceil(N / 256) * 16 * math.ceil(K / 256) * 8 * FRAG < WIDE_WEIGHT_BYTES
+    return (M > 64 or N <= 128 * CU_COUNT or
+            math.ceil(N / 256) * 16 * math.ceil(K / 256) * 8 * FRAG < WIDE_WEIGHT_BYTES)
 
 
 def row_split_splits(M: int, N: int, K: int) -> int:
@@ -144,12 +145,12 @@ def row_split_splits(M: int, N: int, K: int) -> int:
 
 def heuristic_tile(M: int, N: int, K: int, supported=None) -> dict:
     """A reasonable tile without measurement: rows split across the wavefronts (the wide kernel's
-    linears, with ``row_split_splits``'s K splits; the row-split kernel itself for weights past
-    ``WIDE_WEIGHT_BYTES`` at up to 64 rows), else ``k_split_tile``. Up to 16 rows a long K whose K-split
-    items fit the CUs one each keeps those: their join is a sum in LDS and fewer partials, or none.
-    Row-split against K-split, us at 2 to 16 rows: 1024x4096 8.6 / 7.7, 2048x8192 12.6 / 11.4, 2048x5632
-    10.5 / 9.6, 6144x2048 9.2 / 8.2, 8192x2048 9.8 / 9.4; but 2048x2048, which needs four splits, 7.2 / 7.5,
-    3072x1024 4.8 / 6.7 and 2560x10240, whose 320 items take two rounds, 15.4 / 18.1."""
+    linears, with ``row_split_splits``'s K splits; the row-split kernel itself where not ``runs_wide``),
+    else ``k_split_tile``. Up to 16 rows a long K whose K-split items fit the CUs one each keeps those: their
+    join is a sum in LDS and fewer partials, or none. Row-split against K-split, us at 2 to 16 rows:
+    1024x4096 8.6 / 7.7, 2048x8192 12.6 / 11.4, 2048x5632 10.5 / 9.6, 6144x2048 9.2 / 8.2, 8192x2048 9.8 /
+    9.4; but 2048x2048, which needs four splits, 7.2 / 7.5, 3072x1024 4.8 / 6.7 and 2560x10240, whose 320
+    items take two rounds, 15.4 / 18.1."""
     if M <= 16 and K >= 2048 and _first_compiled(M, 2, (8, 4), supported):
         cfg = k_split_tile(M, N, K, supported)
         if items(N, cfg) <= CU_COUNT and (K >= 4096 or cfg["split_k"] == 1):

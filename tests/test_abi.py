@@ -111,6 +111,17 @@ def test_released_calls_the_library_is_faster_at_go_to_f_linear():
     assert fast_gemm._wide_pays(2048, 16384, 3072, True) and not fast_gemm._wide_pays(2049, 16384, 3072, True)
 
 
+def test_untuned_large_weights_at_few_rows_take_the_wide_kernel():
+    """A weight of 128 MiB and more at up to 64 rows: row-split tiles that run on the wide kernel, but for
+    the LM heads' many tiles, which keep 128-row tiles of the row-split kernel."""
+    for N, K in ((16384, 4096), (22000, 4096), (28672, 4096), (32768, 2048)):
+        for M in (1, 7, 30, 64):
+            cfg = fast_gemm.default_config(M, N, K)
+            assert tiles.runs_wide(M, N, K) and cfg["k_waves"] == 1 and cfg["wave_frags"] == 2, (M, N, K, cfg)
+    assert not tiles.runs_wide(64, 50257, 2048) and tiles.runs_wide(65, 50257, 2048)
+    assert fast_gemm.default_config(42, 50257, 2048) == {"wave_frags": 2, "k_waves": 1, "split_k": 1, "unroll": 2}
+
+
 def test_epilogue_argument_validation_happens_before_launch():
     lib = _lib.lib()
     fake = 1 << 20

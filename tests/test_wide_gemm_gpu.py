@@ -74,8 +74,10 @@ def test_silu_mul_of_a_released_gate_up_weight(device, M, N, K):
 
 
 # Rounds on row-split tiles: one row, a tile's edge and past it, the widest; ranges of K steps that
-# start inside a group of packed steps, of odd length, and shorter than the loads in flight.
-@pytest.mark.parametrize("M,N,K", [(1, 64, 96), (17, 1003, 1416), (56, 2048, 8192), (65, 4608, 3072), (128, 777, 1000)])
+# start inside a group of packed steps, of odd length, and shorter than the loads in flight; a weight of
+# 128 MiB, whose widest splits stay on the row-split kernel.
+@pytest.mark.parametrize("M,N,K", [(1, 64, 96), (17, 1003, 1416), (56, 2048, 8192), (65, 4608, 3072), (128, 777, 1000),
+                                   (30, 16384, 4096)])
 @pytest.mark.parametrize("split", [1, 2, 3, 6])
 def test_row_split_tiles_with_k_splits(device, M, N, K, split):
     print(f"row split M={M} N={N} K={K} split={split}", flush=True)
