@@ -143,17 +143,35 @@ def row_split_splits(M: int, N: int, K: int) -> int:
     return min((s for s in ROW_SPLIT_SPLITS if s == 1 or steps // s >= 16), key=cost)
 
 
+def _keeps_k_split(M: int, N: int, K: int, cfg: dict) -> bool:
+    """Whether a long K over few columns keeps its K-split tile ``cfg``, whose items fit the CUs one each:
+    their join is a sum in LDS and fewer partials, or none, while a row-split tile's items each walk a sixth
+    of K at best. Row-split against K-split, us:
+
+    * up to 16 rows: 1024x4096 8.6 / 7.7, 2048x8192 12.6 / 11.4, 2048x5632 10.5 / 9.6, 6144x2048 9.2 / 8.2,
+      8192x2048 9.8 / 9.4, 7168x1536 8.3 / 7.9, 160x2504 6.0 / 5.5, 160x3368 6.7 / 5.9, 2048x3368 8.8 / 8.5;
+      but 4096x3368 10.3 / 10.5, 2048x2048, which needs four splits, 7.2 / 7.5, 7168x1280 the same, 3072x1024
+      4.8 / 6.7 and 2560x10240, whose 320 items take two rounds, 15.4 / 18.1;
+    * 17 to 32: 160x3368 6.9 / 6.6, 512x4096 7.7 / 7.5, 768x6456 8.9 / 8.2, 1024x8192 11.0 / 9.6, 1024x12936
+      13.3 / 12.4; but 768x4096 7.2 / 7.6, 1536x6456 10.9 / 11.9, 1536x12936 16.3 / 18.8;
+    * 33 to 64: 160x4096 7.3 / 6.9 and 256x12936 9.9 / 9.6 at 48, 64x8192 8.3 / 7.3 at 56; but 512x6456
+      8.9 / 9.2 at 42, 160x8192 at 56 the same."""
+    if items(N, cfg) > CU_COUNT:
+        return False
+    if M <= 16:
+        return K >= 4096 or cfg["split_k"] == 1 or (K >= 3072 and N <= 2048) or (K > 2048 and N <= 256)
+    if M <= 32:
+        return (K >= 4096 and N <= min(1024, K // 6)) or (K >= 3328 and N <= 256)
+    return K >= 4096 and N <= (256 if M <= 48 else 64)
+
+
 def heuristic_tile(M: int, N: int, K: int, supported=None) -> dict:
     """A reasonable tile without measurement: rows split across the wavefronts (the wide kernel's
     linears, with ``row_split_splits``'s K splits; the row-split kernel itself where not ``runs_wide``),
-    else ``k_split_tile``. Up to 16 rows a long K whose K-split items fit the CUs one each keeps those: their
-    join is a sum in LDS and fewer partials, or none. Row-split against K-split, us at 2 to 16 rows:
-    1024x4096 8.6 / 7.7, 2048x8192 12.6 / 11.4, 2048x5632 10.5 / 9.6, 6144x2048 9.2 / 8.2, 8192x2048 9.8 /
-    9.4; but 2048x2048, which needs four splits, 7.2 / 7.5, 3072x1024 4.8 / 6.7 and 2560x10240, whose 320
-    items take two rounds, 15.4 / 18.1."""
-    if M <= 16 and K >= 2048 and _first_compiled(M, 2, (8, 4), supported):
+    else, and up to 64 rows where ``_keeps_k_split``, ``k_split_tile``."""
+    if M <= 64 and K >= 1536 and _first_compiled(M, 2, (8, 4), supported):
         cfg = k_split_tile(M, N, K, supported)
-        if items(N, cfg) <= CU_COUNT and (K >= 4096 or cfg["split_k"] == 1):
+        if _keeps_k_split(M, N, K, cfg):
             return cfg
     for nf in (2, 1, 4):
         cfg = _first_compiled(M, nf, (1,), supported)

@@ -122,6 +122,16 @@ def test_untuned_large_weights_at_few_rows_take_the_wide_kernel():
     assert fast_gemm.default_config(42, 50257, 2048) == {"wave_frags": 2, "k_waves": 1, "split_k": 1, "unroll": 2}
 
 
+def test_untuned_long_k_over_few_columns_keeps_the_k_split():
+    """Shapes (M, N, K) on both sides of each line of ``tiles._keeps_k_split``, as timed."""
+    k_split = [(1, 180, 2264), (2, 6434, 1608), (12, 156, 3368), (16, 2048, 3368), (17, 160, 3368), (17, 169, 12936), (17, 512, 4096), (32, 1024, 6456), (48, 160, 4096),
+               (64, 64, 8192)]
+    row_split = [(16, 4096, 3368), (2, 6434, 1528), (16, 160, 2048), (16, 2048, 2048), (17, 512, 3368), (17, 768, 4096), (17, 1536, 12936), (33, 512, 6456),
+                 (49, 160, 8192), (65, 64, 8192)]
+    assert all(fast_gemm.default_config(*s)["k_waves"] > 1 for s in k_split)
+    assert all(fast_gemm.default_config(*s)["k_waves"] == 1 for s in row_split)
+
+
 def test_epilogue_argument_validation_happens_before_launch():
     lib = _lib.lib()
     fake = 1 << 20
