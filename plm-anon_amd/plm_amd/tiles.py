@@ -168,7 +168,11 @@ def _keeps_k_split(M: int, N: int, K: int, cfg: dict) -> bool:
 def heuristic_tile(M: int, N: int, K: int, supported=None) -> dict:
     """A reasonable tile without measurement: rows split across the wavefronts (the wide kernel's
     linears, with ``row_split_splits``'s K splits; the row-split kernel itself where not ``runs_wide``),
-    else, and up to 64 rows where ``_keeps_k_split``, ``k_split_tile``."""
+    else, and up to 64 rows where ``_keeps_k_split``, ``k_split_tile``. K splits only where
+    ``k_split_tile`` has them too: a weight whose items fill the CUs needs no workspace, so that a call on it
+    can be captured first thing, and run beside one on another stream (us unsplit / split: 6144x4096 at
+    M = 30 14.1 / 15.5, 8192x8192 at 42 32.9 / 29.5, 6144x14336 at 42 49.3 / 39.3; K-split tiles 15.5, 42.3,
+    62.7)."""
     if M <= 64 and K >= 1536 and _first_compiled(M, 2, (8, 4), supported):
         cfg = k_split_tile(M, N, K, supported)
         if _keeps_k_split(M, N, K, cfg):
@@ -178,7 +182,8 @@ def heuristic_tile(M: int, N: int, K: int, supported=None) -> dict:
         if cfg is None:
             continue
         if runs_wide(M, N, K):
-            return dict(cfg, split_k=row_split_splits(M, N, K))
+            split = k_split_tile(M, N, K)["split_k"] > 1
+            return dict(cfg, split_k=row_split_splits(M, N, K) if split else 1)
         if math.ceil(N / 16) // (K_WAVES * nf) >= CU_COUNT:
             return cfg
     return k_split_tile(M, N, K, supported)

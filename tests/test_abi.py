@@ -132,6 +132,15 @@ def test_untuned_long_k_over_few_columns_keeps_the_k_split():
     assert all(fast_gemm.default_config(*s)["k_waves"] == 1 for s in row_split)
 
 
+def test_untuned_weights_that_fill_the_device_need_no_workspace():
+    """From 192 tiles of 32 rows on (6144 rows; the K-split tiles of such a weight are not split either) a
+    default tile has no K split, so that a call on it can be captured without a workspace."""
+    for M in (1, 16, 17, 42, 72, 128):
+        for N, K in ((6144, 4096), (6144, 14336), (8192, 8192), (11264, 14336), (28672, 28672), (50257, 2048)):
+            assert fast_gemm.gemm_workspace_bytes(M, N, K, fast_gemm.default_config(M, N, K)) == 0, (M, N, K)
+    assert fast_gemm.default_config(42, 4096, 14336)["split_k"] > 1
+
+
 def test_epilogue_argument_validation_happens_before_launch():
     lib = _lib.lib()
     fake = 1 << 20

@@ -167,3 +167,21 @@ def test_prefill_matches_oracle_on_a_full_block(device):
         cols = torch.randperm(N, generator=torch.Generator().manual_seed(i))[:256]
         check_cols(y, x, ref_w, cols)
         del ref_w
+
+
+def test_untuned_call_on_a_large_weight_is_captured_without_a_workspace(device, monkeypatch):
+    """The first call on a released weight whose tiles fill the device, inside a capture, with no workspace
+    yet; each replay equals the eager call on its input."""
+    x, w = _inputs_on_gpu(17, 6144, 4096, 5, device)
+    release(w)
+    monkeypatch.setattr(fast_gemm, "_workspaces", {})
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        y = released_linear(x, w)
+    assert not fast_gemm._workspaces
+    for _ in range(3):
+        x.copy_(torch.randn(17, 4096, device=device))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, released_linear(x, w))
