@@ -330,9 +330,10 @@ def llama_mlp(x: torch.Tensor, gate_up_weight: torch.Tensor, down_weight: torch.
 
 
 def reserve_workspace(device: torch.device, shapes: dict[tuple[int, int, int], Config] | None = None) -> None:
-    """Size the device workspace for every configured shape, so later calls can be graph-captured."""
-    shapes = CONFIGS if shapes is None else shapes
-    need = max((gemm_workspace_bytes(M, N, K, cfg) for (M, N, K), cfg in shapes.items()), default=0)
+    """Size the device workspace for every configured shape (the activation tiles' too), so later calls can
+    be graph-captured."""
+    shapes = [*CONFIGS.items(), *ACT_CONFIGS.items()] if shapes is None else shapes.items()
+    need = max((gemm_workspace_bytes(M, N, K, cfg) for (M, N, K), cfg in shapes), default=0)
     if need:
         workspace(device, need)
 

@@ -141,6 +141,18 @@ def test_untuned_weights_that_fill_the_device_need_no_workspace():
     assert fast_gemm.default_config(42, 4096, 14336)["split_k"] > 1
 
 
+def test_reserved_workspace_holds_the_activation_tiles(monkeypatch):
+    table, act = {(42, 4096, 1024): {"wave_frags": 2, "k_waves": 1, "split_k": 1, "unroll": 2}}, dict(
+        wave_frags=2, k_waves=1, split_k=2, unroll=2)
+    monkeypatch.setattr(fast_gemm, "CONFIGS", table)
+    monkeypatch.setattr(fast_gemm, "ACT_CONFIGS", {(42, 4096, 1024): act})
+    asked = []
+    monkeypatch.setattr(fast_gemm, "workspace", lambda device, nbytes: asked.append(nbytes))
+    fast_gemm.reserve_workspace(torch.device("cpu"))
+    fast_gemm.reserve_workspace(torch.device("cpu"), table)
+    assert asked == [fast_gemm.gemm_workspace_bytes(42, 4096, 1024, act)]
+
+
 def test_epilogue_argument_validation_happens_before_launch():
     lib = _lib.lib()
     fake = 1 << 20
