@@ -111,6 +111,15 @@ def test_released_calls_the_library_is_faster_at_go_to_f_linear():
     assert fast_gemm._wide_pays(2048, 16384, 3072, True) and not fast_gemm._wide_pays(2049, 16384, 3072, True)
 
 
+def test_wide_tiles_are_the_kernels():
+    """The host's copy of the wide kernel's tiles, its picked table and its compiled switch are one list."""
+    text = (REPO / "plm-anon_amd" / "csrc" / "wide_gemm.hip").read_text()
+    table = re.search(r"kWideTiles\[\] = \{(.*?)\};", text, re.S).group(1)
+    listed = [tuple(map(int, pair)) for pair in re.findall(r"\{(\d+), (\d+)\}", table)]
+    cases = {(int(nf or 1), int(mt)) for nf, mt in re.findall(r"case 16(?: \* (\d))? \+ (\d+): return wide_go", text)}
+    assert tuple(listed) == tiles.WIDE_TILES and set(listed) == cases
+
+
 def test_untuned_large_weights_at_few_rows_take_the_wide_kernel():
     """A weight of 128 MiB and more at up to 64 rows: row-split tiles that run on the wide kernel, but for
     the LM heads' many tiles, which keep 128-row tiles of the row-split kernel."""

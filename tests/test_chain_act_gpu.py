@@ -1,10 +1,12 @@
 """GPU parity of packed chains with SiLU-and-multiply links (``Link(act=True)``, ``out_f32 =
 PLM_OUT_SILU_MUL``): the Llama-style MLP's real dataflow, gate/up projection with its activation,
-then down reading the activation's ``[M, I]`` output, inside one persistent launch.
+then down reading the activation's ``[M, I]`` output, inside one persistent launch, or on the row-split
+tiles of widths above 48 rows as a launch per link, in order.
 
 Every link's output must equal its single-launch equivalent bit for bit (``gate_up_silu`` for an
 act link, ``hip_linear`` otherwise, same tile and split): the chain runs the same kernel over the
-same K partition. The tile-flag mode (each linear reads the one before it) is checked with inputs
+same K partition (on a row-split tile the equivalent is a chain of the link alone, which runs the packed
+kernel where the chain's launches are the wide kernel's). The tile-flag mode (each linear reads the one before it) is checked with inputs
 rewritten and every output filled with NaN before each of several launches and graph replays, so a
 consumer that read a producer's tile before it was written would show; the error flag stays clear."""
 
@@ -44,6 +46,10 @@ def _llama_links(x, layers, hidden, qkv, inter, gen, cfg, G, act=True):
 
 
 def _single(ln, cfg):
+    if cfg["k_waves"] == 1:   # the packed row-split kernel, which a chain of one link runs
+        y = torch.empty_like(ln.y)
+        LinearChain([Link(ln.x, ln.w, y, split_k=ln.split_k, act=ln.act)], cfg).run()
+        return y
     c = dict(cfg, split_k=ln.split_k)
     return gate_up_silu(ln.x, ln.w, c) if ln.act else hip_linear(ln.x, ln.w, c)
 
@@ -71,7 +77,7 @@ def test_mlp_chain_matches_single_launches(device, M):
     chain.check()
     want_act = _single(links[0], cfg)
     assert torch.equal(act, want_act)
-    assert torch.equal(out, hip_linear(want_act, w_d, dict(cfg, split_k=links[1].split_k)))
+    assert torch.equal(out, _single(Link(want_act, w_d, out, split_k=links[1].split_k), cfg))
     # The activation against the oracle: the projection on the CPU, then silu(g) * u.
     cols = torch.randperm(5632, generator=torch.Generator().manual_seed(M))[:128]
     rows = torch.cat([cols, cols + 5632]).to(device)
@@ -80,11 +86,11 @@ def test_mlp_chain_matches_single_launches(device, M):
     assert bool(((sub - ref).abs() <= 2e-2 + 1e-3 * ref.abs()).all())
 
 
-def test_llama_blocks_chain_with_rewritten_inputs(device):
+@pytest.mark.parametrize("M", [42, 56])
+def test_llama_blocks_chain_with_rewritten_inputs(device, M):
     """Three Llama-style 1.3B blocks (qkv 3072, o, gate_up 11264 with its activation, down from 5632)
-    in one tile-flag launch: 6 launches and 3 graph replays, each after rewriting x and filling
-    every output with NaN; each launch's outputs equal the single launches on that launch's x."""
-    M = 56
+    in one tile-flag launch (M = 42) and as a launch per link (56): 6 runs and 3 graph replays, each after
+    rewriting x and filling every output with NaN; each run's outputs equal the single launches on that run's x."""
     gen = torch.Generator(device=device).manual_seed(7)
     cfg = packed_chain_tile(M)
     G = _grid(M, cfg)

@@ -1,10 +1,13 @@
-"""GPU parity of the chained launches: linears back to back in one persistent grid, over packed
+"""GPU parity of chains: linears back to back in one persistent grid, over packed
 weights (plm_gemm_chain_packed: tile-done flags when every linear reads the one before it, else
 grid barriers of per-workgroup progress flags) and over row-major weights (plm_gemm_chain: each
 consumer tile starts once the producer tiles it reads are written).
 
+On a row-split tile a packed chain is a launch per linear (mostly the wide kernel), in order.
+
 Checks: every link's output equals the single-linear kernel's on the same operands bit for bit
-(same kernel, same K partition), and the CPU oracle's within the GEMM tolerance; repeated launches
+(same kernel, same K partition; for a row-split tile the packed kernel's own, as a chain of that link
+alone runs it), and the CPU oracle's within the GEMM tolerance; repeated launches
 and HIP-graph replays give identical results (flags are per launch); the error flag stays clear."""
 
 from __future__ import annotations
@@ -42,14 +45,22 @@ def _chain(x, ws, splits, deps=None, ys=None):
     return links, ys
 
 
+def _single(ln, cfg, packed=True):
+    """The link's linear alone, on a kernel other than the chain's launches for row-split tiles."""
+    if packed and cfg["k_waves"] == 1:
+        y = torch.empty_like(ln.y)
+        LinearChain([Link(ln.x, ln.w, y, split_k=ln.split_k, act=ln.act)], cfg).run()
+        return y
+    linear = hip_linear if packed else hip_linear_rowmajor
+    return linear(ln.x, ln.w, dict(cfg, split_k=ln.split_k))
+
+
 def _check_against_single(links, cfg=CFG, packed=True):
     """Bit for bit the single-linear kernel; against the oracle within 1e-3 rel / 2e-2 abs, or one
     output rounding step where the oracle's own fp32 sum lands on the other side of a rounding
     midpoint (at |y| >= 4 one bf16 step exceeds 2e-2), for at most 0.1 % of a link's elements."""
     for i, ln in enumerate(links):
-        linear = hip_linear if packed else hip_linear_rowmajor
-        single = linear(ln.x, ln.w, dict(cfg, split_k=ln.split_k))
-        assert torch.equal(ln.y, single), f"link {i} differs from the single-linear kernel"
+        assert torch.equal(ln.y, _single(ln, cfg, packed)), f"link {i} differs from the single-linear kernel"
         got = ln.y.cpu().float()
         ref = oracle.linear(ln.x.cpu(), ln.w.cpu()).float()
         diff = (got - ref).abs()
@@ -246,7 +257,7 @@ def _chain_table_entries():
 @pytest.mark.parametrize("hidden,M", _chain_table_entries(), ids=lambda v: str(v))
 def test_round_chain_table_tiles(device, hidden, M):
     """Every measured chain tile (chain_tiles_hidden<H>.json) on one block of the round it was
-    measured on, at its width, each linear reading the one before it (the tile-flag launch), launched twice
+    measured on, at its width, each linear reading the one before it (the tile-flag launch, or a launch per linear), launched twice
     with a new input and NaN-filled outputs: bit for bit the single-linear kernel, and the oracle
     within the GEMM tolerance."""
     from plm_amd import _lib, gemm_tables
@@ -304,7 +315,6 @@ def test_round_chain_graph_replays_with_new_inputs(device):
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=stream):
         chain.run()
-    refs = [torch.empty_like(y) for y in ys]
     sample = torch.randperm(2048, generator=torch.Generator().manual_seed(62))[:96]
     for rep in range(8):
         x.copy_(torch.randn(M, 2048, generator=g, device=device).bfloat16())
@@ -313,10 +323,7 @@ def test_round_chain_graph_replays_with_new_inputs(device):
         torch.cuda.synchronize()
         graph.replay()
         torch.cuda.synchronize()
-        for ln, ref in zip(links, refs):
-            hip_linear(ln.x, ln.w, dict(cfg, split_k=ln.split_k), ref)
-        torch.cuda.synchronize()
-        bad = [i for i, (y, r) in enumerate(zip(ys, refs)) if not torch.equal(y, r)]
+        bad = [i for i, ln in enumerate(links) if not torch.equal(ln.y, _single(ln, cfg))]
         assert not bad, f"replay {rep}: links {bad[:8]} differ from per-linear launches"
         if rep in (0, 7):
             for i in (0, 1, 2, 3, 92, 93, 94, 95):
@@ -327,8 +334,8 @@ def test_round_chain_graph_replays_with_new_inputs(device):
 
 def test_config4_round_chain_all_columns(device):
     """Config 4's round: all 128 block linears of the 32-block hidden-2560 round (QKV 2560 -> 7680,
-    attn-out, MLP up 2560 -> 10240, down) at M = 56 in one tile-flag launch, with the round's chain
-    tile and splits, launched twice with a new input and NaN-filled outputs. Every link equals its
+    attn-out, MLP up 2560 -> 10240, down) at M = 56, with the round's chain tile (a row-split one: a launch
+    per linear) and splits, launched twice with a new input and NaN-filled outputs. Every link equals its
     per-linear launch bit for bit, and the first and last blocks' four linears match the CPU oracle
     on every column."""
     from plm_amd import _lib, gemm_tables
@@ -351,16 +358,12 @@ def test_config4_round_chain_all_columns(device):
     links, ys = _chain(x, ws, [packed_chain_split(n, k, cfg, G) for n, k in shapes])
     chain = LinearChain(links, cfg, packed=True)
     assert chain.sync_mode == 2
-    refs = [torch.empty_like(y) for y in ys]
     for rep in range(2):
         x.copy_(torch.randn(M, hidden, generator=g, device=device).bfloat16())
         for y in ys:
             y.fill_(float("nan"))
         chain.run()
-        for ln, ref in zip(links, refs):
-            hip_linear(ln.x, ln.w, dict(cfg, split_k=ln.split_k), ref)
-        torch.cuda.synchronize()
-        bad = [i for i, (y, r) in enumerate(zip(ys, refs)) if not torch.equal(y, r)]
+        bad = [i for i, ln in enumerate(links) if not torch.equal(ln.y, _single(ln, cfg))]
         assert not bad, f"launch {rep}: links {bad[:8]} differ from per-linear launches"
     for i in (0, 1, 2, 3, 124, 125, 126, 127):
         _oracle_columns(links[i].x, ws[i], ys[i], torch.arange(ws[i].shape[0]))
@@ -389,16 +392,12 @@ def test_fp16_round_chain(device):
     links, ys = _chain(x, ws, [packed_chain_split(n, k, cfg, G) for n, k in shapes])
     chain = LinearChain(links, cfg, packed=True)
     assert chain.sync_mode == 2
-    refs = [torch.empty_like(y) for y in ys]
     for rep in range(2):
         x.copy_(torch.randn(M, hidden, generator=g, device=device).half())
         for y in ys:
             y.fill_(float("nan"))
         chain.run()
-        for ln, ref in zip(links, refs):
-            hip_linear(ln.x, ln.w, dict(cfg, split_k=ln.split_k), ref)
-        torch.cuda.synchronize()
-        bad = [i for i, (y, r) in enumerate(zip(ys, refs)) if not torch.equal(y, r)]
+        bad = [i for i, ln in enumerate(links) if not torch.equal(ln.y, _single(ln, cfg))]
         assert not bad, f"launch {rep}: links {bad[:8]} differ from per-linear launches"
     for i in (0, 1, 2, 3, 92, 93, 94, 95):
         _oracle_columns(links[i].x, ws[i], ys[i], torch.arange(ws[i].shape[0]))

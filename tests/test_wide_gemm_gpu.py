@@ -1,7 +1,8 @@
 """plm_gemm_wide: every output is one MFMA chain over K in ascending order, so it equals the packed
 row-split kernel without K splits, as a one-link chain runs it (its own parity against the oracle:
 tests/test_chain_gpu.py), bit for bit, at the edges of its tiles (16 to 160 rows of X by 64 to 256 of W)
-and of its 64-wide K stages; and with K splits, which single linears on row-split tiles run with. The
+and of its 64-wide K stages; and with K splits, which single linears on row-split tiles run with. Each
+compiled tile and epilogue runs at least once, on shapes that pick it (TILE_SHAPES). The
 activation epilogue equals torch's silu and multiply on the rounded projection up to one output step
 where the two exponentials' last bits part."""
 
@@ -15,6 +16,7 @@ from plm_amd import _lib, fast_gemm
 from plm_amd.chain import Link, LinearChain
 from plm_amd.fast_gemm import hip_linear, hip_linear_f32, pack_weight, release, released_linear
 from plm_amd.gated_lora import gated_linear
+from plm_amd.tiles import CU_COUNT, WIDE_TILES
 from test_gemm_gpu import _inputs_on_gpu
 
 pytestmark = pytest.mark.gpu
@@ -71,6 +73,74 @@ def test_silu_mul_of_a_released_gate_up_weight(device, M, N, K):
     # expf of the two sides may round apart: one step of the silu (2^-8 relative) and one of the product.
     assert int((got != want).sum()) <= max(1, got.numel() // 1000)
     torch.testing.assert_close(got.float(), want.float(), rtol=2 * 2.0 ** -7, atol=1e-30)
+
+
+def _picked(M, N, split=1, act=False):
+    """``wide_pick`` of csrc/wide_gemm.hip: the tile of the least rounds over the CUs times bytes per K step."""
+    def cost(tile):
+        nf, mt = tile
+        columns = 64 * nf // (2 if act else 1)
+        items = -(-(N // 2 if act else N) // columns) * -(-M // (16 * mt)) * split
+        return -(-items // CU_COUNT) * (4 * nf + mt)
+
+    return min((t for t in WIDE_TILES if not (act and t[0] % 2)), key=cost)
+
+
+# (M, N, split) that pick every compiled tile once, with M and N off its edges: past 128 rows and in the
+# whole-weight form (plm_gemm_wide), on row-split tiles with K splits, and the gated-LoRA launch, whose
+# 160-row and 256-column tiles are not compiled.
+TILE_SHAPES = {
+    "plain": [(m, n, 1) for m, n in ((1, 40), (17, 8296), (33, 8296), (49, 8296), (65, 8296), (97, 10944))] +
+             [(m, 16571, 1) for m in (1, 17, 33, 49, 65, 81, 97, 129)] + [(65, 32790, 1)],
+    "split": [(1, 40, 2)] + [(m, 1351, 6) for m in (17, 33, 49, 65)] + [(97, 1807, 6)] +
+             [(m, 2719, 6) for m in (1, 17, 33, 49, 65, 81, 97)] + [(65, 5648, 6)],
+    "act": [(1, 32, 1)] + [(m, 16544, 1) for m in (17, 33, 49, 65, 81, 97, 129)] + [(65, 33120, 1)],
+    "act split": [(1, 32, 2)] + [(m, 5632, 3) for m in (17, 33, 49, 65, 81, 97)] + [(65, 10944, 3)],
+    "lora": [(1, 40, 1)] + [(m, 2719, 3) for m in (17, 33, 49, 65)] + [(97, 3662, 3)] +
+            [(m, 5648, 3) for m in (1, 17, 33, 49, 65, 81, 97)],
+}
+
+
+def test_the_shapes_pick_every_tile():
+    for kind, shapes in TILE_SHAPES.items():
+        act = kind.startswith("act")
+        left_out = {"split": {(2, 10)}, "act split": {(2, 10)}, "lora": {(2, 10), (4, 8)}}.get(kind, set())
+        want = {t for t in WIDE_TILES if not (act and t[0] % 2)} - left_out
+        assert {_picked(*shape, act) for shape in shapes} == want, kind
+
+
+@pytest.mark.parametrize("M,N,split", TILE_SHAPES["plain"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_every_tile(device, M, N, split, dtype):
+    test_matches_the_row_split_chain_bit_for_bit(device, M, N, 136, dtype)
+
+
+@pytest.mark.parametrize("M,N,split", TILE_SHAPES["split"])
+@pytest.mark.parametrize("K", [1000, 1536])   # ranges of K steps off the packed groups, and on them
+def test_every_tile_with_k_splits(device, M, N, split, K):
+    test_row_split_tiles_with_k_splits(device, M, N, K, split)
+
+
+@pytest.mark.parametrize("M,N,split", TILE_SHAPES["act"] + TILE_SHAPES["act split"])
+def test_every_tile_with_the_activation(device, M, N, split):
+    x, w = _inputs_on_gpu(M, N, 1000, M + N, device)
+    if M <= 128:
+        test_silu_mul_on_row_split_tiles(device, M, N, 1000, split)
+        y = torch.empty(M, N // 2, device=device, dtype=x.dtype)
+        LinearChain([Link(x, w, y, act=True)], ROW_SPLIT).run()
+    else:
+        y = _chain(x, w).to(x.dtype)
+        y = F.silu(y[:, : N // 2]) * y[:, N // 2:]
+    if split == 1:   # the whole-weight form; past 128 rows up to a step of each rounding, as above
+        got = _wide(x, pack_weight(w), N, _lib.PLM_OUT_SILU_MUL, torch.empty_like(y))
+        assert int((got != y).sum()) <= (0 if M <= 128 else got.numel() // 1000)
+        torch.testing.assert_close(got.float(), y.float(), rtol=2 * 2.0 ** -7, atol=1e-30)
+
+
+@pytest.mark.parametrize("M,N,split", TILE_SHAPES["lora"])
+def test_every_tile_with_gated_lora(device, M, N, split):
+    """Two shards that meet inside a fragment, a rank past one MFMA's 32 elements."""
+    test_gated_lora_on_row_split_tiles(device, M, (N // 2 | 1, N - (N // 2 | 1)), 1000, 40, M // 3, split)
 
 
 # Rounds on row-split tiles: one row, a tile's edge and past it, the widest; ranges of K steps that
