@@ -252,6 +252,19 @@ def capture_graph(fn):
 
 
 
+def linear_alone(ln, cfg, out):
+    """One linear of a chain outside it, to check the chain's output bit for bit: its per-linear launch, or
+    on a row-split tile, where the chain is those launches, the packed kernel as a chain of that linear
+    alone runs it."""
+    from plm_amd.chain import Link, LinearChain
+    from plm_amd.fast_gemm import gate_up_silu, hip_linear
+
+    if cfg["k_waves"] == 1:
+        LinearChain([Link(ln.x, ln.w, out, split_k=ln.split_k, act=ln.act)], cfg).run()
+    else:
+        (gate_up_silu if ln.act else hip_linear)(ln.x, ln.w, dict(cfg, split_k=ln.split_k), out)
+
+
 class ChainedRound:
     """The round's block linears chained output-to-input over packed weights (plm_gemm_chain_packed, on
     the chain tile measured fastest for the round's hidden size and width, each linear's K split chosen
@@ -360,7 +373,7 @@ def main():
     # The chain computes what the single-linear kernel does with the same tiles, bit for
     # bit, through all 96 block linears; the LM head is the per-GEMM path's own launch.
     for i, ln in enumerate(chain.links):
-        hip_linear(ln.x, ln.w, dict(chain.cfg, split_k=ln.split_k), rnd.outs[i])
+        linear_alone(ln, chain.cfg, rnd.outs[i])
     hip_linear(*chained.head)
     torch.cuda.synchronize()
     mismatched = [i for i, (a, b) in enumerate(zip(chain_outs, rnd.outs)) if not torch.equal(a, b)]
@@ -530,7 +543,7 @@ def time_fp16_round(args, device, tables):
         raise RuntimeError("fp16 chained launch reported a timed-out wait")
     chain_outs = [o.clone() for o in rnd.outs]
     for i, ln in enumerate(chained.chain.links):
-        hip_linear(ln.x, ln.w, dict(chained.chain.cfg, split_k=ln.split_k), rnd.outs[i])
+        linear_alone(ln, chained.chain.cfg, rnd.outs[i])
     hip_linear(*chained.head)
     torch.cuda.synchronize()
     bit_exact = all(torch.equal(a, b) for a, b in zip(chain_outs, rnd.outs))
@@ -649,7 +662,7 @@ def time_configs(args, device, rnd, chained, us_round, us_graph):
     torch.cuda.synchronize()
     chain_outs = [o.clone() for o in r4.outs]
     for i, ln in enumerate(c4.chain.links):
-        hip_linear(ln.x, ln.w, dict(c4.chain.cfg, split_k=ln.split_k), r4.outs[i])
+        linear_alone(ln, c4.chain.cfg, r4.outs[i])
     hip_linear(*c4.head)
     torch.cuda.synchronize()
     same = all(torch.equal(a, b) for a, b in zip(chain_outs, r4.outs))
@@ -702,7 +715,7 @@ def time_wide_round(args, device, rnd):
     torch.cuda.synchronize()
     chain_outs = [o.clone() for o in wide.outs]
     for i, ln in enumerate(cw.chain.links):
-        hip_linear(ln.x, ln.w, dict(cw.chain.cfg, split_k=ln.split_k), wide.outs[i])
+        linear_alone(ln, cw.chain.cfg, wide.outs[i])
     hip_linear(*cw.head)
     torch.cuda.synchronize()
     same = all(torch.equal(a, b) for a, b in zip(chain_outs, wide.outs))
@@ -821,7 +834,7 @@ def time_llama_rounds(args, device):
     import torch
 
     from plm_amd import gemm_tables
-    from plm_amd.fast_gemm import gate_up_silu, hip_linear
+    from plm_amd.fast_gemm import hip_linear
     from plm_amd.workloads import LLAMA_SETS, llama_round
 
     out = {}
@@ -843,8 +856,7 @@ def time_llama_rounds(args, device):
             torch.cuda.synchronize()
             chain_outs = [o.clone() for o in rnd.outs]
             for i, ln in enumerate(chained.chain.links):
-                fn = gate_up_silu if ln.act else hip_linear
-                fn(ln.x, ln.w, dict(chained.chain.cfg, split_k=ln.split_k), rnd.outs[i])
+                linear_alone(ln, chained.chain.cfg, rnd.outs[i])
             hip_linear(*chained.head)
             torch.cuda.synchronize()
             same = all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(chain_outs, rnd.outs))
