@@ -57,10 +57,10 @@ constexpr int kWidePlain = 0, kWideAct = 1, kWideLora = 2;
 
 // The gated-LoRA launch (plm_gemm_packed_lora): workgroups [0, items) form h = X A^T in the model dtype,
 // the base linear's workgroups follow, wait for h once their own sums are formed, and add the rank-r
-// correction as MFMAs. Against the packed kernel's launch, which adds it as scalar products (us, base
-// linear alone in brackets): 3072x2048, rank 16, M = 56 13.6 [9.9] -> 11.1 [7.3]; 11264x2048 38.2 [23.1] ->
-// 15.2 [12.2]; 4608x3072, rank 64, M = 110 61.5 [29.6] -> 16.2 [11.9]. What is left over the base linear is
-// h's chain: X, the partial sums' round trip, h's own.
+// correction as MFMAs. Against the packed kernel's launch, which adds it as scalar products (us, weights
+// from memory): 3072x2048, rank 16, M = 56 13.8 -> 10.9; 11264x2048 24.1 -> 18.7; 4608x3072, rank 64,
+// M = 110 55.1 -> 17.1. What is left over the base linear (6.7, 13.5, 12.3) is h's chain: X, the partial
+// sums' round trip, h's own.
 struct WideLora {
   const void* w;     // A, packed
   uint16_t* h;       // [M][width]
@@ -474,35 +474,41 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_gemm_kernel(WideArgs a) 
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
       const int nf = __builtin_amdgcn_readfirstlane(16 * (of0 + f));
-      const int s_lo = shard_of(nf), s_hi = shard_of(min(nf + 15, a.N - 1));
+      const int s_lo = shard_of(min(nf, a.N - 1)), s_hi = shard_of(min(nf + 15, a.N - 1));
       const int s_own = shard_of(nf + (lane & 15));
-      auto product = [&](int s, f32x4 (&p)[MT]) __attribute__((always_inline)) {
+      // Over the fragment's shards, and for each over 32 rank elements at a time, in one copy of the code (a
+      // second, for straddling fragments only, took 11.3 us at 3072x2048, rank 16, M = 56, this 10.9); `done`
+      // holds the columns of the shards before.
+      f32x4 corr[MT], done[MT];
 #pragma unroll
-        for (int t = 0; t < MT; ++t) p[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int j = 0; 32 * j < z.rank; ++j) {
-          const u32x4 row = j == 0 ? b_first[f] : load_b(f, j);
-          const u32x4 bs = s_own == s ? row : u32x4{0u, 0u, 0u, 0u};
-          const int e = 32 * j + 8 * (lane >> 4);
-          u32x4 hv[MT];
+      for (int t = 0; t < MT; ++t) corr[t] = done[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      int s = s_lo;
+      for (int j = 0;;) {
+        const u32x4 row = j == 0 ? b_first[f] : load_b(f, j);
+        const u32x4 bs = s_own == s ? row : u32x4{0u, 0u, 0u, 0u};
+        const int e = 32 * j + 8 * (lane >> 4);
+        u32x4 hv[MT];
 #pragma unroll
-          for (int t = 0; t < MT; ++t) {
-            const int m = mt * 16 * MT + 16 * t + (lane & 15);
-            const uint32_t off = m < a.M && e < z.rank ? static_cast<uint32_t>((m * z.width + s * z.rank + e) * 2) : kOutOfRange;
-            hv[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(hr, static_cast<int>(off), 0, kCoherent));
-          }
-#pragma unroll
-          for (int t = 0; t < MT; ++t) p[t] = mfma_16x16x32<DT>(bs, hv[t], p[t]);
+        for (int t = 0; t < MT; ++t) {
+          const int m = mt * 16 * MT + 16 * t + (lane & 15);
+          const uint32_t off = m < a.M && e < z.rank ? static_cast<uint32_t>((m * z.width + s * z.rank + e) * 2) : kOutOfRange;
+          hv[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(hr, static_cast<int>(off), 0, kCoherent));
         }
-      };
-      f32x4 corr[MT];
-      product(s_lo, corr);
-      for (int s = s_lo + 1; s <= s_hi; ++s) {
-        f32x4 part[MT];
-        product(s, part);
 #pragma unroll
-        for (int t = 0; t < MT; ++t)
+        for (int t = 0; t < MT; ++t) corr[t] = mfma_16x16x32<DT>(bs, hv[t], corr[t]);
+        if (32 * ++j < z.rank) continue;
+        if (s_lo != s_hi) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) corr[t][r] = shard_of(nf + 4 * (lane >> 4) + r) == s ? part[t][r] : corr[t][r];
+          for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int own = shard_of(nf + 4 * (lane >> 4) + r);
+              done[t][r] = own == s ? corr[t][r] : done[t][r];
+              corr[t][r] = s == s_hi ? done[t][r] : 0.f;
+            }
+        }
+        if (++s > s_hi) break;
+        j = 0;
       }
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
