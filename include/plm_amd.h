@@ -70,12 +70,14 @@ enum plm_status {
  *     split_k    : workgroups splitting K (1..64); their fp32 partials are summed in split order
  *                  0..split_k-1 by the last workgroup of the tile to finish (no float atomics).
  *     unroll     : K steps of loads in flight per wavefront (2, 4, 6 or 8).
- *   row-major streaming kernel (plm_gemm, plm_gemm_chain, plm_lm_head_verify):
+ *   row-major streaming kernel (plm_gemm, plm_gemm_chain):
  *     wave_frags : 16-row fragments per compute wavefront; a workgroup has four compute wavefronts
  *                  (tile = 64*wave_frags rows), four loader wavefronts and one epilogue wavefront.
  *     k_waves    : 4 (the compute wavefronts).
  *     split_k    : as above.
  *     unroll     : 2 (one 128-byte line of every weight row per streamed chunk).
+ * plm_lm_head_verify takes k_waves 4, split_k 1, wave_frags 2 or 4 and unroll 2, 4 or 8, refuses the
+ * combinations that do not suit its R and K, and tiles by rules of its own.
  */
 typedef struct plm_tile {
   int32_t wave_frags;
@@ -119,12 +121,14 @@ int plm_unpack_weight(int32_t dtype, const void* packed, size_t packed_bytes, in
  * wavefronts split the tile's K range (summed in LDS in wavefront order), or k_waves = 1: a
  * workgroup tile is 64*wave_frags rows, each wavefront owns 16*wave_frags of them over the whole
  * K range, and the four share one copy of X through LDS (except at M <= 64 over a packed weight of 128 MiB
- * and more with N > 32768, such a call runs on the wide kernel, with the same sums in the same order); split_k = workgroups splitting K (1..64,
- * partials summed in split order); unroll = K steps of loads in flight per wavefront (2, 4, 6,
+ * and more with N > 32768, or with N * split_k >= 65536 where K is split, such a call runs on the wide
+ * kernel, with the same sums in the same order); split_k = workgroups splitting K (1..64, partials summed
+ * in split order); unroll = K steps of loads in flight per wavefront (2, 4, 6,
  * 8). Requirements as plm_gemm (K % 8 == 0, K <= 2^24, ldx % 8 == 0, x 16-byte aligned) except
  * that M may exceed 128: wider calls (prefill chunks, plm/rounds.py:16, which the reference hands to
  * F.linear) run on the wide kernel (X through LDS, weights straight to registers, no K split), whose
- * tiling is its own: `tile` must be valid but is not used. Workspace: plm_gemm_packed_workspace_bytes.
+ * tiling is its own: `tile` must be valid but is not used. Workspace: plm_gemm_packed_workspace_bytes, above
+ * 128 rows too, where the size is the interface's and the kernel reads none of it.
  */
 int plm_gemm_packed(int32_t dtype, const void* x, int64_t ldx, const void* packed_w, void* y, int64_t ldy, int64_t M,
                     int64_t N, int64_t K, const plm_tile* tile, void* workspace, size_t workspace_bytes, void* stream);
@@ -147,8 +151,8 @@ int plm_gemm_packed_f32out(int32_t dtype, const void* x, int64_t ldx, const void
 int plm_gemm_packed_noalloc(int32_t dtype, const void* x, int64_t ldx, const void* packed_w, void* y, int64_t ldy,
                             int64_t M, int64_t N, int64_t K, const plm_tile* tile, void* stream);
 
-/* Workspace bytes plm_gemm_packed needs for this shape and tile (0 without split-K), and whether a
- * kernel is compiled for the tile at this M. */
+/* Workspace bytes plm_gemm_packed asks for at this shape and tile (up to 128 rows 0 without split-K), and
+ * whether a kernel is compiled for the tile at this M. */
 size_t plm_gemm_packed_workspace_bytes(int64_t M, int64_t N, int64_t K, const plm_tile* tile);
 int plm_gemm_packed_tile_supported(int32_t dtype, int64_t M, int64_t K, const plm_tile* tile);
 
@@ -275,7 +279,7 @@ int plm_gemm_tile_supported(int32_t dtype, int64_t M, int64_t K, const plm_tile*
  *               An id outside [0, V) is never accepted.
  *   argmax[r] = index of the row maximum, lowest index on ties (plm/decoder.py:362).
  * `round_mode` (enum plm_round_mode) fixes the logits the decision reads. Requirements as
- * plm_gemm. `tile` uses split_k == 1.
+ * plm_gemm. `tile`: see plm_tile.
  */
 int plm_lm_head_verify(int32_t dtype, const void* x, int64_t ldx, const void* w, int64_t ldw, int64_t R, int64_t V,
                        int64_t K, const int64_t* pending, int32_t rule, float p, int32_t round_mode, uint8_t* accept,

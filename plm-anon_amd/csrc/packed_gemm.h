@@ -113,7 +113,8 @@ struct PackedArgs {
   int G;           // workgroups in the grid
   int sync;        // 0: no linear reads another's output; 1: grid barriers after such linears
                    // (progress flags); 2: tile flags (every linear after the first reads the one
-                   // before it: each wavefront waits only for the producer tiles it reads)
+                   // before it: each wavefront waits only for the producer tiles it reads). Always 0
+                   // with KW = 1: linears that read one another are launches of their own there
   int spin_limit;  // polls before a wait gives up
   int* counters;
   float* partial;

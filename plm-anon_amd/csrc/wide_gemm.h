@@ -1,6 +1,6 @@
-// The wide GEMM over packed weights (M > 128: prefill chunks), behind plm_gemm_packed,
-// plm_gemm_packed_f32out and plm_gemm_wide_silu_mul. Arguments are checked by the caller
-// (csrc/packed_api.hip).
+// The wide GEMM over packed weights: behind plm_gemm_wide, behind plm_gemm_packed and its variants above 128
+// rows and for row-split tiles, and behind plm_gemm_packed_silu_mul, plm_gemm_packed_lora and the links of
+// plm_gemm_chain_packed on such tiles. Arguments are checked by the caller (csrc/packed_api.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -59,7 +59,7 @@ constexpr int kWidePlain = 0, kWideAct = 1, kWideLora = 2;
 // the base linear's workgroups follow, wait for h once their own sums are formed, and add the rank-r
 // correction as MFMAs. Against the packed kernel's launch, which adds it as scalar products (us, weights
 // from memory): 3072x2048, rank 16, M = 56 13.8 -> 10.9; 11264x2048 24.1 -> 18.7; 4608x3072, rank 64,
-// M = 110 55.1 -> 17.1. What is left over the base linear (6.7, 13.5, 12.3) is h's chain: X, the partial
+// M = 110 55.1 -> 17.1. What is left over the base linear (7.6, 13.5, 13.0) is h's chain: X, the partial
 // sums' round trip, h's own.
 struct WideLora {
   const void* w;     // A, packed

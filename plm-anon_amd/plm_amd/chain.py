@@ -7,8 +7,9 @@ of start-up and tail in which HBM idles; a chain keeps one persistent grid strea
 across the linears. With packed weights (the default) the workgroups meet at a grid barrier after
 each linear another one reads, with the next linear's first weights already requested; the
 streaming kernel on row-major weights (``packed=False``) starts each tile of a linear as soon as
-the producer tiles it reads are written. On a row-split tile (``k_waves`` 1, what rounds of more than 48
-rows run on) a chain of linears that read one another is a launch per linear, back to back on the stream.
+the producer tiles it reads are written. On a row-split tile (``k_waves`` 1: ``tiles.packed_chain_tile``'s
+above 48 rows, and what ``gemm_tables.round_chain_tile`` holds where it measured faster) a chain of linears
+that read one another is a launch per linear, back to back on the stream.
 """
 
 from __future__ import annotations

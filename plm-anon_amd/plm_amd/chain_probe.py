@@ -198,7 +198,7 @@ def run(out: Path) -> None:
         gen.manual_seed(1 + 3000 + i)
         weights.append((0.02 * torch.randn(g.N, g.K, generator=gen, device=dev)).bfloat16())
     names = ["qkv", "attn-out", "mlp-up", "mlp-down"]
-    for M in (28, 7):   # widths whose rounds run on the chained kernel
+    for M in (56, 7):   # widths whose rounds run on the chained kernel
         ch = bench.ChainedRound(bench.Round(M, 2048, 8192, 24, weights, gemm_tables.read_table(2048), dev))
         for _ in range(5):
             ch.chain.run()

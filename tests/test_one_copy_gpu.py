@@ -1,7 +1,7 @@
 """One copy per weight: ``fast_gemm.release`` frees a weight's row-major storage and every product
 with it runs on the packed copy, at the round widths (tuned tiles, plm/gemm_tables.py) and at the
 prefill widths the reference hands to ``F.linear`` (M = 64 ... 640, plm/rounds.py:16; above 128 rows
-as 128-row slices). Parity as tests/test_gemm_gpu.py (within one rounding of the exact product and
+on the wide kernel). Parity as tests/test_gemm_gpu.py (within one rounding of the exact product and
 within tolerance of the oracle), on sampled columns for the wide calls."""
 
 from __future__ import annotations
