@@ -472,13 +472,11 @@ def _wide(x: torch.Tensor, weight: torch.Tensor, packed: torch.Tensor, out_kind:
     (``out_kind`` as plm_gemm_wide's), or None for a call that ``F.linear`` on the unpacked weight has to
     take. The two have the same sums in the same order where F.linear's library does not split K;
     measured (M = 640, 1.3B block): 137 us with F.linear, 97 us here."""
-    if not _plain(x) or x.device != weight.device:
+    (M, K), N = x.shape, weight.shape[0]
+    if not _plain(x) or x.device != weight.device or not _wide_pays(M, N, K, out_kind == _lib.PLM_OUT_SILU_MUL):
         return None
     x = _row_major(x)
-    (M, K), N = x.shape, weight.shape[0]
     if x.data_ptr() % 16 or not _wide_takes(M, x.stride(0), packed.numel()):
-        return None
-    if not _wide_pays(M, N, K, out_kind == _lib.PLM_OUT_SILU_MUL):
         return None
     y = torch.empty(M, N // 2 if out_kind == _lib.PLM_OUT_SILU_MUL else N, device=x.device, dtype=x.dtype)
     status = _lib.lib().plm_gemm_wide(_lib.DTYPE_CODES[x.dtype], x.data_ptr(), x.stride(0), packed.data_ptr(),
